@@ -2,8 +2,8 @@
 //
 // Orchestrates, per call, on one HIP stream:
 //   prior_kernel -> rates_kernel -> bucket order of particles by expected cost
-//   (heaviest first) -> item offsets -> burn_kernel (burn-in of every cell up
-//   to its labelling window) -> ssa_kernel (the window, persistent, lane-level
+//   (heaviest first) -> burn_kernel (burn-in of every cell up to its labelling
+//   window) -> cell order by expected cost -> ssa_kernel (the window, persistent, lane-level
 //   work stealing) -> stats_kernel -> error / acceptance kernels.
 // Device buffers are owned by the context and grow on demand.  The *_dev
 // sequences use kernels only (no memset, no host wait), so they can be
@@ -22,8 +22,13 @@
 // Device memory of abc_simulate_noalloc_dev: one array per GPU, alive until
 // the process ends.  Host code reaches it only through the address
 // hipGetSymbolAddress returns for the current device (scratch_address).
+// The limit on the particles of a call is a formula of its own
+// (noalloc_bytes); the workspace carved for an accepted call never exceeds it
+// by more than the fixed bucket tables, which the margin holds.
 #define ABC_NOALLOC_SCRATCH_BYTES ((size_t)256 << 20)
-static __device__ __align__(256) unsigned char scratch[ABC_NOALLOC_SCRATCH_BYTES];
+#define ABC_NOALLOC_MARGIN_BYTES ((size_t)64 << 10)
+static __device__ __align__(256) unsigned char
+    scratch[ABC_NOALLOC_SCRATCH_BYTES + ABC_NOALLOC_MARGIN_BYTES];
 
 namespace {
 
@@ -88,9 +93,9 @@ struct abc_ctx {
   DesignDev* dd = nullptr;
   double* d_betas = nullptr;
   int64_t* d_goff = nullptr;
-  DevBuf theta, rates, cost, hist, order, bsum, off, cellrec, cu, cl,
-      cb, steps, react, queue, stats, moments, superset, edata, ese, err, cand, ccount, ah, al,
-      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, presc, apidx, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, coff, pitems, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
+  DevBuf theta, rates, cost, hist, order, cellord, chist, ctabs, cellrec, cu, cl,
+      cb, steps, queue, stats, moments, superset, edata, ese, err, cand, ccount, ah, al,
+      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, presc, apidx, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
   AcceptState acc;
   hipEvent_t ev[5]{};
   bool timed[4]{};
@@ -193,23 +198,22 @@ int grid1(int64_t n, int bs) { return (int)((n + bs - 1) / bs); }
 unsigned pgrid(int64_t n) { return (unsigned)std::min<int64_t>(n, (int64_t)1 << 20); }
 
 // Device memory one simulation of n particles works in: per-particle rates,
-// queue order and item offsets, each cell's burn-in record, sub-lane offsets
-// and observed counts, and the counters.  Filled from the context's buffers
+// queue order, each cell's burn-in record, place in the window's queue and
+// observed counts, and the counters.  Filled from the context's buffers
 // (ws_from_ctx) or carved from one block of memory (ws_carve).
 struct SimWs {
   PRates* rates = nullptr;
   float* cost = nullptr;
   unsigned* hist = nullptr;             // 2 * ABC_NBUCKET: histogram, cursors
   int32_t* order = nullptr;
-  int64_t* bsum = nullptr;
-  int64_t* off = nullptr;               // n + 1
+  unsigned* chist = nullptr;            // ABC_CELL_BUCKETS: cells per bucket
+  CellTables* ctabs = nullptr;
   CellStart* cellrec = nullptr;         // n * C
-  int32_t* coff = nullptr;              // n * (C + 1)
-  int64_t* pitems = nullptr;
-  uint32_t* cu = nullptr;               // n * C, rounded up to whole u64 words
+  uint32_t* cellord = nullptr;          // n * C: cells, heaviest bucket first
+  uint32_t* cu = nullptr;               // n * C, rounded up to whole u64 words (the
+                                        // cells' queue keys until the window starts)
   uint32_t* cl = nullptr;
   uint8_t* cb = nullptr;                // n * C
-  unsigned long long* react = nullptr;
   unsigned long long* queue = nullptr;  // 8 words: burn-in and SSA work queues
   unsigned long long* tally = nullptr;  // 2 words: burn-in draws
   unsigned long long* steps = nullptr;  // n: draws per particle when the caller keeps none
@@ -222,7 +226,6 @@ int64_t cell_words(int64_t n, int C) { return (n * (int64_t)C + 1) / 2; }
 // to 256 bytes); with base != NULL the pointers of w are set into it.
 size_t ws_carve(char* base, int64_t n, int C, SimWs* w) {
   const size_t nn = (size_t)n, cells = (size_t)n * (size_t)C;
-  const int64_t nblk = (n + ABC_SCAN_BLOCK - 1) / ABC_SCAN_BLOCK;
   size_t at = 0;
   auto take = [&](size_t bytes) -> char* {
     char* q = base ? base + at : nullptr;
@@ -234,19 +237,31 @@ size_t ws_carve(char* base, int64_t n, int C, SimWs* w) {
   v.cost = reinterpret_cast<float*>(take(sizeof(float) * nn));
   v.hist = reinterpret_cast<unsigned*>(take(sizeof(unsigned) * 2 * ABC_NBUCKET));
   v.order = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * nn));
-  v.bsum = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * (size_t)nblk));
-  v.off = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * (nn + 1)));
+  v.chist = reinterpret_cast<unsigned*>(take(sizeof(unsigned) * ABC_CELL_BUCKETS));
+  v.ctabs = reinterpret_cast<CellTables*>(take(sizeof(CellTables)));
   v.cellrec = reinterpret_cast<CellStart*>(take(sizeof(CellStart) * cells));
-  v.coff = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * nn * (size_t)(C + 1)));
-  v.pitems = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * nn));
+  v.cellord = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * cells));
   v.cu = reinterpret_cast<uint32_t*>(take(sizeof(uint64_t) * (size_t)cell_words(n, C)));
   v.cl = reinterpret_cast<uint32_t*>(take(sizeof(uint64_t) * (size_t)cell_words(n, C)));
   v.cb = reinterpret_cast<uint8_t*>(take(cells));
-  v.react = reinterpret_cast<unsigned long long*>(take(sizeof(uint64_t) * nn));
   v.queue = reinterpret_cast<unsigned long long*>(take(64));
   v.tally = reinterpret_cast<unsigned long long*>(take(16));
   v.steps = reinterpret_cast<unsigned long long*>(take(sizeof(uint64_t) * nn));
   if (base && w) *w = v;
+  return at;
+}
+
+// Bytes that bound a call of abc_simulate_noalloc_dev: about 77 per cell and
+// 620 per particle, rounded up array by array.
+size_t noalloc_bytes(int64_t n, int C) {
+  const size_t nn = (size_t)n, cells = nn * (size_t)C;
+  const size_t blk = (size_t)((n + 1023) / 1024);
+  const size_t part[] = {sizeof(PRates) * nn, 4 * nn, 8 * ABC_NBUCKET, 4 * nn, 8 * blk,
+                         8 * (nn + 1), sizeof(CellStart) * cells, 4 * nn * (size_t)(C + 1),
+                         8 * nn, 8 * (size_t)cell_words(n, C), 8 * (size_t)cell_words(n, C),
+                         cells, 8 * nn, 64, 16, 8 * nn};
+  size_t at = 0;
+  for (size_t b : part) at += (std::max<size_t>(b, 16) + 255) / 256 * 256;
   return at;
 }
 
@@ -256,20 +271,18 @@ int ws_from_ctx(abc_ctx* c, int64_t n, SimWs* w) {
   int rc;
   const int C = c->hd.C;
   const size_t nn = (size_t)n, cells = (size_t)n * (size_t)C;
-  const int64_t nblk = (n + ABC_SCAN_BLOCK - 1) / ABC_SCAN_BLOCK;
   if ((rc = ensure(c, c->rates, sizeof(PRates) * nn))) return rc;
   if ((rc = ensure(c, c->cost, sizeof(float) * nn))) return rc;
   if ((rc = ensure(c, c->hist, sizeof(unsigned) * 2 * ABC_NBUCKET))) return rc;
   if ((rc = ensure(c, c->order, sizeof(int32_t) * nn))) return rc;
-  if ((rc = ensure(c, c->bsum, sizeof(int64_t) * (size_t)nblk))) return rc;
-  if ((rc = ensure(c, c->off, sizeof(int64_t) * (nn + 1)))) return rc;
+  if ((rc = ensure(c, c->chist, sizeof(unsigned) * ABC_CELL_BUCKETS))) return rc;
+  if ((rc = ensure(c, c->ctabs, sizeof(CellTables)))) return rc;
   if ((rc = ensure(c, c->cellrec, sizeof(CellStart) * cells))) return rc;
-  if ((rc = ensure(c, c->coff, sizeof(int32_t) * nn * (size_t)(C + 1)))) return rc;
-  if ((rc = ensure(c, c->pitems, sizeof(int64_t) * nn))) return rc;
+  if (cells > 0xFFFFFFFFull) return fail(c, ABC_E_OOM, "at most 2^32 - 1 cells per call");
+  if ((rc = ensure(c, c->cellord, sizeof(uint32_t) * cells))) return rc;
   if ((rc = ensure(c, c->cu, sizeof(uint64_t) * (size_t)cell_words(n, C)))) return rc;
   if ((rc = ensure(c, c->cl, sizeof(uint64_t) * (size_t)cell_words(n, C)))) return rc;
   if ((rc = ensure(c, c->cb, cells))) return rc;
-  if ((rc = ensure(c, c->react, sizeof(uint64_t) * nn))) return rc;
   if ((rc = ensure(c, c->queue, 64))) return rc;
   if ((rc = ensure(c, c->steps, sizeof(uint64_t) * nn))) return rc;
   if (!c->tally.p) {
@@ -283,15 +296,13 @@ int ws_from_ctx(abc_ctx* c, int64_t n, SimWs* w) {
   w->cost = P<float>(c->cost);
   w->hist = P<unsigned>(c->hist);
   w->order = P<int32_t>(c->order);
-  w->bsum = P<int64_t>(c->bsum);
-  w->off = P<int64_t>(c->off);
+  w->chist = P<unsigned>(c->chist);
+  w->ctabs = P<CellTables>(c->ctabs);
   w->cellrec = P<CellStart>(c->cellrec);
-  w->coff = P<int32_t>(c->coff);
-  w->pitems = P<int64_t>(c->pitems);
+  w->cellord = P<uint32_t>(c->cellord);
   w->cu = P<uint32_t>(c->cu);
   w->cl = P<uint32_t>(c->cl);
   w->cb = P<uint8_t>(c->cb);
-  w->react = P<unsigned long long>(c->react);
   w->queue = P<unsigned long long>(c->queue);
   w->tally = P<unsigned long long>(c->tally);
   w->steps = P<unsigned long long>(c->steps);
@@ -320,18 +331,20 @@ int launch_order(abc_ctx* c, const SimWs& w, int64_t n) {
   return ABC_OK;
 }
 
-// after the burn-in: each cell's sub-lanes -> per-particle cell offsets and
-// item counts -> the item offsets of the particles in queue order
+// after the burn-in: the window's queue order of all n * C cells, from the
+// keys burn_kernel left in w.cu (which is cleared here for the counts)
 int stage_items(abc_ctx* c, const SimWs& w, int64_t n) {
-  const int64_t nblk = (n + ABC_SCAN_BLOCK - 1) / ABC_SCAN_BLOCK;
-  const int C = c->hd.C;
-  hipLaunchKernelGGL(cell_items_kernel, dim3(pgrid(n)), dim3(256), 0, c->stream, n, C, w.cellrec,
-                     w.coff, w.pitems);
-  hipLaunchKernelGGL(items_scan_kernel, dim3((unsigned)nblk), dim3(256), 0, c->stream, w.pitems,
-                     w.order, n, w.off, w.bsum);
-  hipLaunchKernelGGL(bsum_scan_kernel, dim3(1), dim3(256), 0, c->stream, w.bsum, nblk);
-  hipLaunchKernelGGL(add_bsum_kernel, dim3(grid1(n, 256)), dim3(256), 0, c->stream, w.off, n,
-                     w.bsum);
+  const int64_t cells = n * (int64_t)c->hd.C, words = cell_words(n, c->hd.C);
+  hipLaunchKernelGGL(cell_hist_kernel,
+                     dim3((unsigned)std::min<int64_t>((cells + 4095) / 4096, c->num_cu * 8)),
+                     dim3(256), 0, c->stream, w.cu, cells, w.chist);
+  hipLaunchKernelGGL(cell_scan_kernel, dim3(1), dim3(ABC_CELL_BUCKETS), 0, c->stream, w.chist,
+                     w.ctabs);
+  hipLaunchKernelGGL(cell_scatter_kernel,
+                     dim3((unsigned)((cells + ABC_CELL_TILE - 1) / ABC_CELL_TILE)), dim3(256), 0,
+                     c->stream, w.cu, cells, w.ctabs, w.cellord);
+  hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(words, 256)), dim3(256), 0, c->stream,
+                     reinterpret_cast<unsigned long long*>(w.cu), words);
   HIPCHK(c, hipGetLastError());
   return ABC_OK;
 }
@@ -362,11 +375,11 @@ int simulate_core(abc_ctx* c, const SimWs& w, uint64_t seed, int64_t n, int64_t 
   const int64_t words = cell_words(n, c->hd.C);  // u32 counts cleared as u64 words
   // counters cleared by a kernel (no memset nodes, so the sequence can be captured)
   hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(words, 256)), dim3(256), 0, c->stream,
-                     reinterpret_cast<unsigned long long*>(w.cu), words);
-  hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(words, 256)), dim3(256), 0, c->stream,
                      reinterpret_cast<unsigned long long*>(w.cl), words);
   hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(n, 256)), dim3(256), 0, c->stream, steps, n);
-  hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(n, 256)), dim3(256), 0, c->stream, w.react, n);
+  hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(ABC_CELL_BUCKETS / 2, 256)), dim3(256), 0,
+                     c->stream, reinterpret_cast<unsigned long long*>(w.chist),
+                     (int64_t)(ABC_CELL_BUCKETS / 2));
   hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream, w.queue, (int64_t)8);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, record(c, c->ev[1]));
@@ -381,14 +394,14 @@ int simulate_core(abc_ctx* c, const SimWs& w, uint64_t seed, int64_t n, int64_t 
   const int blocks = c->ssa_blocks > 0 ? c->ssa_blocks : c->ssa_blocks_default;
   hipLaunchKernelGGL(burn_kernel, dim3(c->burn_blocks), dim3(SSA_WG), 0, c->stream, c->dd,
                      w.rates, w.order, n, (uint32_t)first, key0(seed), key1(seed), mtag_all,
-                     mtags, c->d_betas, c->d_goff, w.queue, w.cellrec, steps, w.react, pidx_dev,
+                     mtags, c->d_betas, c->d_goff, w.queue, w.cellrec, w.cu, steps, pidx_dev,
                      w.tally);
   HIPCHK(c, hipGetLastError());
   if ((rc = stage_items(c, w, n))) return rc;
   if (trio) HIPCHK(c, hipEventRecord(trio[1], c->stream));
   hipLaunchKernelGGL(ssa_kernel, dim3(blocks), dim3(SSA_WG), 0, c->stream, c->dd, w.rates,
-                     w.order, w.off, n, (uint32_t)first, key0(seed), key1(seed), mtag_all, mtags,
-                     w.cellrec, w.coff, w.queue + 1, w.cu, w.cl, w.cb, steps, pidx_dev,
+                     w.ctabs, w.cellord, (uint32_t)first, key0(seed), key1(seed), mtag_all, mtags,
+                     w.cellrec, w.queue + 1, w.cu, w.cl, w.cb, steps, pidx_dev,
                      (uint32_t)c->ssa_claim);
   HIPCHK(c, hipGetLastError());
   if (trio) HIPCHK(c, hipEventRecord(trio[2], c->stream));
@@ -589,12 +602,12 @@ int32_t abc_create(abc_ctx** out, int32_t device, const abc_design* d) {
 int32_t abc_destroy(abc_ctx* c) {
   if (!c) return ABC_OK;
   if (c->stream) hipStreamSynchronize(c->stream);
-  DevBuf* bufs[] = {&c->theta, &c->rates, &c->cost, &c->hist, &c->order, &c->bsum, &c->off,
-                    &c->cellrec,
-                    &c->cu, &c->cl, &c->cb, &c->steps, &c->react, &c->queue,
+  DevBuf* bufs[] = {&c->theta, &c->rates, &c->cost, &c->hist, &c->order, &c->cellord, &c->chist,
+                    &c->ctabs, &c->cellrec,
+                    &c->cu, &c->cl, &c->cb, &c->steps, &c->queue,
                     &c->stats, &c->moments, &c->superset, &c->edata, &c->ese, &c->err,
                     &c->cand, &c->ccount, &c->ah, &c->al, &c->pflag, &c->bh, &c->bl,
-                    &c->cg, &c->gflag, &c->thr, &c->wf, &c->sy, &c->tally, &c->mss, &c->mmap, &c->coff, &c->pitems, &c->mpidx, &c->mk1, &c->mcost, &c->mord, &c->dmeta, &c->dw,
+                    &c->cg, &c->gflag, &c->thr, &c->wf, &c->sy, &c->tally, &c->mss, &c->mmap, &c->mpidx, &c->mk1, &c->mcost, &c->mord, &c->dmeta, &c->dw,
                     &c->dboot, &c->dflag, &c->du, &c->dl, &c->dout, &c->dsort, &c->dpt, &c->dxs, &c->selb,
                     &c->pool, &c->pooln, &c->poolb, &c->presc, &c->apidx, &c->thrlow, &c->spass,
                     &c->mom, &c->mth, &c->mst, &c->selc, &c->selo};
@@ -810,17 +823,19 @@ int32_t abc_simulate_noalloc_dev(abc_ctx* c, int32_t model, uint64_t seed, int64
   if ((rc = check_range(c, model, first, n))) return rc;
   if (n == 0) return ABC_OK;
   const int C = c->hd.C;
-  if (ws_carve(nullptr, n, C, nullptr) > ABC_NOALLOC_SCRATCH_BYTES) {
+  if (noalloc_bytes(n, C) > ABC_NOALLOC_SCRATCH_BYTES) {
     int64_t lo = 0, hi = (int64_t)1 << 31;  // the largest n whose workspace fits
     while (hi - lo > 1) {
       const int64_t mid = lo + (hi - lo) / 2;
-      (ws_carve(nullptr, mid, C, nullptr) <= ABC_NOALLOC_SCRATCH_BYTES ? lo : hi) = mid;
+      (noalloc_bytes(mid, C) <= ABC_NOALLOC_SCRATCH_BYTES ? lo : hi) = mid;
     }
     return fail(c, ABC_E_ARG,
                 "abc_simulate_noalloc_dev takes at most " + std::to_string(lo) +
                     " particles of " + std::to_string(C) + " cells per call (" +
                     std::to_string(ABC_NOALLOC_SCRATCH_BYTES >> 20) + " MiB of scratch)");
   }
+  if (ws_carve(nullptr, n, C, nullptr) > ABC_NOALLOC_SCRATCH_BYTES + ABC_NOALLOC_MARGIN_BYTES)
+    return fail(c, ABC_E_ARG, "the scratch array is too small");
   SimWs w;
   ws_carve(static_cast<char*>(c->scratch), n, C, &w);
   w.timed = false;  // its burn-in draws are not in the context's tally

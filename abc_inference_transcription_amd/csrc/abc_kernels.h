@@ -12,7 +12,9 @@
 #define ABC_MAX_PARTS 16
 #define SSA_WG 256
 #define ABC_NBUCKET 256      // cost buckets of the queue order
-#define ABC_SCAN_BLOCK 1024  // ranks per block of the item scan
+#define ABC_CELL_BUCKETS 1024  // 64 cost classes x 16 sub-lane counts of the cell order
+#define ABC_LIGHT_CLASS 36     // cost classes below this are claimed several items at a time
+#define ABC_CELL_TILE 4096     // cells one workgroup places in the cell order
 
 // Experimental design in device memory (read through uniform scalar loads).
 struct DesignDev {
@@ -47,7 +49,9 @@ struct __align__(16) PRates {
   uint64_t thr_pi;                 // floor(P(gene on at cycle start) * 2^32)
   int32_t B, step, scaling;        // burn-in cycles, grid stride, size scaling
   int32_t gene_varies;             // kon differs between bins (burst-frequency model)
-  int32_t M, pad[3];               // typical sub-lanes per cell (the queue-order key only)
+  float swrate, gmean;             // gene switches and decays per hour, means over the bins
+                                   // (queue-order keys only)
+  int32_t pad[2];
 };
 
 // A cell at the start of its labelling window (burn_kernel -> ssa_kernel).
@@ -59,6 +63,13 @@ struct __align__(16) CellStart {
   uint64_t gctr;    // gene-stream counter
   uint8_t bin, g, gneed;
   uint8_t msh;      // log2 of the cell's sub-lanes M
+};
+
+// Tables of the cell order (cell_scan_kernel), by rank from the heaviest
+// bucket: first item (and all items at the end), first cell, scatter cursor.
+struct CellTables {
+  unsigned long long ioff[ABC_CELL_BUCKETS + 1];
+  unsigned cbase[ABC_CELL_BUCKETS], cursor[ABC_CELL_BUCKETS];
 };
 
 struct ErrSpec {
@@ -92,27 +103,24 @@ __global__ void bucket_hist_kernel(const float* cost, int64_t n, unsigned* hist)
 __global__ void bucket_scan_kernel(const unsigned* hist, unsigned* cursor);
 __global__ void bucket_scatter_kernel(const float* cost, int64_t n, unsigned* cursor,
                                       int32_t* order);
-__global__ void items_scan_kernel(const int64_t* pitems, const int32_t* order, int64_t n,
-                                  int64_t* off, int64_t* bsum);
-__global__ void bsum_scan_kernel(int64_t* bsum, int64_t nblk);
-__global__ void add_bsum_kernel(int64_t* off, int64_t n, const int64_t* bsum);
+__global__ void cell_hist_kernel(const uint32_t* key, int64_t cells, unsigned* hist);
+__global__ void cell_scan_kernel(const unsigned* hist, CellTables* T);
+__global__ void cell_scatter_kernel(const uint32_t* key, int64_t cells, CellTables* T,
+                                    uint32_t* cellord);
 __global__ void fill_ids_kernel(int64_t n, int64_t first, const int64_t* src, uint32_t mtag,
                                 int64_t* pidx, uint32_t* mtags);
 __global__ void copy_u64_kernel(const unsigned long long* src, unsigned long long* dst,
                                 int64_t n);
-__global__ void cell_items_kernel(int64_t n, int C, const CellStart* rec, int32_t* coff,
-                                  int64_t* pitems);
 __global__ void burn_kernel(const DesignDev* D, const PRates* R, const int32_t* order, int64_t n,
                             uint32_t first, uint32_t k0, uint32_t k1, uint32_t mtag_all,
                             const uint32_t* mtags, const double* betas,
                             const int64_t* goff, unsigned long long* queue, CellStart* rec,
-                            unsigned long long* steps_out, unsigned long long* react_out,
+                            uint32_t* cellkey, unsigned long long* steps_out,
                             const int64_t* pidx, unsigned long long* burn_tally);
-__global__ void ssa_kernel(const DesignDev* D, const PRates* R, const int32_t* order,
-                           const int64_t* off, int64_t n, uint32_t first, uint32_t k0,
+__global__ void ssa_kernel(const DesignDev* D, const PRates* R, const CellTables* tabs,
+                           const uint32_t* cellord, uint32_t first, uint32_t k0,
                            uint32_t k1, uint32_t mtag_all, const uint32_t* mtags,
                            const CellStart* rec,
-                           const int32_t* coff,
                            unsigned long long* queue,
                            uint32_t* out_u, uint32_t* out_l, uint8_t* out_bin,
                            unsigned long long* steps_out,

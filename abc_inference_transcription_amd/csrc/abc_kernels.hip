@@ -5,7 +5,8 @@
 //   rates_kernel ...... log10 parameters -> per-particle rates, thinning
 //                       bounds, periodic gene law, burn-in length, cost key
 //                       (scripts/model.jl:1-43)
-//   bucket_* / *scan .. heaviest-first queue order and work-item offsets
+//   bucket_*, cell_* .. heaviest-first queue orders: particles for the burn-in,
+//                       cells for the window
 //   burn_kernel ....... burn-in of every cell (gene path + Poisson means of the
 //                       unlabelled molecules) up to its labelling window; the
 //                       stochastic counterpart of scripts/model.jl:114-142
@@ -169,7 +170,7 @@ __global__ __launch_bounds__(256) void rates_kernel(const DesignDev* __restrict_
   // Mean birth rate with the gene's activity (before capture): the per-cell
   // split below uses it with the operations of the CPU replay, since it
   // selects random streams.  The typical sub-lanes M of an average cell
-  // (longest window, mean capture) only orders the work queue.
+  // (longest window, mean capture) only orders the burn-in's queue.
   double births = 0.0;
   for (int j = 0; j < nb; ++j) births = births + r.amax[j] * (r.kon[j] / (r.kon[j] + r.koff[j]));
   r.brate = births / (double)nb;
@@ -178,8 +179,6 @@ __global__ __launch_bounds__(256) void rates_kernel(const DesignDev* __restrict_
     const double est = ((r.brate * D->split_scale) * D->wmax) * 3.0;
     while (M < D->split_max && est > D->split_target * (double)M) M *= 2;
   }
-  r.M = M;
-  R[i] = r;
   // Expected Philox draws per work item (a scheduling key only, never a
   // result): gene switches over the whole path + molecule events (births
   // times 1 + splicing + loss, a 1/M share) over about half the longest window.
@@ -191,6 +190,9 @@ __global__ __launch_bounds__(256) void rates_kernel(const DesignDev* __restrict_
     obs += b;
     loss += b * (r.bs / (r.bs + r.gam[j]) + 1.0);
   }
+  r.swrate = (float)(sw / (double)nb);
+  r.gmean = (float)(gsum / (double)nb);
+  R[i] = r;
   cost[i] = (float)((sw / (double)nb) * T * ((double)B + 0.5) +
                     ((obs + loss) / ((double)nb * (double)M)) * (0.5 * D->wmax) + 4.0);
 }
@@ -268,104 +270,87 @@ __global__ __launch_bounds__(256) void copy_u64_kernel(const unsigned long long*
   if (i < n) dst[i] = src[i];
 }
 
-// Sub-lane offsets of every particle's cells after the burn-in: one
-// workgroup per particle scans its cells' M = 2^msh into coff[p * (C + 1) + c]
-// (exclusive; coff[.. + C] is the total) and pitems[p].
-__global__ __launch_bounds__(256) void cell_items_kernel(int64_t n, int C,
-                                                         const CellStart* __restrict__ rec,
-                                                         int32_t* __restrict__ coff,
-                                                         int64_t* __restrict__ pitems) {
-  __shared__ int32_t s[256];
-  const int t = threadIdx.x;
-  const int per = (C + 255) / 256;
-  const int c0 = t * per, c1 = min(C, c0 + per);
-  for (int64_t p = blockIdx.x; p < n; p += gridDim.x) {
-    const CellStart* rp = rec + (size_t)p * (size_t)C;
-    int32_t acc = 0;
-    for (int c = c0; c < c1; ++c) acc += 1 << rp[c].msh;
-    s[t] = acc;
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-      const int32_t x = t >= d ? s[t - d] : 0;
-      __syncthreads();
-      s[t] += x;
-      __syncthreads();
-  }
-  int32_t run = t ? s[t - 1] : 0;
-  int32_t* co = coff + (size_t)p * (size_t)(C + 1);
-  for (int c = c0; c < c1; ++c) {
-    co[c] = run;
-    run += 1 << rp[c].msh;
-  }
-  if (t == 255) {
-    co[C] = s[255];
-    pitems[p] = s[255];
-  }
-  __syncthreads();  // s[] is reused by the next particle
-  }
-}
-
-// Work items of particle rank r = the sub-lanes of all its cells (pitems).
-// off[r + 1] = inclusive sum over ranks <= r, computed per block of
-// ABC_SCAN_BLOCK ranks here (block totals to bsum), then offset by
-// bsum_scan_kernel / add_bsum_kernel.
-__global__ __launch_bounds__(256) void items_scan_kernel(const int64_t* __restrict__ pitems,
-                                                         const int32_t* __restrict__ order,
-                                                         int64_t n, int64_t* __restrict__ off,
-                                                         int64_t* __restrict__ bsum) {
-  constexpr int PER = ABC_SCAN_BLOCK / 256;
-  __shared__ int64_t s[256];
-  const int t = threadIdx.x;
-  const int64_t base = (int64_t)blockIdx.x * ABC_SCAN_BLOCK + (int64_t)t * PER;
-  int64_t v[PER];
-  int64_t acc = 0;
-  for (int q = 0; q < PER; ++q) {
-    const int64_t r = base + q;
-    acc += r < n ? pitems[order[r]] : 0;
-    v[q] = acc;
-  }
-  s[t] = acc;
+// ---------------------------------------------------------- cell queue order
+// ssa_kernel takes the cells of all particles heaviest item first, through a
+// counting sort on the key burn_kernel leaves per cell: bucket = 16 * (cost
+// class of one of the cell's items, a quarter octave) + log2 of its sub-lanes
+// M.  All cells of a bucket have the same M, so a queue position is found from
+// the bucket tables alone: cell cbase + (q - ioff) / M, sub-lane (q - ioff) % M.
+// What sets a launch's end is its last long item: a particle's items differ by
+// their conditions' windows (0.5 to 28 h, a factor of 50 in events), which an
+// order of whole particles left mixed.  ssa_kernel, five configured models:
+// 353 ms in particle order with two items a claim, 335 ms in this order, 296 ms
+// with claims by weight as well (5 x 1,024 particles); 1,068 -> 991 ms at
+// 5 x 4,096; 56 -> 40 ms at 5 x 64, where the longest item sets the time.
+// Ranks run from the heaviest bucket (rank 0 = bucket ABC_CELL_BUCKETS - 1).
+__global__ __launch_bounds__(256) void cell_hist_kernel(const uint32_t* __restrict__ key,
+                                                        int64_t cells,
+                                                        unsigned* __restrict__ hist) {
+  __shared__ unsigned h[ABC_CELL_BUCKETS];
+  for (int b = threadIdx.x; b < ABC_CELL_BUCKETS; b += blockDim.x) h[b] = 0u;
   __syncthreads();
-  for (int d = 1; d < 256; d <<= 1) {
-    const int64_t x = t >= d ? s[t - d] : 0;
-    __syncthreads();
-    s[t] += x;
-    __syncthreads();
-  }
-  const int64_t pre = t ? s[t - 1] : 0;
-  for (int q = 0; q < PER; ++q)
-    if (base + q < n) off[base + q + 1] = pre + v[q];
-  if (t == 255) bsum[blockIdx.x] = s[255];
-  if (blockIdx.x == 0 && t == 0) off[0] = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cells;
+       i += (int64_t)gridDim.x * blockDim.x)
+    atomicAdd(&h[key[i] & (ABC_CELL_BUCKETS - 1)], 1u);
+  __syncthreads();
+  for (int b = threadIdx.x; b < ABC_CELL_BUCKETS; b += blockDim.x)
+    if (h[b]) atomicAdd(&hist[b], h[b]);
 }
 
-// Exclusive scan of nblk block totals in place (launch: 1 x 256).
-__global__ __launch_bounds__(256) void bsum_scan_kernel(int64_t* __restrict__ bsum, int64_t nblk) {
-  __shared__ int64_t s[256];
-  const int t = threadIdx.x;
-  int64_t carry = 0;
-  for (int64_t b0 = 0; b0 < nblk; b0 += 256) {
-    const int64_t b = b0 + t;
-    const int64_t x = b < nblk ? bsum[b] : 0;
-    s[t] = x;
+// Bucket tables by rank (launch: 1 x ABC_CELL_BUCKETS): first cell and first
+// item of the rank (T.ioff[ABC_CELL_BUCKETS]: all items), scatter cursors.
+__global__ __launch_bounds__(ABC_CELL_BUCKETS) void cell_scan_kernel(
+    const unsigned* __restrict__ hist, CellTables* __restrict__ T) {
+  __shared__ unsigned sc[ABC_CELL_BUCKETS];
+  __shared__ unsigned long long si[ABC_CELL_BUCKETS];
+  const int t = threadIdx.x, id = ABC_CELL_BUCKETS - 1 - t;
+  const unsigned x = hist[id];
+  const unsigned long long it = (unsigned long long)x << (id & 15);
+  sc[t] = x;
+  si[t] = it;
+  __syncthreads();
+  for (int d = 1; d < ABC_CELL_BUCKETS; d <<= 1) {
+    const unsigned a = t >= d ? sc[t - d] : 0u;
+    const unsigned long long b = t >= d ? si[t - d] : 0ull;
     __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-      const int64_t y = t >= d ? s[t - d] : 0;
-      __syncthreads();
-      s[t] += y;
-      __syncthreads();
-    }
-    if (b < nblk) bsum[b] = carry + s[t] - x;
-    carry += s[255];
+    sc[t] += a;
+    si[t] += b;
     __syncthreads();
   }
+  T->cbase[t] = sc[t] - x;
+  T->cursor[t] = sc[t] - x;
+  T->ioff[t] = si[t] - it;
+  if (t == ABC_CELL_BUCKETS - 1) T->ioff[ABC_CELL_BUCKETS] = si[t];
 }
 
-__global__ __launch_bounds__(256) void add_bsum_kernel(int64_t* __restrict__ off, int64_t n,
-                                                       const int64_t* __restrict__ bsum) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  off[r + 1] += bsum[r / ABC_SCAN_BLOCK];
+// Each workgroup places a tile of cells: ranks within the tile from LDS
+// counters, one global atomic per bucket and tile, so the cells of a tile
+// (mostly one or two particles) stay together inside a bucket.
+__global__ __launch_bounds__(256) void cell_scatter_kernel(const uint32_t* __restrict__ key,
+                                                           int64_t cells,
+                                                           CellTables* __restrict__ T,
+                                                           uint32_t* __restrict__ cellord) {
+  constexpr int PER = ABC_CELL_TILE / 256;
+  __shared__ unsigned h[ABC_CELL_BUCKETS];
+  for (int b = threadIdx.x; b < ABC_CELL_BUCKETS; b += blockDim.x) h[b] = 0u;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * ABC_CELL_TILE;
+  unsigned k[PER], at[PER];
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int64_t i = base + q * 256 + threadIdx.x;
+    k[q] = i < cells ? key[i] & (ABC_CELL_BUCKETS - 1) : 0u;
+    at[q] = i < cells ? atomicAdd(&h[k[q]], 1u) : 0u;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < ABC_CELL_BUCKETS; b += blockDim.x)
+    if (h[b]) h[b] = atomicAdd(&T->cursor[ABC_CELL_BUCKETS - 1 - b], h[b]);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int64_t i = base + q * 256 + threadIdx.x;
+    if (i < cells) cellord[h[k[q]] + at[q]] = (uint32_t)i;
+  }
 }
 
 // ------------------------------------------------------- shared helpers
@@ -556,8 +541,8 @@ __global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restric
                                                       const int64_t* __restrict__ goff,
                                                       unsigned long long* __restrict__ queue,
                                                       CellStart* __restrict__ rec,
+                                                      uint32_t* __restrict__ cellkey,
                                                       unsigned long long* __restrict__ steps_out,
-                                                      unsigned long long* __restrict__ react_out,
                                                       const int64_t* __restrict__ pidx,
                                                       unsigned long long* __restrict__ burn_tally) {
   const double T = D->T;
@@ -594,7 +579,7 @@ __global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restric
     double ikon = rp->ikon[0], ikoff = rp->ikoff[0];
     double atx = rp->amax[0] * bc, gam = rp->gam[0], bound = D->bound[0];
     double iku = rp->iku[0], ikt = rp->ikt[0], abnd = atx / bound;
-    unsigned long long st = 0, re = 0;
+    unsigned long long st = 0;
     for (;;) {
       double tb = age;
       if (gk < tb) tb = gk;
@@ -618,7 +603,6 @@ __global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restric
       if (tg < tb) {
         t = tg;
         g = !g;
-        re++;
         gneed = true;
         continue;
       }
@@ -675,10 +659,21 @@ __global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restric
         }
       }
       r.msh = (uint8_t)msh;
+      // key of the cell's place in the window queue (a schedule only): expected
+      // draws of one of its items, quarter-octave classes from 4 draws up.
+      // Gene switches of the window; a 1/M share of the births and of the
+      // splicing and loss of those molecules and of the ones at the start
+      const float w = (float)(D->pulse[cond] + D->chase[cond]);
+      const float ps = fminf(1.0f, (float)bs * w), pd = fminf(1.0f, rp->gmean * w);
+      const float mol = (float)lu * ps + (float)lt * pd +
+                        (float)(rp->brate * bc) * w * (1.0f + 0.5f * ps + 0.5f * pd);
+      const float cost = rp->swrate * w + ldexpf(mol, -msh) + 4.0f;
+      int cls = (int)((__float_as_uint(cost) >> 21) & 0x3FFu) - 127 * 4 - 8;
+      cls = cls < 0 ? 0 : (cls > ABC_CELL_BUCKETS / 16 - 1 ? ABC_CELL_BUCKETS / 16 - 1 : cls);
+      cellkey[(size_t)p * (size_t)C + (size_t)c] = (uint32_t)(cls * 16 + msh);
     }
     rec[(size_t)p * (size_t)C + (size_t)c] = r;
     atomicAdd(steps_out + p, st);
-    atomicAdd(react_out + p, re);
     lane_steps += st;
   }
   atomicAdd(burn_tally, lane_steps);
@@ -700,13 +695,12 @@ __global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restric
 // key the same in every lane it fits 128 VGPRs without spilling.
 __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) void ssa_kernel(const DesignDev* __restrict__ D,
                                                      const PRates* __restrict__ R,
-                                                     const int32_t* __restrict__ order,
-                                                     const int64_t* __restrict__ off, int64_t n,
+                                                     const CellTables* __restrict__ tabs,
+                                                     const uint32_t* __restrict__ cellord,
                                                      uint32_t first, uint32_t k0, uint32_t k1,
                                                      uint32_t mtag_all,
                                                      const uint32_t* __restrict__ mtags,
                                                      const CellStart* __restrict__ rec,
-                                                     const int32_t* __restrict__ coff,
                                                      unsigned long long* __restrict__ queue,
                                                      uint32_t* __restrict__ out_u,
                                                      uint32_t* __restrict__ out_l,
@@ -717,14 +711,16 @@ __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) voi
   const double T = D->T;
   const int nb = D->nb, J = D->J, C = D->C;
   const double h = T / (double)nb;  // hours between rate-bin edges
-  const unsigned long long total = (unsigned long long)off[n];
   __shared__ LogEntry ltab[ABC_LOG_N];
   __shared__ LogEntry32 ltab32[ABC_LOG_N];
   __shared__ double rk[ABC_RECIP_N];
+  __shared__ unsigned long long ioff[ABC_CELL_BUCKETS + 1];
   load_log_table(ltab);
   load_log32_table(ltab32);
   for (int q = threadIdx.x; q < ABC_RECIP_N; q += blockDim.x) rk[q] = abc_recip_k[q];
+  for (int q = threadIdx.x; q <= ABC_CELL_BUCKETS; q += blockDim.x) ioff[q] = tabs->ioff[q];
   __syncthreads();
+  const unsigned long long total = ioff[ABC_CELL_BUCKETS];
 
   uint32_t cw = 0;  // counter word of the current item: cell | model << 24
   // per-lane item state
@@ -752,73 +748,56 @@ __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) voi
   bool gneed = false, pend = false;
   double erem = 0.0;
   uint32_t py = 0, pz = 0, pw = 0;
-  // next item of the lane's claim: claim (a power of two) consecutive items
-  // per queue atomic, a launch shape only (items are independent).  The
-  // queue advances by whole claims, so a claim is used up exactly when qnext
-  // reaches a multiple of it.
+  // The lane's claim: qleft more items from queue position qnext on.  A refill
+  // holds up the whole wave for the queue's atomic, so light items are claimed
+  // several at a time, the more the lighter (twice as many per two octaves of
+  // cost, from claim * 2 just below class ABC_LIGHT_CLASS, 2,048 draws); heavy
+  // ones singly, since a second one waiting behind the first would end late.
+  // 5 x 1,024 particles: 329 ms with one item a claim throughout, 312 ms with
+  // claims of `claim` items below class 36, 296 ms so; the line at class 32 or
+  // 40 measured 297 and 299 ms.
   unsigned long long qnext = 0;
-  // where the lane's last item lies, so the next item of the same claim (the
-  // next queue position) is found by one step instead of two searches: queue
-  // rank of its particle, item within the particle, the particle's items,
-  // the end of the cell's sub-lanes (item offsets within the particle) and
-  // the sub-lane
-  int32_t wr = 0, wrem = 0, witems = 0, wcend = 0, wsub = 0;
+  uint32_t qleft = 0;
+  // the bucket that the lane's last item lies in: its rank, first item, the
+  // item after its last and its first cell.  The lane's queue positions only
+  // grow, so the bucket is searched again only once they pass its end.
+  unsigned long long qbase = 0, qend = 0;
+  uint32_t qcell = 0;
+  int qrank = 0;
 
   for (;;) {
     if (!have) {
-      const bool fresh = (qnext & (unsigned long long)(claim - 1u)) == 0ull;
-      if (fresh) qnext = atomicAdd(queue, (unsigned long long)claim);
-      const unsigned long long q = qnext++;
-      if (q >= total) break;
-      if (fresh) {
-        // particle rank: largest r with off[r] <= q
-        int64_t lo = 0, hi = n;
-        while (hi - lo > 1) {
-          const int64_t mid = (lo + hi) >> 1;
-          if ((unsigned long long)off[mid] <= q) lo = mid; else hi = mid;
-        }
-        wr = (int32_t)lo;
-        p = order[lo];
-        wrem = (int32_t)(q - (unsigned long long)off[lo]);
-        witems = (int32_t)(off[lo + 1] - off[lo]);
-        // cell: largest c with coff[c] <= wrem among the particle's C cells
-        const int32_t* co = coff + (size_t)p * (size_t)(C + 1);
-        int clo = 0, chi = C;
-        while (chi - clo > 1) {
-          const int mid = (clo + chi) >> 1;
-          if (co[mid] <= wrem) clo = mid; else chi = mid;
-        }
-        c = clo;
-        wsub = wrem - co[c];
-        wcend = co[c + 1];
-      } else if (++wrem < witems) {
-        // the next item of the same particle: the next sub-lane, or the next
-        // cell's first (every cell has at least one sub-lane)
-        if (wrem < wcend) {
-          wsub++;
-        } else {
-          c++;
-          wsub = 0;
-          wcend = coff[(size_t)p * (size_t)(C + 1) + (size_t)(c + 1)];
-        }
-      } else {
-        // the first item of the next particle in queue order
-        wr++;
-        p = order[wr];
-        wrem = 0;
-        witems = (int32_t)(off[wr + 1] - off[wr]);
-        c = 0;
-        wsub = 0;
-        wcend = coff[(size_t)p * (size_t)(C + 1) + 1];
+      if (qleft == 0u) {
+        const int cls = (ABC_CELL_BUCKETS - 1 - qrank) >> 4;
+        qleft = cls < ABC_LIGHT_CLASS ? claim << ((ABC_LIGHT_CLASS + 8 - cls) >> 3) : 1u;
+        qnext = atomicAdd(queue, (unsigned long long)qleft);
       }
+      const unsigned long long q = qnext++;
+      qleft--;
+      if (q >= total) break;
+      if (q >= qend) {
+        int lo = qrank, hi = ABC_CELL_BUCKETS;  // largest rank with ioff[rank] <= q
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (ioff[mid] <= q) lo = mid; else hi = mid;
+        }
+        qrank = lo;
+        qbase = ioff[lo];
+        qend = ioff[lo + 1];
+        qcell = tabs->cbase[lo];
+      }
+      const int qsh = (ABC_CELL_BUCKETS - 1 - qrank) & 15;
+      const uint32_t cell = cellord[qcell + (uint32_t)((q - qbase) >> qsh)];
+      const int sub = (int)((uint32_t)(q - qbase) & ((1u << qsh) - 1u));
+      p = (int)(cell / (uint32_t)C);
+      c = (int)(cell - (uint32_t)p * (uint32_t)C);
       const PRates* rp = R + p;
-      const int sub = wsub;
       pid = pidx ? (uint32_t)pidx[p] : first + (uint32_t)p;
       cw = (uint32_t)c | (mtags ? mtags[p] : mtag_all);
       sstream = 1u + (uint32_t)sub;
       shi = sstream << 16;
       const CellStart* rc = rec + ((size_t)p * (size_t)C + (size_t)c);
-      ishare = ldexp(1.0, -(int)rc->msh);  // x / M == x * ishare exactly
+      ishare = ldexp(1.0, -qsh);  // x / M == x * ishare exactly
       mctr = 0;
       // every loop-carried value is reset here, so none stays live across the
       // sampler below

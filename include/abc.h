@@ -426,11 +426,10 @@ int32_t abc_screen_score_dev(abc_ctx* ctx, abc_mlp* mlp, int64_t n, const float*
  * default).  Set by the autotuner. */
 int32_t abc_set_ssa_blocks(abc_ctx* ctx, int32_t blocks);
 int32_t abc_get_ssa_blocks(const abc_ctx* ctx);
-/* Work items (cell sub-lanes) a lane of the SSA kernel claims per atomic on
- * its work queue: 1, 2, 4 or 8 consecutive items (default 2, the fastest on
- * the configured workload).  The first item
- * of a claim is located by binary search, the others by a step from the
- * previous one.  Items are independent, so this changes the schedule only.
+/* Unit of the work items (cell sub-lanes) a lane of the SSA kernel claims per
+ * atomic on its work queue: 1, 2, 4 or 8 (default 2).  Items are queued
+ * heaviest first; light ones are claimed in small multiples of the unit, heavy
+ * ones singly.  Items are independent, so this changes the schedule only.
  * Set by the autotuner. */
 int32_t abc_set_ssa_claim(abc_ctx* ctx, int32_t claim);
 int32_t abc_get_ssa_claim(const abc_ctx* ctx);
@@ -440,8 +439,8 @@ int32_t abc_get_ssa_claim(const abc_ctx* ctx);
  * n prior particles (from first) of each listed model, simulates them (all
  * models in one multi-model call, as abc_simulate_multi_dev) once per
  * candidate grid (1, 2, 3, 4, 6, 8, 12, 16 workgroups per CU, up to
- * occupancy) and then, on the fastest grid, twice per queue claim (2, 4 and 8
- * work items per atomic against 1), times ssa_kernel with HIP events and keeps
+ * occupancy) and then, on the fastest grid, twice per queue claim (units of 2, 4
+ * and 8 items against 1), times ssa_kernel with HIP events and keeps
  * the fastest shape for later calls.  Outputs never depend on the shape, so
  * tuning changes speed only.  best_blocks / best_ms (optional) receive the
  * grid and its time; abc_get_ssa_claim gives the claim. */
