@@ -16,7 +16,9 @@
 //   pool_select_kernel keeps each gene's k smallest (error, index) keys
 //     (radix select over the 128-bit key, then a stable in-place compaction)
 //     and lowers thr[g] to the k-th error.
-// pool_sort_kernel orders each gene's final entries by (error, index).
+// list_sort_kernel orders each gene's final entries by (error, index) and packs
+// them into the lists the host receives; the fixed-epsilon rule's accepted pairs
+// reach it through list_scatter_kernel.
 #include <hip/hip_runtime.h>
 
 #include "abc_kernels.h"
@@ -237,24 +239,84 @@ __global__ __launch_bounds__(256) void pool_select_kernel(
   }
 }
 
-// One workgroup per gene (grid-stride): the pool's entries (at most
-// ABC_POOL_SORT_MAX) sorted in place by (error, index), a bitonic sort in LDS.
-__global__ __launch_bounds__(256) void pool_sort_kernel(PoolEntry* __restrict__ pool,
-                                                        int64_t capg,
-                                                        const uint32_t* __restrict__ pool_n,
-                                                        int64_t G) {
+// Exclusive scan of the genes' entry counts (off[G] = all entries); clears the
+// scatter cursors when there are any.  One workgroup, 1,024 genes a turn: the
+// counts of a session are a few kilobytes.
+__global__ __launch_bounds__(1024) void list_scan_kernel(const uint32_t* __restrict__ cnt,
+                                                         int64_t G,
+                                                         unsigned long long* __restrict__ off,
+                                                         uint32_t* __restrict__ cursor) {
+  __shared__ unsigned long long s[1024];
+  const int t = threadIdx.x;
+  unsigned long long carry = 0;
+  for (int64_t g0 = 0; g0 < G; g0 += 1024) {
+    const int64_t g = g0 + t;
+    const unsigned long long x = g < G ? cnt[g] : 0ull;
+    s[t] = x;
+    __syncthreads();
+    for (int d = 1; d < 1024; d <<= 1) {
+      const unsigned long long y = t >= d ? s[t - d] : 0ull;
+      __syncthreads();
+      s[t] += y;
+      __syncthreads();
+    }
+    if (g < G) {
+      off[g] = carry + s[t] - x;
+      if (cursor) cursor[g] = 0u;
+    }
+    carry += s[1023];
+    __syncthreads();
+  }
+  if (t == 0) off[G] = carry;
+}
+
+// The fixed-epsilon rule's accepted pairs grouped by gene: entry q goes to
+// ent[off[gene] + its place among the gene's entries so far].
+__global__ __launch_bounds__(256) void list_scatter_kernel(const Candidate* __restrict__ acc,
+                                                           int64_t n,
+                                                           const unsigned long long* __restrict__ off,
+                                                           uint32_t* __restrict__ cursor,
+                                                           PoolEntry* __restrict__ ent) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const Candidate c = acc[q];
+  ent[off[c.gene] + atomicAdd(cursor + c.gene, 1u)] = PoolEntry{c.err, c.particle};
+}
+
+// One workgroup per gene (grid-stride): the gene's cnt[g] entries, at ent + g *
+// stride (ent + off[g] when stride is 0), sorted by (error, index), go to the
+// flat lists the host receives: 1-based indices and errors from off[g] on.  Up
+// to ABC_POOL_SORT_MAX entries are sorted here, a bitonic sort in LDS; a
+// longer list is copied as it is and sorted by the host.  Sorting and packing
+// on the device instead of on the host: abc_accept_end of 2,000 genes x 1,000
+// entries 33 -> 3 ms, most of it the copy.
+__global__ __launch_bounds__(256) void list_sort_kernel(const PoolEntry* __restrict__ ent,
+                                                        int64_t stride,
+                                                        const uint32_t* __restrict__ n_of,
+                                                        const unsigned long long* __restrict__ off,
+                                                        int64_t G, int64_t* __restrict__ idx_out,
+                                                        double* __restrict__ err_out) {
   __shared__ uint64_t kh[ABC_POOL_SORT_MAX], kl[ABC_POOL_SORT_MAX];
   const int tid = threadIdx.x;
   for (int64_t g = blockIdx.x; g < G; g += gridDim.x) {
-    const int cnt = (int)min((int64_t)pool_n[g], (int64_t)ABC_POOL_SORT_MAX);
-    if (cnt <= 1) continue;  // uniform
-    int N = 2;
+    const int64_t cnt = n_of[g];
+    if (cnt == 0) continue;  // uniform
+    const PoolEntry* pg = stride ? ent + g * stride : ent + off[g];
+    const unsigned long long o = off[g];
+    if (cnt > ABC_POOL_SORT_MAX) {
+      for (int64_t e = tid; e < cnt; e += kWG) {
+        idx_out[o + e] = pg[e].idx + 1;
+        err_out[o + e] = pg[e].err;
+      }
+      continue;
+    }
+    int N = 1;
     while (N < cnt) N <<= 1;
-    PoolEntry* pg = pool + g * capg;
     for (int e = tid; e < N; e += kWG) {
       if (e < cnt) {
-        kh[e] = err_key(pg[e].err);
-        kl[e] = (uint64_t)pg[e].idx;
+        const PoolEntry x = pg[e];
+        kh[e] = err_key(x.err);
+        kl[e] = (uint64_t)x.idx;
       } else {
         kh[e] = ~0ull;
         kl[e] = ~0ull;
@@ -262,10 +324,10 @@ __global__ __launch_bounds__(256) void pool_sort_kernel(PoolEntry* __restrict__ 
     }
     __syncthreads();
     for (int size = 2; size <= N; size <<= 1) {
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int st = size >> 1; st > 0; st >>= 1) {
         for (int t = tid; t < N / 2; t += kWG) {
-          const int i = 2 * t - (t & (stride - 1));
-          const int j = i + stride;
+          const int i = 2 * t - (t & (st - 1));
+          const int j = i + st;
           const bool up = (i & size) == 0;
           const bool gt = !key_le(kh[i], kl[i], kh[j], kl[j]);
           if (gt == up) {
@@ -277,7 +339,10 @@ __global__ __launch_bounds__(256) void pool_sort_kernel(PoolEntry* __restrict__ 
         __syncthreads();
       }
     }
-    for (int e = tid; e < cnt; e += kWG) pg[e] = PoolEntry{key_err(kh[e]), (int64_t)kl[e]};
+    for (int e = tid; e < cnt; e += kWG) {
+      idx_out[o + e] = (int64_t)kl[e] + 1;
+      err_out[o + e] = key_err(kh[e]);
+    }
     __syncthreads();
   }
 }

@@ -74,6 +74,9 @@ struct AcceptState {
   bool pooled = false;
   int64_t n_sub = 0, capg = 0;
   std::vector<double> thr_host;                                // per-gene threshold
+  // fixed epsilon (mode 0): accepted pairs in device memory, and per gene on
+  // the host those moved there when the device list passed its bound
+  int64_t n_acc = 0;
   std::vector<std::vector<std::pair<double, int64_t>>> kept;   // per-gene (err, index)
 };
 
@@ -95,7 +98,7 @@ struct abc_ctx {
   int64_t* d_goff = nullptr;
   DevBuf theta, rates, cost, hist, order, cellord, chist, ctabs, cellrec, cu, cl,
       cb, steps, queue, stats, moments, superset, edata, ese, err, cand, ccount, ah, al,
-      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, presc, apidx, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
+      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, presc, apidx, acclist, accn, accgn, accent, accoff, acccur, accidx, accerr, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
   AcceptState acc;
   hipEvent_t ev[5]{};
   bool timed[4]{};
@@ -150,7 +153,9 @@ hipError_t record(abc_ctx* c, hipEvent_t e) {
       return fail(ctx, ABC_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-int ensure(abc_ctx* c, DevBuf& b, size_t bytes) {
+// in_graphs: captured sequences may hold the buffer's address, so replacing it
+// ends the life of graphs captured before
+int ensure(abc_ctx* c, DevBuf& b, size_t bytes, bool in_graphs = true) {
   if (bytes == 0) bytes = 16;
   if (b.bytes >= bytes) return ABC_OK;
   if (c->capturing)
@@ -163,7 +168,7 @@ int ensure(abc_ctx* c, DevBuf& b, size_t bytes) {
     hipFree(b.p);
     b.p = nullptr;
     b.bytes = 0;
-    c->gen++;
+    if (in_graphs) c->gen++;
   }
   size_t want = bytes + bytes / 4;
   if (hipMalloc(&b.p, want) != hipSuccess) {
@@ -609,7 +614,8 @@ int32_t abc_destroy(abc_ctx* c) {
                     &c->cand, &c->ccount, &c->ah, &c->al, &c->pflag, &c->bh, &c->bl,
                     &c->cg, &c->gflag, &c->thr, &c->wf, &c->sy, &c->tally, &c->mss, &c->mmap, &c->mpidx, &c->mk1, &c->mcost, &c->mord, &c->dmeta, &c->dw,
                     &c->dboot, &c->dflag, &c->du, &c->dl, &c->dout, &c->dsort, &c->dpt, &c->dxs, &c->selb,
-                    &c->pool, &c->pooln, &c->poolb, &c->presc, &c->apidx, &c->thrlow, &c->spass,
+                    &c->pool, &c->pooln, &c->poolb, &c->presc, &c->apidx, &c->acclist, &c->accn, &c->accgn, &c->accent,
+                    &c->accoff, &c->acccur, &c->accidx, &c->accerr, &c->thrlow, &c->spass,
                     &c->mom, &c->mth, &c->mst, &c->selc, &c->selo};
   for (DevBuf* b : bufs)
     if (b->p) hipFree(b->p);
@@ -943,12 +949,6 @@ int32_t abc_errors(abc_ctx* c, int64_t n, int32_t K, const double* stats, int64_
 // ------------------------------------------------------------ accept session
 namespace {
 
-struct GeneHit {
-  double err;
-  int64_t idx;  // global 0-based particle index
-  bool operator<(const GeneHit& o) const { return err < o.err || (err == o.err && idx < o.idx); }
-};
-
 int64_t pad_to(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // Top-k batches (mode 1): screened, rescored and selected per gene entirely
@@ -994,6 +994,49 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
   return ABC_OK;
 }
 
+// Accepted pairs kept in device memory at most (1.6 GB); more move to the host.
+constexpr int64_t kAccOnDevice = (int64_t)1 << 26;
+
+// room for `more` accepted pairs behind the n_acc in the list, which are kept
+int acc_reserve(abc_ctx* c, int64_t more) {
+  AcceptState& A = c->acc;
+  const size_t need = sizeof(Candidate) * (size_t)(A.n_acc + more);
+  if (c->acclist.bytes >= need) return ABC_OK;
+  DevBuf old = c->acclist;
+  c->acclist = DevBuf{};
+  const int rc = ensure(c, c->acclist, need, false);
+  if (rc) {
+    c->acclist = old;
+    return rc;
+  }
+  if (old.p) {
+    if (A.n_acc > 0)
+      HIPCHK(c, hipMemcpyAsync(c->acclist.p, old.p, sizeof(Candidate) * (size_t)A.n_acc,
+                               hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    hipFree(old.p);
+  }
+  return ABC_OK;
+}
+
+// the accepted pairs of the device list into the host's per-gene lists
+int acc_to_host(abc_ctx* c) {
+  AcceptState& A = c->acc;
+  if (A.n_acc == 0) return ABC_OK;
+  std::vector<Candidate> h((size_t)A.n_acc);
+  HIPCHK(c, hipMemcpyAsync(h.data(), c->acclist.p, sizeof(Candidate) * h.size(),
+                           hipMemcpyDeviceToHost, c->stream));
+  hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1((A.G + 1) / 2, 256)), dim3(256), 0, c->stream,
+                     P<unsigned long long>(c->accgn), (A.G + 1) / 2);
+  hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
+                     P<unsigned long long>(c->accn), (int64_t)1);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  for (const Candidate& x : h) A.kept[x.gene].push_back({x.err, x.particle});
+  A.n_acc = 0;
+  return ABC_OK;
+}
+
 int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_index,
                  const int64_t* pidx_host = nullptr) {
   AcceptState& A = c->acc;
@@ -1004,6 +1047,13 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
   if ((rc = ensure(c, c->al, sizeof(uint16_t) * npad * 2 * A.Kp))) return rc;
   if ((rc = ensure(c, c->pflag, npad))) return rc;
   if ((rc = ensure(c, c->ccount, 64))) return rc;
+  const int64_t* pidx_dev = nullptr;
+  if (pidx_host) {
+    if ((rc = ensure(c, c->apidx, sizeof(int64_t) * (size_t)n, false))) return rc;
+    HIPCHK(c, hipMemcpyAsync(c->apidx.p, pidx_host, sizeof(int64_t) * (size_t)n,
+                             hipMemcpyHostToDevice, c->stream));
+    pidx_dev = P<int64_t>(c->apidx);
+  }
   hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 256)), dim3(256), 0, c->stream,
                      stats_dev, n, n, A.E.K, A.Kp, npad, P<__bf16>(c->ah), P<__bf16>(c->al),
                      P<uint8_t>(c->pflag));
@@ -1011,6 +1061,8 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
   unsigned long long cap = std::max<unsigned long long>(A.cand_cap, 1ull << 16);
   for (;;) {
     if ((rc = ensure(c, c->cand, sizeof(Candidate) * cap))) return rc;
+    if (A.n_acc > 0 && A.n_acc + (int64_t)cap > kAccOnDevice && (rc = acc_to_host(c))) return rc;
+    if ((rc = acc_reserve(c, (int64_t)cap))) return rc;
     hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
                        P<unsigned long long>(c->ccount), (int64_t)1);
     hipLaunchKernelGGL(gemm_screen_kernel, dim3((unsigned)(npad / 64), (unsigned)(A.Gpad / 64)),
@@ -1023,10 +1075,13 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
     HIPCHK(c, hipGetLastError());
     hipLaunchKernelGGL(rescore_kernel, dim3(grid1((int64_t)cap, 256)), dim3(256), 0, c->stream,
                        stats_dev, n, P<double>(c->edata), P<double>(c->ese), A.G, A.E,
-                       P<Candidate>(c->cand), P<unsigned long long>(c->ccount), cap);
+                       P<Candidate>(c->cand), P<unsigned long long>(c->ccount), cap, A.eps,
+                       first_index, pidx_dev, P<Candidate>(c->acclist),
+                       P<unsigned long long>(c->accn), P<uint32_t>(c->accgn));
     HIPCHK(c, hipGetLastError());
-    unsigned long long cnt = 0;
+    unsigned long long cnt = 0, nacc = 0;
     HIPCHK(c, hipMemcpyAsync(&cnt, c->ccount.p, 8, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(&nacc, c->accn.p, 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (cnt > cap) {  // grow and screen the batch again (the GEMM is cheap)
       cap = cnt + cnt / 8;
@@ -1034,39 +1089,7 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
       continue;
     }
     A.n_candidates += (int64_t)cnt;
-    std::vector<Candidate> h(cnt);
-    if (cnt)
-      HIPCHK(c, hipMemcpy(h.data(), c->cand.p, sizeof(Candidate) * cnt, hipMemcpyDeviceToHost));
-    std::vector<char> touched(A.mode == 1 ? A.G : 0, 0);
-    for (const Candidate& x : h) {
-      if (!(x.err == x.err)) continue;  // NaN errors are never accepted
-      if (A.mode == 0) {
-        if (x.err <= A.eps) A.kept[x.gene].push_back({x.err, pidx_host ? pidx_host[x.particle] : first_index + x.particle});
-      } else {
-        A.kept[x.gene].push_back({x.err, pidx_host ? pidx_host[x.particle] : first_index + x.particle});
-        touched[x.gene] = 1;
-      }
-    }
-    if (A.mode == 1) {
-      bool changed = false;
-      for (int64_t g = 0; g < A.G; ++g) {
-        if (!touched[g]) continue;
-        auto& v = A.kept[g];
-        if ((int64_t)v.size() > A.k) {
-          std::nth_element(v.begin(), v.begin() + A.k, v.end(),
-                           [](const auto& a, const auto& b) { return GeneHit{a.first, a.second} < GeneHit{b.first, b.second}; });
-          v.resize(A.k);
-        }
-        if ((int64_t)v.size() == A.k && A.k > 0) {
-          double t = v[0].first;
-          for (auto& e : v) t = std::max(t, e.first);
-          if (t != A.thr_host[g]) { A.thr_host[g] = t; changed = true; }
-        }
-      }
-      if (changed)
-        HIPCHK(c, hipMemcpyAsync(c->thr.p, A.thr_host.data(), sizeof(double) * A.G,
-                                 hipMemcpyHostToDevice, c->stream));
-    }
+    A.n_acc = (int64_t)nacc;
     break;
   }
   A.n_screened += n;
@@ -1098,6 +1121,7 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
   A.margin_rel = margin_rel;
   A.n_candidates = 0;
   A.n_screened = 0;
+  A.n_acc = 0;
   A.kept.assign(mode == 1 ? 0 : G, {});
   A.thr_host.assign(std::max<int64_t>(G, 1), mode == 0 ? eps : HUGE_VAL);
   A.pooled = mode == 1;
@@ -1127,6 +1151,14 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
                        P<unsigned long long>(c->poolb), (G + 1) / 2);
     hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
                        P<unsigned long long>(c->presc), (int64_t)1);
+    HIPCHK(c, hipGetLastError());
+  } else {
+    if ((rc = ensure(c, c->accgn, 8 * (size_t)((G + 1) / 2), false))) return rc;
+    if ((rc = ensure(c, c->accn, 8, false))) return rc;
+    hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1((G + 1) / 2, 256)), dim3(256), 0, c->stream,
+                       P<unsigned long long>(c->accgn), (G + 1) / 2);
+    hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
+                       P<unsigned long long>(c->accn), (int64_t)1);
     HIPCHK(c, hipGetLastError());
   }
   if ((rc = ensure(c, c->edata, sizeof(double) * G * K))) return rc;
@@ -1275,47 +1307,106 @@ int32_t abc_accept_end(abc_ctx* c, int64_t* counts, int64_t* idx, double* err_ou
   AcceptState& A = c->acc;
   if (!A.active) return fail(c, ABC_E_ARG, "abc_accept_begin was not called");
   if (A.G > 0 && !counts) return ABC_E_ARG;
-  if (A.pooled && A.G > 0) {
-    // each gene's kept entries: sorted by (error, index) on the device, then copied
-    if (A.k <= ABC_POOL_SORT_MAX) {
-      const int grid = (int)std::min<int64_t>(A.G, (int64_t)c->num_cu * 8);
-      hipLaunchKernelGGL(pool_sort_kernel, dim3(grid), dim3(256), 0, c->stream,
-                         P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln), A.G);
-      HIPCHK(c, hipGetLastError());
-    }
-    std::vector<uint32_t> cnt(A.G);
-    unsigned long long nres = 0;
-    HIPCHK(c, hipMemcpyAsync(cnt.data(), c->pooln.p, sizeof(uint32_t) * A.G,
-                             hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(&nres, c->presc.p, 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    uint32_t mx = 0;
-    for (uint32_t v : cnt) mx = std::max(mx, v);
-    std::vector<PoolEntry> h((size_t)A.G * mx);
-    if (mx)
-      HIPCHK(c, hipMemcpy2D(h.data(), sizeof(PoolEntry) * mx, c->pool.p,
-                            sizeof(PoolEntry) * (size_t)A.capg, sizeof(PoolEntry) * mx, A.G,
-                            hipMemcpyDeviceToHost));
-    A.kept.assign(A.G, {});
+  if (A.G == 0) {
+    if (n_candidates) *n_candidates = 0;
+    A.active = false;
+    return ABC_OK;
+  }
+  int rc;
+  int64_t total = 0;
+  bool on_host = false;
+  if (!A.pooled)
+    for (auto& v : A.kept) on_host |= !v.empty();
+  if (on_host) {
+    // pairs beyond the device list's bound: merged and sorted here
+    if ((rc = acc_to_host(c))) return rc;
     for (int64_t g = 0; g < A.G; ++g) {
       auto& v = A.kept[g];
-      v.reserve(cnt[g]);
-      for (uint32_t q = 0; q < cnt[g]; ++q)
-        v.push_back({h[(size_t)g * mx + q].err, h[(size_t)g * mx + q].idx});
-    }
-    A.n_candidates = (int64_t)nres;
-  }
-  int64_t total = 0;
-  for (int64_t g = 0; g < A.G; ++g) {
-    auto& v = A.kept[g];
-    std::sort(v.begin(), v.end());
-    counts[g] = (int64_t)v.size();
-    for (auto& pr : v) {
-      if (total < cap) {
-        idx[total] = pr.second + 1;
-        if (err_out) err_out[total] = pr.first;
+      std::sort(v.begin(), v.end());
+      counts[g] = (int64_t)v.size();
+      for (auto& pr : v) {
+        if (total < cap) {
+          idx[total] = pr.second + 1;
+          if (err_out) err_out[total] = pr.first;
+        }
+        total++;
       }
-      total++;
+    }
+  } else {
+    // every gene's entries sorted by (error, index) and packed on the device
+    const uint32_t* n_of = P<uint32_t>(A.pooled ? c->pooln : c->accgn);
+    std::vector<uint32_t> cnt((size_t)A.G);
+    unsigned long long nres = 0;
+    HIPCHK(c, hipMemcpyAsync(cnt.data(), n_of, sizeof(uint32_t) * A.G, hipMemcpyDeviceToHost,
+                             c->stream));
+    if (A.pooled)
+      HIPCHK(c, hipMemcpyAsync(&nres, c->presc.p, 8, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (A.pooled) A.n_candidates = (int64_t)nres;
+    bool long_list = false;
+    for (int64_t g = 0; g < A.G; ++g) {
+      counts[g] = (int64_t)cnt[g];
+      total += counts[g];
+      long_list |= cnt[g] > ABC_POOL_SORT_MAX;
+    }
+    const size_t tot = (size_t)total;
+    if (total > 0) {
+      if ((rc = ensure(c, c->accoff, sizeof(uint64_t) * (size_t)(A.G + 1), false))) return rc;
+      if ((rc = ensure(c, c->accidx, sizeof(int64_t) * tot, false))) return rc;
+      if ((rc = ensure(c, c->accerr, sizeof(double) * tot, false))) return rc;
+      unsigned long long* off = P<unsigned long long>(c->accoff);
+      uint32_t* cursor = nullptr;
+      const PoolEntry* ent = P<PoolEntry>(c->pool);
+      if (!A.pooled) {
+        if ((rc = ensure(c, c->accent, sizeof(PoolEntry) * tot, false))) return rc;
+        if ((rc = ensure(c, c->acccur, sizeof(uint32_t) * (size_t)A.G, false))) return rc;
+        cursor = P<uint32_t>(c->acccur);
+        ent = P<PoolEntry>(c->accent);
+      }
+      hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, c->stream, n_of, A.G, off,
+                         cursor);
+      if (!A.pooled)
+        hipLaunchKernelGGL(list_scatter_kernel, dim3(grid1(total, 256)), dim3(256), 0, c->stream,
+                           P<Candidate>(c->acclist), total, off, cursor, P<PoolEntry>(c->accent));
+      hipLaunchKernelGGL(list_sort_kernel, dim3((unsigned)std::min<int64_t>(A.G, 1 << 20)),
+                         dim3(256), 0, c->stream, ent, A.pooled ? A.capg : (int64_t)0, n_of, off,
+                         A.G, P<int64_t>(c->accidx), P<double>(c->accerr));
+      HIPCHK(c, hipGetLastError());
+      if (long_list) {  // lists of more than ABC_POOL_SORT_MAX entries are sorted here
+        std::vector<int64_t> hi(tot);
+        std::vector<double> he(tot);
+        HIPCHK(c, hipMemcpyAsync(hi.data(), c->accidx.p, sizeof(int64_t) * tot,
+                                 hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(he.data(), c->accerr.p, sizeof(double) * tot,
+                                 hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        std::vector<std::pair<double, int64_t>> v;
+        size_t at = 0;
+        for (int64_t g = 0; g < A.G; ++g) {
+          const size_t m = cnt[g];
+          if (m > ABC_POOL_SORT_MAX) {
+            v.resize(m);
+            for (size_t q = 0; q < m; ++q) v[q] = {he[at + q], hi[at + q]};
+            std::sort(v.begin(), v.end());
+            for (size_t q = 0; q < m; ++q) {
+              he[at + q] = v[q].first;
+              hi[at + q] = v[q].second;
+            }
+          }
+          at += m;
+        }
+        const size_t m = std::min(tot, (size_t)cap);
+        std::copy_n(hi.begin(), m, idx);
+        if (err_out) std::copy_n(he.begin(), m, err_out);
+      } else if (cap > 0) {
+        const size_t m = std::min(tot, (size_t)cap);
+        HIPCHK(c, hipMemcpyAsync(idx, c->accidx.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost,
+                                 c->stream));
+        if (err_out)
+          HIPCHK(c, hipMemcpyAsync(err_out, c->accerr.p, sizeof(double) * m, hipMemcpyDeviceToHost,
+                                   c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+      }
     }
   }
   if (n_candidates) *n_candidates = A.n_candidates;

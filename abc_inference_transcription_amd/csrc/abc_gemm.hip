@@ -226,18 +226,27 @@ __global__ __launch_bounds__(256) void gemm_screen_kernel(
   }
 }
 
-// FP64 rescoring of candidates in the reference operation order
-// (compute_errors.jl:30-64).  Candidate.particle holds the batch-local row.
+// FP64 rescoring of the batch's *count candidates in the reference operation
+// order (compute_errors.jl:30-64); those with err <= eps_acc join the session's
+// accepted pairs acc[0 .. *n_acc), counted per gene.  With more candidates than
+// cap the batch is screened again, so nothing is accepted.  Candidate.particle
+// holds the batch-local row on entry, the global particle index (pidx[row], or
+// first_index + row) in acc.
 __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__ stats, int64_t n,
                                                       const double* __restrict__ data,
                                                       const double* __restrict__ se, int64_t G,
-                                                      ErrSpec E, Candidate* __restrict__ cand,
+                                                      ErrSpec E,
+                                                      const Candidate* __restrict__ cand,
                                                       const unsigned long long* __restrict__ count,
-                                                      unsigned long long cap) {
+                                                      unsigned long long cap, double eps_acc,
+                                                      int64_t first_index,
+                                                      const int64_t* __restrict__ pidx,
+                                                      Candidate* __restrict__ acc,
+                                                      unsigned long long* __restrict__ n_acc,
+                                                      uint32_t* __restrict__ gene_n) {
   const unsigned long long q = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned long long m = *count;
-  if (m > cap) m = cap;
-  if (q >= m) return;
+  const unsigned long long m = *count;
+  if (m > cap || q >= m) return;
   Candidate c = cand[q];
   const int64_t i = c.particle, g = c.gene;
   const double s2 = 0.1 * 0.1;
@@ -257,6 +266,10 @@ __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__
     err += e / (double)E.K;
   }
   if (err > E.clamp) err = E.clamp;
-  c.err = err;
-  cand[q] = c;
+  if (err <= eps_acc) {  // never for NaN
+    c.err = err;
+    c.particle = pidx ? pidx[i] : first_index + i;
+    acc[atomicAdd(n_acc, 1ull)] = c;
+    atomicAdd(gene_n + g, 1u);
+  }
 }

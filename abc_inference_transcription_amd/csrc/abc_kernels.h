@@ -206,10 +206,6 @@ __global__ void stats_kernel(const DesignDev* D, const uint32_t* cu, const uint3
                              double* superset);
 __global__ void err_fp64_kernel(const double* stats, int64_t n, const double* data,
                                 const double* se, int64_t G, int64_t g0, ErrSpec E, double* err);
-__global__ void accept_fp64_kernel(const double* stats, int64_t n, const double* data,
-                                   const double* se, int64_t G, int64_t g0, ErrSpec E,
-                                   double eps, int64_t first, Candidate* cand, unsigned long long* count,
-                                   unsigned long long cap);
 __global__ void zero_u64_kernel(unsigned long long* p, int64_t n);
 __global__ void math_probe_kernel(int kind, int64_t n, const double* x, double* y);
 
@@ -244,9 +240,17 @@ __global__ void pool_rescore_kernel(const double* scol, int64_t ld, const double
 __global__ void pool_select_kernel(PoolEntry* pool, int64_t capg, uint32_t* pool_n,
                                    uint32_t* pool_base, int64_t G, int64_t k, double* thr,
                                    unsigned long long* n_rescored);
-__global__ void pool_sort_kernel(PoolEntry* pool, int64_t capg, const uint32_t* pool_n,
-                                 int64_t G);
+__global__ void list_scan_kernel(const uint32_t* cnt, int64_t G, unsigned long long* off,
+                                 uint32_t* cursor);
+__global__ void list_scatter_kernel(const Candidate* acc, int64_t n,
+                                    const unsigned long long* off, uint32_t* cursor,
+                                    PoolEntry* ent);
+__global__ void list_sort_kernel(const PoolEntry* ent, int64_t stride, const uint32_t* n_of,
+                                 const unsigned long long* off, int64_t G, int64_t* idx_out,
+                                 double* err_out);
 __global__ void thr_min_kernel(double* thr, const double* lower, int64_t G);
 __global__ void rescore_kernel(const double* stats, int64_t n, const double* data,
-                               const double* se, int64_t G, ErrSpec E, Candidate* cand,
-                               const unsigned long long* count, unsigned long long cap);
+                               const double* se, int64_t G, ErrSpec E, const Candidate* cand,
+                               const unsigned long long* count, unsigned long long cap,
+                               double eps_acc, int64_t first_index, const int64_t* pidx,
+                               Candidate* acc, unsigned long long* n_acc, uint32_t* gene_n);

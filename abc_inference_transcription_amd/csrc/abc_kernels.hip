@@ -21,8 +21,6 @@
 //                       estimators of scripts/data_summary_statistics.jl)
 //   err_fp64_kernel ... reference-order FP64 error matrix
 //                       (scripts/compute_errors.jl:30-70)
-//   accept_fp64_kernel  fixed-epsilon candidates from the same FP64 errors
-//                       (scripts/accepted_particles.jl:20-22)
 #include "abc_kernels.h"
 
 using namespace abcd;
@@ -1221,25 +1219,6 @@ __global__ __launch_bounds__(256) void err_fp64_kernel(const double* __restrict_
   const int64_t g = g0 + blockIdx.y;
   if (i >= n) return;
   err[i + n * (int64_t)blockIdx.y] = err_pair(data, se, G, g, stats, n, i, E);
-}
-
-__global__ __launch_bounds__(256) void accept_fp64_kernel(const double* __restrict__ stats,
-                                                          int64_t n,
-                                                          const double* __restrict__ data,
-                                                          const double* __restrict__ se,
-                                                          int64_t G, int64_t g0, ErrSpec E,
-                                                          double eps, int64_t first,
-                                                          Candidate* __restrict__ cand,
-                                                          unsigned long long* __restrict__ count,
-                                                          unsigned long long cap) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t g = g0 + blockIdx.y;
-  if (i >= n) return;
-  const double e = err_pair(data, se, G, g, stats, n, i, E);
-  if (e <= eps) {
-    const unsigned long long slot = atomicAdd(count, 1ull);
-    if (slot < cap) cand[slot] = Candidate{e, first + i, (int32_t)g, 0};
-  }
 }
 
 // The device's elementary functions on n inputs, for validation: kind 0 =
