@@ -465,6 +465,29 @@ int make_spec(abc_ctx* c, int K, const int32_t* parts, int n_parts, double clamp
   return ABC_OK;
 }
 
+// Error matrix of n particles x G genes.  64-particle tiles from one workgroup
+// per CU up, 16-particle tiles while those fill most CUs, one lane per pair
+// below that, where a tile's chain over the statistics sets the time (53
+// statistics, us: 1,000 x 1,000 pairs 40 / 41 / 64, 700 x 620 37 / 29 / 38,
+// 300 x 300 35 / 24 / 24, 100 x 500 35 / 24 / 20).
+void launch_errors(abc_ctx* c, int64_t n, const double* stats, int64_t G, const double* data,
+                   const double* se, const ErrSpec& E, double* err) {
+  const int64_t gt = (G + 63) / 64;
+  auto tile = [&](auto kernel, int pt) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 4 * pt - 1) / (4 * pt)), (unsigned)gt),
+                       dim3(256), 0, c->stream, stats, n, n, data, se, G, E, err,
+                       (PoolEntry*)nullptr, (int64_t)0, (int64_t)0, (const int64_t*)nullptr);
+  };
+  if (n >= 16 && gt <= 65535 && (n + 63) / 64 * gt >= c->num_cu) return tile(err_tile_kernel<16, false>, 16);
+  if (n >= 4 && gt <= 65535 && (n + 15) / 16 * gt >= 200) return tile(err_tile_kernel<4, false>, 4);
+  // grid.y is limited to 65535: split genes into slices
+  for (int64_t g0 = 0; g0 < G; g0 += 65535) {
+    const int64_t gn = std::min<int64_t>(65535, G - g0);
+    hipLaunchKernelGGL(err_fp64_kernel, dim3(grid1(n, 256), (unsigned)gn), dim3(256), 0, c->stream,
+                       stats, n, data, se, G, g0, E, err + n * g0);
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -904,12 +927,7 @@ int32_t abc_errors_dev(abc_ctx* c, int64_t n, int32_t K, const double* stats_dev
   if (n == 0 || G == 0) return ABC_OK;
   if (G > 65535 * 64) return fail(c, ABC_E_ARG, "too many genes for one call");
   HIPCHK(c, record(c, c->ev[3]));
-  // grid.y is limited to 65535: split genes into slices
-  for (int64_t g0 = 0; g0 < G; g0 += 65535) {
-    const int64_t gn = std::min<int64_t>(65535, G - g0);
-    hipLaunchKernelGGL(err_fp64_kernel, dim3(grid1(n, 256), (unsigned)gn), dim3(256), 0, c->stream,
-                       stats_dev, n, data_dev, se_dev, G, g0, E, err_dev + n * g0);
-  }
+  launch_errors(c, n, stats_dev, G, data_dev, se_dev, E, err_dev);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, record(c, c->ev[4]));
   c->timed[3] = !c->capturing;
@@ -932,12 +950,8 @@ int32_t abc_errors(abc_ctx* c, int64_t n, int32_t K, const double* stats, int64_
   HIPCHK(c, hipMemcpyAsync(c->stats.p, stats, sizeof(double) * n * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->edata.p, data, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->ese.p, se, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
-  for (int64_t g0 = 0; g0 < G; g0 += 65535) {
-    const int64_t gn = std::min<int64_t>(65535, G - g0);
-    hipLaunchKernelGGL(err_fp64_kernel, dim3(grid1(n, 256), (unsigned)gn), dim3(256), 0, c->stream,
-                       P<double>(c->stats), n, P<double>(c->edata), P<double>(c->ese), G, g0, E,
-                       P<double>(c->err) + n * g0);
-  }
+  launch_errors(c, n, P<double>(c->stats), G, P<double>(c->edata), P<double>(c->ese), E,
+                P<double>(c->err));
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(err, c->err.p, sizeof(double) * n * G, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));

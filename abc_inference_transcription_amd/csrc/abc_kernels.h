@@ -78,6 +78,48 @@ struct ErrSpec {
   double clamp;
 };
 
+// denominator of a squared difference (compute_errors.jl:30-43)
+ABC_DEV double err_den(double d, double sg) {
+  const double s2 = 0.1 * 0.1;
+  const double eps = (sg + d != 0.0) ? 0.0 : 0.0001;
+  return (sg * sg + s2 * (d * d)) + eps;
+}
+
+// ---- x / y for a divisor known in advance, correctly rounded without the
+// division sequence (about 16 issue slots): with zh = RN(1 / y) and zl = 1 / y -
+// zh, q = RN(x zh + RN(x zl)) is within an ulp of x / y, so x - q y is exact in
+// one fused multiply-add and RN(q + (x - q y) zh) is RN(x / y) (Markstein, IBM
+// J. Res. Dev. 34, 1990).  x >= 0; neither x, y nor the quotient may come near
+// the ends of the exponent range: err_range below bounds the operands.
+struct Divisor {
+  double y, zh, zl;
+};
+ABC_DEV Divisor divisor_of(double y) {
+  const double zh = 1.0 / y;
+  return Divisor{y, zh, fma(-zh, y, 1.0) * zh};
+}
+ABC_DEV double div_by(double x, double y, double zh, double zl) {
+  const double q = fma(x, zh, x * zl);
+  return fma(fma(-q, y, x), zh, q);
+}
+// v is zero or 2^-120 <= |v| < 2^200: differences of two such values are zero
+// or at least 2^-172, their squares over a denominator in [2^-300, 2^300] and
+// the remainders above stay normal numbers
+ABC_DEV bool err_range(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t e = (uint32_t)(b >> 52) & 0x7FFu;
+  return (e - (1023u - 120u)) < 320u || (b << 1) == 0ull;
+}
+ABC_DEV bool den_range(double y) {
+  const uint32_t e = (uint32_t)((uint64_t)__double_as_longlong(y) >> 52);  // y > 0: no sign bit
+  return (e - (1023u - 300u)) < 600u;
+}
+
+// One gene's data value and denominator for one statistic.
+struct __align__(32) ErrGene {
+  double d, y, zh, zl;
+};
+
 // One entry of a gene's acceptance pool (abc_accept.hip): the FP64 error
 // and the global 0-based particle index (the batch row until rescored).
 struct PoolEntry {
@@ -206,6 +248,11 @@ __global__ void stats_kernel(const DesignDev* D, const uint32_t* cu, const uint3
                              double* superset);
 __global__ void err_fp64_kernel(const double* stats, int64_t n, const double* data,
                                 const double* se, int64_t G, int64_t g0, ErrSpec E, double* err);
+template <int PT, bool POOL>
+__global__ void err_tile_kernel(const double* stats, int64_t n, int64_t ld, const double* data,
+                                const double* se, int64_t G, ErrSpec E, double* err_out,
+                                PoolEntry* pool, int64_t capg, int64_t first_index,
+                                const int64_t* pidx);
 __global__ void zero_u64_kernel(unsigned long long* p, int64_t n);
 __global__ void math_probe_kernel(int kind, int64_t n, const double* x, double* y);
 
