@@ -98,7 +98,7 @@ struct abc_ctx {
   int64_t* d_goff = nullptr;
   DevBuf theta, rates, cost, hist, order, cellord, chist, ctabs, cellrec, cu, cl,
       cb, steps, queue, stats, moments, superset, edata, ese, err, cand, ccount, ah, al,
-      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, presc, apidx, acclist, accn, accgn, accent, accoff, acccur, accidx, accerr, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
+      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, poolk, presc, apidx, acclist, accn, accgn, accent, accoff, acccur, accidx, accerr, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
   AcceptState acc;
   hipEvent_t ev[5]{};
   bool timed[4]{};
@@ -637,7 +637,7 @@ int32_t abc_destroy(abc_ctx* c) {
                     &c->cand, &c->ccount, &c->ah, &c->al, &c->pflag, &c->bh, &c->bl,
                     &c->cg, &c->gflag, &c->thr, &c->wf, &c->sy, &c->tally, &c->mss, &c->mmap, &c->mpidx, &c->mk1, &c->mcost, &c->mord, &c->dmeta, &c->dw,
                     &c->dboot, &c->dflag, &c->du, &c->dl, &c->dout, &c->dsort, &c->dpt, &c->dxs, &c->selb,
-                    &c->pool, &c->pooln, &c->poolb, &c->presc, &c->apidx, &c->acclist, &c->accn, &c->accgn, &c->accent,
+                    &c->pool, &c->pooln, &c->poolb, &c->poolk, &c->presc, &c->apidx, &c->acclist, &c->accn, &c->accgn, &c->accent,
                     &c->accoff, &c->acccur, &c->accidx, &c->accerr, &c->thrlow, &c->spass,
                     &c->mom, &c->mth, &c->mst, &c->selc, &c->selo};
   for (DevBuf* b : bufs)
@@ -1000,7 +1000,7 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
     hipLaunchKernelGGL(pool_select_kernel, dim3(grid), dim3(256), 0, c->stream,
                        P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln),
                        P<uint32_t>(c->poolb), A.G, A.k, P<double>(c->thr),
-                       P<unsigned long long>(c->presc));
+                       P<unsigned long long>(c->poolk), P<unsigned long long>(c->presc));
     HIPCHK(c, hipGetLastError());
     if (pidx_host) HIPCHK(c, hipStreamSynchronize(c->stream));  // apidx is reused
   }
@@ -1154,6 +1154,7 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
     if ((rc = ensure(c, c->pool, sizeof(PoolEntry) * (size_t)G * (size_t)A.capg))) return rc;
     if ((rc = ensure(c, c->pooln, 8 * (size_t)((G + 1) / 2)))) return rc;
     if ((rc = ensure(c, c->poolb, 8 * (size_t)((G + 1) / 2)))) return rc;
+    if ((rc = ensure(c, c->poolk, 16 * (size_t)G))) return rc;
     if ((rc = ensure(c, c->presc, 8))) return rc;
     if ((rc = ensure(c, c->apidx, sizeof(int64_t) * (size_t)ns))) return rc;
     if ((rc = ensure(c, c->ah, sizeof(uint16_t) * npad * 2 * A.Kp))) return rc;
@@ -1163,6 +1164,8 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
                        P<unsigned long long>(c->pooln), (G + 1) / 2);
     hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1((G + 1) / 2, 256)), dim3(256), 0, c->stream,
                        P<unsigned long long>(c->poolb), (G + 1) / 2);
+    hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(2 * G, 256)), dim3(256), 0, c->stream,
+                       P<unsigned long long>(c->poolk), 2 * G);
     hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
                        P<unsigned long long>(c->presc), (int64_t)1);
     HIPCHK(c, hipGetLastError());

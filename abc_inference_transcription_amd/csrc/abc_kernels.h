@@ -127,6 +127,7 @@ struct PoolEntry {
   int64_t idx;
 };
 #define ABC_POOL_SORT_MAX 2048  // entries per gene sorted on the device
+#define ABC_POOL_LDS 4096       // entries per gene selected in LDS
 
 struct Candidate {
   double err;
@@ -286,6 +287,7 @@ __global__ void pool_rescore_kernel(const double* scol, int64_t ld, const double
                                     const int64_t* pidx);
 __global__ void pool_select_kernel(PoolEntry* pool, int64_t capg, uint32_t* pool_n,
                                    uint32_t* pool_base, int64_t G, int64_t k, double* thr,
+                                   unsigned long long* kth,
                                    unsigned long long* n_rescored);
 __global__ void list_scan_kernel(const uint32_t* cnt, int64_t G, unsigned long long* off,
                                  uint32_t* cursor);

@@ -97,3 +97,29 @@ def test_more_pairs_than_the_device_list(oracle, eng):
     for g in (0, 777, G - 1):
         i, e = _want(oracle, np.vstack(stats), data[g:g + 1], se[g:g + 1], 2 * n)[0]
         assert np.array_equal(idx.reshape(G, -1)[g], i) and np.array_equal(err.reshape(G, -1)[g], e)
+
+
+# rows per batch around what one gene's selection holds in LDS (4,096 live
+# entries: k kept and a batch), later batches with smaller or larger indices,
+# clamped errors (ties decided by the index) and NaN errors among them
+@pytest.mark.parametrize("rows,k,order", [
+    ([4096, 1], 4096, 1), ([4097, 64], 100, -1), ([2000, 2096], 2000, -1),
+    ([2000, 2097], 2000, -1), ([500, 500, 500], 100, 1), ([3000, 3000], 1, -1),
+    ([50, 60, 7000], 5000, 1), ([6000, 6000], 5500, -1)])
+def test_topk_stream_selection(oracle, eng, rows, k, order):
+    stats, data, se = _case(sum(rows), seed=k)
+    data[1:3] = data[1:3] * 1.7          # many errors at the clamp
+    stats[::97] = np.nan
+    firsts, at = [], 0
+    for r in rows:
+        firsts.append(at)
+        at += r
+    err = oracle.errors(stats, data, se, PARTS, clamp=2.0)
+    batches = [(stats[a:a + r], a) for a, r in zip(firsts, rows)][::order]
+    print(f"\n[lists] rows={rows} k={k} order={order}", flush=True)
+    got, _ = eng.accept_stream(batches, data, se, parts=PARTS, clamp=2.0, mode=1, k=k)
+    for g in range(data.shape[0]):
+        o = np.argsort(err[:, g], kind="stable")
+        o = o[~np.isnan(err[o, g])][:k]
+        assert np.array_equal(got[g][0], o + 1), g
+        assert np.array_equal(got[g][1], err[o, g]), g
