@@ -74,47 +74,66 @@ __device__ __forceinline__ unsigned block_scan_flag(bool f, unsigned* scratch, u
 // a gene's new entries come from the screen in nearly increasing row order,
 // so the lanes' loads of one statistic are mostly contiguous.  An entry's
 // index field holds its batch row on entry.
+// The gene's data values, denominators and their reciprocals (genes[g K + k])
+// are uniform over the workgroup: scalar loads, and quotients by the known
+// denominators (div_by) unless the gene (gflag bit 1) or the particle (pflag
+// bit 1) leaves the range for that.  2,000 genes x 4,096 rows x 90 statistics:
+// 522 -> 363 us, bound by the L2 reads of the statistics (16 TB/s).
 __global__ __launch_bounds__(256) void pool_rescore_kernel(
-    const double* __restrict__ scol, int64_t ld, const double* __restrict__ data,
-    const double* __restrict__ se, int64_t G, ErrSpec E, PoolEntry* __restrict__ pool,
-    int64_t capg, const uint32_t* __restrict__ pool_n, const uint32_t* __restrict__ pool_base,
-    int64_t first_index, const int64_t* __restrict__ pidx) {
-  __shared__ double s_d[ABC_MAX_STATS], s_den[ABC_MAX_STATS];
+    const double* __restrict__ scol, int64_t ld, const ErrGene* __restrict__ genes,
+    const uint8_t* __restrict__ gflag, const uint8_t* __restrict__ pflag, int64_t G, ErrSpec E,
+    PoolEntry* __restrict__ pool, int64_t capg, const uint32_t* __restrict__ pool_n,
+    const uint32_t* __restrict__ pool_base, int64_t first_index,
+    const int64_t* __restrict__ pidx) {
   const int K = E.K;
-  const double s2 = 0.1 * 0.1;
+  const Divisor dk = divisor_of((double)K);
   const int64_t stride = (int64_t)kWG * gridDim.y;
   for (int64_t g = blockIdx.x; g < G; g += gridDim.x) {
     const int64_t cnt = min((int64_t)pool_n[g], capg);
     const int64_t b = pool_base[g] + (int64_t)blockIdx.y * kWG;
     if (cnt <= b) continue;  // uniform over the workgroup
-    for (int k = threadIdx.x; k < K; k += kWG) {
-      const double d = data[g + G * k];
-      const double sg = se[g + G * k];
-      const double eps = (sg + d != 0.0) ? 0.0 : 0.0001;
-      s_d[k] = d;
-      s_den[k] = (sg * sg + s2 * (d * d)) + eps;
-    }
-    __syncthreads();
+    const ErrGene* gg = genes + g * K;
+    const bool gbad = (gflag[g] & 2) != 0;
     PoolEntry* pg = pool + g * capg;
     for (int64_t e = b + threadIdx.x; e < cnt; e += stride) {
       const int64_t i = pg[e].idx;
       const double* s = scol + i;
       double err = 0.0;
       int k = 0;
-      for (int pp = 0; pp < E.n_parts; ++pp) {
-        double acc = 0.0;
-        const int end = k + E.parts[pp];
-        for (; k < end; ++k) {
-          const double diff = s_d[k] - s[ld * k];
-          acc += (diff * diff) / s_den[k];
+      if (!gbad && !(pflag[i] & 2)) {
+        for (int pp = 0; pp < E.n_parts; ++pp) {
+          double acc = 0.0;
+          const int end = k + E.parts[pp];
+#pragma unroll 5
+          for (; k < end; ++k) {
+            const ErrGene w = gg[k];
+            const double diff = w.d - s[ld * k];
+            acc += div_by(diff * diff, w.y, w.zh, w.zl);
+          }
+          err += div_by(acc, dk.y, dk.zh, dk.zl);
         }
-        err += acc / (double)K;
+      } else {
+        for (int pp = 0; pp < E.n_parts; ++pp) {
+          double acc = 0.0;
+          const int end = k + E.parts[pp];
+          for (; k < end; ++k) {
+            const double diff = gg[k].d - s[ld * k];
+            acc += (diff * diff) / gg[k].y;
+          }
+          err += acc / (double)K;
+        }
       }
       if (err > E.clamp) err = E.clamp;
       pg[e] = PoolEntry{err, pidx ? pidx[i] : first_index + i};
     }
-    __syncthreads();
   }
+}
+
+// n rows were appended to every gene's pool
+__global__ __launch_bounds__(256) void pool_grow_kernel(uint32_t* __restrict__ pool_n, int64_t G,
+                                                        uint32_t n) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < G) pool_n[g] += n;
 }
 
 // The smallest and largest of a per-thread 64-bit key over the workgroup,

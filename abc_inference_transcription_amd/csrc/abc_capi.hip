@@ -72,6 +72,7 @@ struct AcceptState {
   // top-k (mode 1): per-gene pools of capg = k + n_sub entries in device
   // memory; batches are screened n_sub rows at a time
   bool pooled = false;
+  bool lowered = false;     // thresholds were set by the caller
   int64_t n_sub = 0, capg = 0;
   std::vector<double> thr_host;                                // per-gene threshold
   // fixed epsilon (mode 0): accepted pairs in device memory, and per gene on
@@ -98,7 +99,7 @@ struct abc_ctx {
   int64_t* d_goff = nullptr;
   DevBuf theta, rates, cost, hist, order, cellord, chist, ctabs, cellrec, cu, cl,
       cb, steps, queue, stats, moments, superset, edata, ese, err, cand, ccount, ah, al,
-      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, poolk, presc, apidx, acclist, accn, accgn, accent, accoff, acccur, accidx, accerr, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
+      pflag, bh, bl, cg, gflag, thr, wf, sy, pool, pooln, poolb, poolk, presc, apidx, acclist, accn, accgn, accent, accoff, acccur, accidx, accerr, gtab, thrlow, spass, tally, mss, mmap, mom, mth, mst, selc, selo, mpidx, mk1, mcost, mord, dmeta, dw, dboot, dflag, du, dl, dout, dsort, dpt, dxs, selb;
   AcceptState acc;
   hipEvent_t ev[5]{};
   bool timed[4]{};
@@ -476,7 +477,8 @@ void launch_errors(abc_ctx* c, int64_t n, const double* stats, int64_t G, const 
   auto tile = [&](auto kernel, int pt) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 4 * pt - 1) / (4 * pt)), (unsigned)gt),
                        dim3(256), 0, c->stream, stats, n, n, data, se, G, E, err,
-                       (PoolEntry*)nullptr, (int64_t)0, (int64_t)0, (const int64_t*)nullptr);
+                       (PoolEntry*)nullptr, (int64_t)0, (int64_t)0, (const int64_t*)nullptr,
+                       (const uint32_t*)nullptr);
   };
   if (n >= 16 && gt <= 65535 && (n + 63) / 64 * gt >= c->num_cu) return tile(err_tile_kernel<16, false>, 16);
   if (n >= 4 && gt <= 65535 && (n + 15) / 16 * gt >= 200) return tile(err_tile_kernel<4, false>, 4);
@@ -638,7 +640,7 @@ int32_t abc_destroy(abc_ctx* c) {
                     &c->cg, &c->gflag, &c->thr, &c->wf, &c->sy, &c->tally, &c->mss, &c->mmap, &c->mpidx, &c->mk1, &c->mcost, &c->mord, &c->dmeta, &c->dw,
                     &c->dboot, &c->dflag, &c->du, &c->dl, &c->dout, &c->dsort, &c->dpt, &c->dxs, &c->selb,
                     &c->pool, &c->pooln, &c->poolb, &c->poolk, &c->presc, &c->apidx, &c->acclist, &c->accn, &c->accgn, &c->accent,
-                    &c->accoff, &c->acccur, &c->accidx, &c->accerr, &c->thrlow, &c->spass,
+                    &c->accoff, &c->acccur, &c->accidx, &c->accerr, &c->gtab, &c->thrlow, &c->spass,
                     &c->mom, &c->mth, &c->mst, &c->selc, &c->selo};
   for (DevBuf* b : bufs)
     if (b->p) hipFree(b->p);
@@ -973,6 +975,12 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
                         const int64_t* pidx_host) {
   AcceptState& A = c->acc;
   const int grid = (int)std::min<int64_t>(A.G, (int64_t)c->num_cu * 8);
+  auto launch_select = [&]() {
+    hipLaunchKernelGGL(pool_select_kernel, dim3(grid), dim3(256), 0, c->stream,
+                       P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln),
+                       P<uint32_t>(c->poolb), A.G, A.k, P<double>(c->thr),
+                       P<unsigned long long>(c->poolk), P<unsigned long long>(c->presc));
+  };
   for (int64_t off = 0; off < n; off += A.n_sub) {
     const int64_t nb = std::min(A.n_sub, n - off);
     const int64_t npad = pad_to(nb, 64);
@@ -981,6 +989,24 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
       HIPCHK(c, hipMemcpyAsync(c->apidx.p, pidx_host + off, sizeof(int64_t) * nb,
                                hipMemcpyHostToDevice, c->stream));
       pidx_dev = P<int64_t>(c->apidx);
+    }
+    // Before any threshold every pair is a candidate: the first rows of a
+    // session are rescored densely, without the screen (2,000 genes x 4,096
+    // rows: 258 us against 540 screened).  Not in a captured graph, which may be replayed later.
+    if (A.n_screened + off == 0 && !A.lowered && !c->capturing && nb >= 16) {
+      const int64_t gt = (A.G + 63) / 64;
+      if (gt <= 65535) {
+        hipLaunchKernelGGL((err_tile_kernel<16, true>), dim3((unsigned)((nb + 63) / 64), (unsigned)gt),
+                           dim3(256), 0, c->stream, stats_dev + off, nb, n, P<double>(c->edata),
+                           P<double>(c->ese), A.G, A.E, (double*)nullptr, P<PoolEntry>(c->pool),
+                           A.capg, first_index + off, pidx_dev, P<uint32_t>(c->pooln));
+        hipLaunchKernelGGL(pool_grow_kernel, dim3(grid1(A.G, 256)), dim3(256), 0, c->stream,
+                           P<uint32_t>(c->pooln), A.G, (uint32_t)nb);
+        launch_select();
+        HIPCHK(c, hipGetLastError());
+        if (pidx_host) HIPCHK(c, hipStreamSynchronize(c->stream));  // apidx is reused
+        continue;
+      }
     }
     hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 256)), dim3(256), 0, c->stream,
                        stats_dev + off, nb, n, A.E.K, A.Kp, npad, P<__bf16>(c->ah),
@@ -994,13 +1020,10 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
                        P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln));
     // four workgroups share each gene's new entries
     hipLaunchKernelGGL(pool_rescore_kernel, dim3(grid, 4), dim3(256), 0, c->stream,
-                       stats_dev + off, n, P<double>(c->edata), P<double>(c->ese), A.G, A.E,
-                       P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln),
-                       P<uint32_t>(c->poolb), first_index + off, pidx_dev);
-    hipLaunchKernelGGL(pool_select_kernel, dim3(grid), dim3(256), 0, c->stream,
-                       P<PoolEntry>(c->pool), A.capg, P<uint32_t>(c->pooln),
-                       P<uint32_t>(c->poolb), A.G, A.k, P<double>(c->thr),
-                       P<unsigned long long>(c->poolk), P<unsigned long long>(c->presc));
+                       stats_dev + off, n, P<ErrGene>(c->gtab), P<uint8_t>(c->gflag),
+                       P<uint8_t>(c->pflag), A.G, A.E, P<PoolEntry>(c->pool), A.capg,
+                       P<uint32_t>(c->pooln), P<uint32_t>(c->poolb), first_index + off, pidx_dev);
+    launch_select();
     HIPCHK(c, hipGetLastError());
     if (pidx_host) HIPCHK(c, hipStreamSynchronize(c->stream));  // apidx is reused
   }
@@ -1136,6 +1159,7 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
   A.n_candidates = 0;
   A.n_screened = 0;
   A.n_acc = 0;
+  A.lowered = false;
   A.kept.assign(mode == 1 ? 0 : G, {});
   A.thr_host.assign(std::max<int64_t>(G, 1), mode == 0 ? eps : HUGE_VAL);
   A.pooled = mode == 1;
@@ -1186,13 +1210,14 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
   if ((rc = ensure(c, c->gflag, G))) return rc;
   if ((rc = ensure(c, c->thr, sizeof(double) * G))) return rc;
   if ((rc = ensure(c, c->wf, sizeof(float) * G * K))) return rc;
+  if ((rc = ensure(c, c->gtab, sizeof(ErrGene) * G * K))) return rc;
   HIPCHK(c, hipMemcpyAsync(c->edata.p, data, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->ese.p, se, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->thr.p, A.thr_host.data(), sizeof(double) * G, hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL(gene_prep_kernel, dim3(grid1(A.Gpad, 256)), dim3(256), 0, c->stream,
                      P<double>(c->edata), P<double>(c->ese), G, K, A.Kp, A.Gpad,
                      P<__bf16>(c->bh), P<__bf16>(c->bl), P<double>(c->cg), P<uint8_t>(c->gflag),
-                     P<float>(c->wf));
+                     P<float>(c->wf), P<ErrGene>(c->gtab));
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return ABC_OK;
@@ -1287,6 +1312,7 @@ int32_t abc_accept_set_thresholds(abc_ctx* c, const double* thr) {
   NO_CAPTURE(c);
   AcceptState& A = c->acc;
   if (!A.active) return fail(c, ABC_E_ARG, "abc_accept_begin was not called");
+  A.lowered = true;
   for (int64_t g = 0; g < A.G; ++g) A.thr_host[g] = std::min(A.thr_host[g], thr[g]);
   if (A.G > 0 && A.pooled) {
     // the device thresholds may already be lower (k-th errors found so far)

@@ -33,8 +33,9 @@ __device__ __forceinline__ void split_bf16(double x, bf16* hi, bf16* lo) {
   *lo = (bf16)(float)r;
 }
 
-// One thread per gene: B rows (transposed: Bt[g][k], 2*Kp per gene), c_g and
-// a flag for genes whose weights leave the screened range.
+// One thread per gene: B rows (transposed: Bt[g][k], 2*Kp per gene), c_g, the
+// operands of the FP64 rescoring, and flags for genes whose weights leave the
+// screened range (1) or whose operands leave div_by's (2).
 __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict__ data,
                                                         const double* __restrict__ se, int64_t G,
                                                         int K, int Kp, int64_t Gpad,
@@ -42,7 +43,8 @@ __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict
                                                         bf16* __restrict__ Bl,
                                                         double* __restrict__ cg,
                                                         uint8_t* __restrict__ gflag,
-                                                        float* __restrict__ Wf) {
+                                                        float* __restrict__ Wf,
+                                                        ErrGene* __restrict__ genes) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= Gpad) return;
   bf16* bh = Bh + g * 2 * Kp;
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict
   }
   const double s2 = 0.1 * 0.1;
   double c = 0.0;
-  bool bad = false;
+  bool bad = false, odd = false;
   for (int k = 0; k < Kp; ++k) {
     if (k < K) {
       const double d = data[g + G * k];
@@ -64,6 +66,9 @@ __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict
       const double W = 1.0 / ((double)K * den);
       const double WD = W * d;
       c += WD * d;
+      const Divisor v = divisor_of(den);
+      genes[g * K + k] = ErrGene{d, v.y, v.zh, v.zl};
+      odd |= !err_range(d) || !den_range(den);
       if (!(fabs(W) <= SCREEN_LIMIT) || !(fabs(WD) <= SCREEN_LIMIT)) bad = true;
       Wf[g + G * k] = (float)W;
       split_bf16(-2.0 * WD, bh + k, bl + k);
@@ -74,11 +79,12 @@ __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict
   }
   if (!(c <= SCREEN_LIMIT)) bad = true;
   cg[g] = c;
-  gflag[g] = bad ? 1 : 0;
+  gflag[g] = (bad ? 1 : 0) | (odd ? 2 : 0);
 }
 
-// One thread per particle: A rows [s | s^2] split into bf16 hi/lo.  Row i of
-// the n rows is stats[i + ld * k] (a block of rows of a larger batch).
+// One thread per particle: A rows [s | s^2] split into bf16 hi/lo, and flags
+// as gene_prep_kernel's.  Row i of the n rows is stats[i + ld * k] (a block of
+// rows of a larger batch).
 __global__ __launch_bounds__(256) void particle_prep_kernel(const double* __restrict__ stats,
                                                             int64_t n, int64_t ld, int K, int Kp,
                                                             int64_t npad,
@@ -90,10 +96,11 @@ __global__ __launch_bounds__(256) void particle_prep_kernel(const double* __rest
   bf16* ah = Ah + i * 2 * Kp;
   bf16* al = Al + i * 2 * Kp;
   const bf16 z = (bf16)0.0f;
-  bool bad = false;
+  bool bad = false, odd = false;
   for (int k = 0; k < Kp; ++k) {
     if (i < n && k < K) {
       const double s = stats[i + ld * k];
+      odd |= !err_range(s);
       if (!(fabs(s) <= SCREEN_LIMIT)) bad = true;
       const double sc = bad ? 0.0 : s;
       split_bf16(sc, ah + k, al + k);
@@ -102,7 +109,7 @@ __global__ __launch_bounds__(256) void particle_prep_kernel(const double* __rest
       ah[k] = z; al[k] = z; ah[Kp + k] = z; al[Kp + k] = z;
     }
   }
-  if (i < n) pflag[i] = bad ? 1 : 0;
+  if (i < n) pflag[i] = (bad ? 1 : 0) | (odd ? 2 : 0);
 }
 
 // 256 threads = 4 waves; the workgroup covers 64 particles x 64 genes, each
@@ -168,7 +175,7 @@ __global__ __launch_bounds__(256) void gemm_screen_kernel(
     const bool gok = g < G;
     const double c = gok ? cg[g] : 0.0;
     const double t = gok ? thr[g] : 0.0;
-    const bool gbad = gok && gflag[g] != 0;
+    const bool gbad = gok && (gflag[g] & 1) != 0;
     unsigned cmask = 0;  // bit rb * 4 + q: row i0 + rb * 16 + (lane >> 4) * 4 + q
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
@@ -189,7 +196,7 @@ __global__ __launch_bounds__(256) void gemm_screen_kernel(
         double lo = approx - bound;
         if (t < 1e300) lo -= margin_rel * fabs(t);
         if (lo > clamp) lo = clamp;
-        const bool must = pflag[i] != 0 || gbad;
+        const bool must = (pflag[i] & 1) != 0 || gbad;
         if (must || !(lo > t)) cmask |= 1u << (rb * 4 + q);
       }
     if (pool) {

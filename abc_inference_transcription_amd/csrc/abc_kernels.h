@@ -253,14 +253,14 @@ template <int PT, bool POOL>
 __global__ void err_tile_kernel(const double* stats, int64_t n, int64_t ld, const double* data,
                                 const double* se, int64_t G, ErrSpec E, double* err_out,
                                 PoolEntry* pool, int64_t capg, int64_t first_index,
-                                const int64_t* pidx);
+                                const int64_t* pidx, const uint32_t* pool_n);
 __global__ void zero_u64_kernel(unsigned long long* p, int64_t n);
 __global__ void math_probe_kernel(int kind, int64_t n, const double* x, double* y);
 
 // screening (abc_gemm.hip)
 __global__ void gene_prep_kernel(const double* data, const double* se, int64_t G, int K, int Kp,
                                  int64_t Gpad, __bf16* Bh, __bf16* Bl, double* cg, uint8_t* gflag,
-                                 float* Wf);
+                                 float* Wf, ErrGene* genes);
 // surrogate screen (abc_mlp.hip)
 __global__ void screen_kernel(const float* y, int64_t n, int K, const float* mean, const float* sd,
                               float z, const float* Wf, const double* data, int64_t G,
@@ -280,11 +280,12 @@ __global__ void gemm_screen_kernel(const __bf16* Ah, const __bf16* Al, int64_t n
                                    float* approx_out, float* bound_out, PoolEntry* pool,
                                    int64_t capg, uint32_t* pool_n);
 // per-gene top-k pools (abc_accept.hip)
-__global__ void pool_rescore_kernel(const double* scol, int64_t ld, const double* data,
-                                    const double* se, int64_t G, ErrSpec E, PoolEntry* pool,
-                                    int64_t capg, const uint32_t* pool_n,
-                                    const uint32_t* pool_base, int64_t first_index,
-                                    const int64_t* pidx);
+__global__ void pool_rescore_kernel(const double* scol, int64_t ld, const ErrGene* genes,
+                                    const uint8_t* gflag, const uint8_t* pflag, int64_t G,
+                                    ErrSpec E, PoolEntry* pool, int64_t capg,
+                                    const uint32_t* pool_n, const uint32_t* pool_base,
+                                    int64_t first_index, const int64_t* pidx);
+__global__ void pool_grow_kernel(uint32_t* pool_n, int64_t G, uint32_t n);
 __global__ void pool_select_kernel(PoolEntry* pool, int64_t capg, uint32_t* pool_n,
                                    uint32_t* pool_base, int64_t G, int64_t k, double* thr,
                                    unsigned long long* kth,

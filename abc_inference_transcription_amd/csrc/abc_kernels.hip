@@ -1230,8 +1230,8 @@ __global__ __launch_bounds__(256) void err_fp64_kernel(const double* __restrict_
 // operands leave err_range / den_range (infinite and NaN statistics among
 // them) are formed again by err_pair.  Waves at the end of the particles
 // overlap the ones before (the same values are written twice).  POOL: errors
-// and global particle indices to the genes' acceptance pools instead (row i at
-// entry i), for a batch that meets no threshold yet.
+// and global particle indices behind the pool_n[g] entries of the genes'
+// acceptance pools instead, for a batch that meets no threshold yet.
 // 9,973 particles x 3,419 genes: 1,524 -> 558 us with 53 statistics, 3,093 ->
 // 840 us with 90 (0.65 of the FP64 issue peak by the 7 operations).
 #define ERR_KC 16
@@ -1242,7 +1242,8 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
                                                        ErrSpec E, double* __restrict__ err_out,
                                                        PoolEntry* __restrict__ pool, int64_t capg,
                                                        int64_t first_index,
-                                                       const int64_t* __restrict__ pidx) {
+                                                       const int64_t* __restrict__ pidx,
+                                                       const uint32_t* __restrict__ pool_n) {
   __shared__ double s_d[ERR_KC][64], s_y[ERR_KC][64], s_zh[ERR_KC][64], s_zl[ERR_KC][64];
   __shared__ unsigned long long s_gbad;
   const int lane = threadIdx.x & 63;
@@ -1340,7 +1341,7 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
 #pragma unroll
   for (int p = 0; p < PT; ++p) err[p] += div_by(e[p], dk.y, dk.zh, dk.zl);
   if (g >= G) return;
-  PoolEntry* pg = POOL ? pool + g * capg : nullptr;
+  PoolEntry* pg = POOL ? pool + g * capg + pool_n[g] : nullptr;
   double* eg = POOL ? nullptr : err_out + n * g;
 #pragma unroll
   for (int p = 0; p < PT; ++p) {
@@ -1362,10 +1363,16 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
 
 template __global__ void err_tile_kernel<16, false>(const double*, int64_t, int64_t, const double*,
                                                     const double*, int64_t, ErrSpec, double*,
-                                                    PoolEntry*, int64_t, int64_t, const int64_t*);
+                                                    PoolEntry*, int64_t, int64_t, const int64_t*,
+                                                    const uint32_t*);
+template __global__ void err_tile_kernel<16, true>(const double*, int64_t, int64_t, const double*,
+                                                   const double*, int64_t, ErrSpec, double*,
+                                                   PoolEntry*, int64_t, int64_t, const int64_t*,
+                                                   const uint32_t*);
 template __global__ void err_tile_kernel<4, false>(const double*, int64_t, int64_t, const double*,
                                                    const double*, int64_t, ErrSpec, double*,
-                                                   PoolEntry*, int64_t, int64_t, const int64_t*);
+                                                   PoolEntry*, int64_t, int64_t, const int64_t*,
+                                                    const uint32_t*);
 
 // The device's elementary functions on n inputs, for validation: kind 0 =
 // ex (every kernel except the loops below), 1 = ex_core (the burn-in and the
