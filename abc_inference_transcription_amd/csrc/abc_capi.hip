@@ -1008,7 +1008,7 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
         continue;
       }
     }
-    hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 256)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 16)), dim3(256), 0, c->stream,
                        stats_dev + off, nb, n, A.E.K, A.Kp, npad, P<__bf16>(c->ah),
                        P<__bf16>(c->al), P<uint8_t>(c->pflag));
     hipLaunchKernelGGL(gemm_screen_kernel, dim3((unsigned)(npad / 64), (unsigned)(A.Gpad / 64)),
@@ -1091,7 +1091,7 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
                              hipMemcpyHostToDevice, c->stream));
     pidx_dev = P<int64_t>(c->apidx);
   }
-  hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 256)), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 16)), dim3(256), 0, c->stream,
                      stats_dev, n, n, A.E.K, A.Kp, npad, P<__bf16>(c->ah), P<__bf16>(c->al),
                      P<uint8_t>(c->pflag));
   HIPCHK(c, hipGetLastError());
@@ -1214,7 +1214,7 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
   HIPCHK(c, hipMemcpyAsync(c->edata.p, data, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->ese.p, se, sizeof(double) * G * K, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->thr.p, A.thr_host.data(), sizeof(double) * G, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(gene_prep_kernel, dim3(grid1(A.Gpad, 256)), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(gene_prep_kernel, dim3(grid1(A.Gpad, 16)), dim3(256), 0, c->stream,
                      P<double>(c->edata), P<double>(c->ese), G, K, A.Kp, A.Gpad,
                      P<__bf16>(c->bh), P<__bf16>(c->bl), P<double>(c->cg), P<uint8_t>(c->gflag),
                      P<float>(c->wf), P<ErrGene>(c->gtab));
@@ -1488,7 +1488,7 @@ int32_t abc_screen_errors(abc_ctx* c, int64_t n, int32_t K, const double* stats,
   if ((rc = ensure(c, c->pflag, npad))) return rc;
   if ((rc = ensure(c, c->err, sizeof(float) * 2 * n * G))) return rc;
   HIPCHK(c, hipMemcpyAsync(c->stats.p, stats, sizeof(double) * n * K, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 256)), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(particle_prep_kernel, dim3(grid1(npad, 16)), dim3(256), 0, c->stream,
                      P<double>(c->stats), n, n, K, A.Kp, npad, P<__bf16>(c->ah),
                      P<__bf16>(c->al), P<uint8_t>(c->pflag));
   float* ap = P<float>(c->err);

@@ -123,3 +123,28 @@ def test_topk_stream_selection(oracle, eng, rows, k, order):
         o = o[~np.isnan(err[o, g])][:k]
         assert np.array_equal(got[g][0], o + 1), g
         assert np.array_equal(got[g][1], err[o, g]), g
+
+
+@pytest.mark.parametrize("n,G,K", [(1, 1, 1), (15, 17, 31), (16, 16, 32), (17, 63, 33),
+                                   (64, 65, 127), (129, 33, 128)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_operand_rows_at_their_edges(oracle, eng, mode, n, G, K):
+    """Row remainders of the operand kernels, the statistics' padding, and rows
+    whose statistics leave the screened range (always rescored in FP64)."""
+    rng = np.random.default_rng(n * K)
+    stats = rng.lognormal(0.0, 0.5, (n, K))
+    data = rng.lognormal(0.0, 0.5, (G, K))
+    se = 0.3 * data
+    stats[::5, K // 2] = rng.choice([1e16, np.inf, np.nan, -1e200], len(stats[::5]))
+    data[1::7, K // 3] = 1e-20
+    se[1::7, K // 3] = 0.0
+    parts = np.array([K], np.int32)
+    err = oracle.errors(stats, data, se, parts, clamp=30.0)
+    eps = float(np.nanquantile(err, 0.3))
+    print(f"\n[lists] n={n} G={G} K={K} mode={mode}", flush=True)
+    got = eng.accept(stats, data, se, parts=parts, clamp=30.0, mode=mode, eps=eps, k=7)
+    for g in range(G):
+        o = np.argsort(err[:, g], kind="stable")
+        o = o[~np.isnan(err[o, g])]
+        o = o[:7] if mode else o[err[o, g] <= eps]
+        assert np.array_equal(got[g][0], o + 1) and np.array_equal(got[g][1], err[o, g]), g
