@@ -1760,10 +1760,22 @@ int32_t abc_model_probs(abc_ctx* c, int64_t G, int32_t M, const int64_t* counts,
   const unsigned parts = (unsigned)((n_boot + rpb - 1) / rpb);
   for (int64_t g0 = 0; g0 < G; g0 += chunk) {
     const int64_t cnt = G - g0 < chunk ? G - g0 : chunk;
-    hipLaunchKernelGGL(model_prob_kernel, dim3((unsigned)cnt, parts), dim3(ABC_SEL_WG), 0,
-                       c->stream, G, g0, M, P<int64_t>(c->selc), (uint32_t)seed,
-                       (uint32_t)(seed >> 32) ^ 0x5851F42Du, n_boot, rpb, P<double>(c->selb), o,
-                       o + gm, o + 2 * gm);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)cnt, parts), dim3(ABC_SEL_WG), 0, c->stream, G, g0,
+                         P<int64_t>(c->selc), (uint32_t)seed,
+                         (uint32_t)(seed >> 32) ^ 0x5851F42Du, n_boot, rpb, P<double>(c->selb), o,
+                         o + gm, o + 2 * gm);
+    };
+    switch (M) {
+      case 1: launch(model_prob_kernel<1>); break;
+      case 2: launch(model_prob_kernel<2>); break;
+      case 3: launch(model_prob_kernel<3>); break;
+      case 4: launch(model_prob_kernel<4>); break;
+      case 5: launch(model_prob_kernel<5>); break;
+      case 6: launch(model_prob_kernel<6>); break;
+      case 7: launch(model_prob_kernel<7>); break;
+      default: launch(model_prob_kernel<8>); break;
+    }
     HIPCHK(c, hipGetLastError());
     hipLaunchKernelGGL(model_prob_bounds_kernel, dim3((unsigned)cnt), dim3(ABC_SEL_WG), 0,
                        c->stream, G, g0, M, P<int64_t>(c->selc), n_boot, alpha,

@@ -238,7 +238,8 @@ __global__ void data_se_kernel(int64_t G, int64_t g0, int64_t genes, int nc, int
 #define ABC_SEL_MAX_GROUPS 8
 #define ABC_SEL_MAX_BOOT 256
 #define ABC_SEL_BOOT_PER_WG 8  // resamples per workgroup of model_prob_kernel
-__global__ void model_prob_kernel(int64_t G, int64_t g0, int M, const int64_t* counts,
+template <int M>
+__global__ void model_prob_kernel(int64_t G, int64_t g0, const int64_t* counts,
                                   uint32_t k0, uint32_t k1, int n_boot, int rpb, double* shares,
                                   double* prob, double* lb, double* ub);
 __global__ void model_prob_bounds_kernel(int64_t G, int64_t g0, int M, const int64_t* counts,

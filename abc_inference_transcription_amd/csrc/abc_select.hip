@@ -37,24 +37,36 @@ ABC_DEV double jl_quantile_sorted(const double* v, int n, double p) {
 
 }  // namespace
 
-// Workgroup (x, y): gene g0 + x, resamples y * rpb .. y * rpb + rpb - 1;
-// each resample's share of every group goes to shares[(x M + m) n_boot + b].
-// A gene with at most one accepting group is written here by y = 0.
+// Workgroup (x, y): gene g0 + x, resamples y * rpb .. y * rpb + rpb - 1, one
+// wave per resample; each resample's share of every group goes to
+// shares[(x M + m) n_boot + b].  A gene with at most one accepting group is
+// written here by y = 0.
+// Bound by VALU issue: a label is half a Philox block (30 slots) and one 64-bit
+// comparison per group boundary.  A label idx = floor(u S / 2^64) reaches the
+// cumulative count A (idx >= A) exactly when u >= ceil(A 2^64 / S), so the
+// boundaries are scaled once per workgroup and the index, a 64 x 32
+// multiply-high per label, is never formed; the comparisons are counted by
+// scalar popcounts of their lane masks, the M - 1 counts in scalar registers.  2,000 genes, 2 groups, 33,000 labels a
+// gene on average, 100 resamples: PROB_NOTE
+template <int M>
 __global__ __launch_bounds__(ABC_SEL_WG) void model_prob_kernel(
-    int64_t G, int64_t g0, int M, const int64_t* __restrict__ counts, uint32_t k0, uint32_t k1,
+    int64_t G, int64_t g0, const int64_t* __restrict__ counts, uint32_t k0, uint32_t k1,
     int n_boot, int rpb, double* __restrict__ shares, double* __restrict__ prob,
     double* __restrict__ lb, double* __restrict__ ub) {
-  __shared__ unsigned long long cnt[ABC_SEL_MAX_GROUPS];
   const int64_t gl = blockIdx.x, g = g0 + gl;
   const int tid = threadIdx.x;
-  int64_t l[ABC_SEL_MAX_GROUPS];
   int64_t S = 0;
   int nz = 0, which = -1;
+  // over[k] = ceil(A_k 2^64 / S) - 1 with A_k = l_0 + ... + l_k: a draw u
+  // reaches A_k when u > over[k] (never when A_k = S; always when A_k = 0)
+  uint64_t over[M];
+  bool all[M];
 #pragma unroll
-  for (int m = 0; m < ABC_SEL_MAX_GROUPS; ++m) {
-    l[m] = m < M ? counts[g + G * m] : 0;
-    S += l[m];
-    if (l[m] > 0) {
+  for (int m = 0; m < M; ++m) {
+    const int64_t l = counts[g + G * m];
+    S += l;
+    over[m] = (uint64_t)S;
+    if (l > 0) {
       nz++;
       which = m;
     }
@@ -68,58 +80,71 @@ __global__ __launch_bounds__(ABC_SEL_WG) void model_prob_kernel(
     }
     return;
   }
-  // S < 2^32 (the caller checks it), so with u = hi 2^32 + lo a label
-  // floor(u S / 2^64) = floor((hi S + floor(lo S / 2^32)) / 2^32): the low
-  // word of lo S cannot carry the sum past a multiple of 2^32
-  const uint32_t S32 = (uint32_t)S;
-  // cumulative counts A[k] = l_0 + ... + l_k: a draw's label is the number of
-  // them its index reaches (a prefix, since A is nondecreasing)
-  uint32_t A[ABC_SEL_MAX_GROUPS - 1];
-  {
-    uint32_t acc = 0;
+  const uint32_t S32 = (uint32_t)S;  // S < 2^32 (the caller checks it)
 #pragma unroll
-    for (int k = 0; k < ABC_SEL_MAX_GROUPS - 1; ++k) {
-      acc += (uint32_t)l[k];
-      A[k] = acc;
+  for (int k = 0; k < M - 1; ++k) {
+    const uint64_t A = over[k];
+    all[k] = A == 0;
+    if (A == (uint64_t)S) {
+      over[k] = ~0ull;
+    } else {
+      const uint64_t n1 = A << 32, q1 = n1 / S32, n2 = (n1 - q1 * S32) << 32, q0 = n2 / S32;
+      over[k] = ((q1 << 32) | q0) - (n2 - q0 * S32 == 0 ? 1ull : 0ull);
     }
   }
-  const int64_t pairs = (S + 1) / 2;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b_lo = (int)blockIdx.y * rpb;
   const int b_hi = b_lo + rpb < n_boot ? b_lo + rpb : n_boot;
-  for (int b = b_lo; b < b_hi; ++b) {
-    if (tid < M) cnt[tid] = 0ull;
-    __syncthreads();
-    // this lane's draws, and how many of them reach A[k]: group m has
-    // r[m - 1] - r[m] of them (the draws for r[-1], none for r[M - 1])
-    uint32_t nd = 0u, r[ABC_SEL_MAX_GROUPS - 1];
+  const uint32_t full = S32 >> 1;  // whole blocks of two draws
+  for (int b = b_lo + wave; b < b_hi; b += ABC_SEL_WG / 64) {
+    uint32_t r[M];  // draws that reach A_k, uniform over the wave
 #pragma unroll
-    for (int k = 0; k < ABC_SEL_MAX_GROUPS - 1; ++k) r[k] = 0u;
-    for (int64_t q = tid; q < pairs; q += blockDim.x) {
-      const u4 w = philox((uint32_t)q, (uint32_t)b, (uint32_t)g, 0u, k0, k1);
+    for (int k = 0; k < M; ++k) r[k] = 0u;
+    auto count = [&](uint32_t q, bool in) {
+      const u4 w = philox(q, (uint32_t)b, (uint32_t)g, 0u, k0, k1);
+      const uint64_t ua = (uint64_t)w.y << 32 | w.x, ub_ = (uint64_t)w.w << 32 | w.z;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (2 * q + h >= S) break;
-        const uint32_t lo = h == 0 ? w.x : w.z, hi = h == 0 ? w.y : w.w;
-        const uint32_t idx = (uint32_t)(((uint64_t)hi * S32 + __umulhi(lo, S32)) >> 32);
-        nd++;
+      for (int k = 0; k < M - 1; ++k)
+        r[k] += (uint32_t)__popcll(__ballot(in && ua > over[k])) +
+                (uint32_t)__popcll(__ballot(in && ub_ > over[k]));
+    };
+    uint32_t q0 = 0;  // uniform: the counts stay in scalar registers
+    for (; q0 + 64u <= full; q0 += 64u) count(q0 + (uint32_t)lane, true);
+    if (q0 < full) count(q0 + (uint32_t)lane, q0 + (uint32_t)lane < full);
+    if (S32 & 1u) {  // the last draw of an odd number
+      const u4 w = philox(full, (uint32_t)b, (uint32_t)g, 0u, k0, k1);
+      const uint64_t ua = (uint64_t)w.y << 32 | w.x;
 #pragma unroll
-        for (int k = 0; k < ABC_SEL_MAX_GROUPS - 1; ++k)
-          if (k < M - 1) r[k] += idx >= A[k] ? 1u : 0u;
+      for (int k = 0; k < M - 1; ++k) r[k] += ua > over[k] ? 1u : 0u;
+    }
+    if (lane == 0) {
+      uint32_t reach = S32;
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const uint32_t next = m < M - 1 ? (all[m] ? S32 : r[m]) : 0u;
+        shares[(gl * M + m) * n_boot + b] = (double)(reach - next) / (double)S;
+        reach = next;
       }
     }
-#pragma unroll
-    for (int m = 0; m < ABC_SEL_MAX_GROUPS; ++m) {
-      if (m < M) {
-        const uint32_t reach = m == 0 ? nd : r[m > 0 ? m - 1 : 0];
-        const uint32_t cm = reach - (m < M - 1 ? r[m < ABC_SEL_MAX_GROUPS - 1 ? m : 0] : 0u);
-        if (cm) atomicAdd(&cnt[m], (unsigned long long)cm);
-      }
-    }
-    __syncthreads();
-    if (tid < M) shares[(gl * M + tid) * n_boot + b] = (double)cnt[tid] / (double)S;
-    __syncthreads();
   }
 }
+
+template __global__ void model_prob_kernel<1>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<2>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<3>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<4>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<5>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<6>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<7>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
+template __global__ void model_prob_kernel<8>(int64_t, int64_t, const int64_t*, uint32_t, uint32_t,
+                                              int, int, double*, double*, double*, double*);
 
 // One workgroup per gene g0 + x with two or more accepting groups: each
 // group's n_boot shares in ascending order (value i goes to place #{j: x_j <
