@@ -1552,6 +1552,26 @@ int moment_cfg(abc_ctx* c, int model, const abc_moment_cfg* u, MomCfgDev* m) {
   return ABC_OK;
 }
 
+// Particles, the costliest first, that the integrating kernels give to teams of
+// eight lanes (a multiple of 8).  Teams shorten an integration's chain 2.6 times
+// for about 2.4 times the issue slots, so they pay while the longest chains set
+// the time: for nearly all particles of a small call, for ever fewer of the
+// costliest as the call fills the machine.  Team waves 0 / 512 / 2,048 / 16,384,
+// ms per call of models 1 to 5 (reference prior): n = 4,096 model 1 62 / 36 / 30 /
+// 26, model 4 72 / 56 / 51 / 43; n = 8,192 model 3 139 / 87 / 66 / 69, model 5
+// 91 / 92 / 95 / 114; n = 32,768 model 3 155 / 144 / 153 / 192, model 5 248 / 252 /
+// 259 / 314.
+int64_t moment_heavy(int64_t n, int64_t items) {
+  const int64_t waves = n <= 4096 ? 16384 : (n <= 12288 ? 1024 : 512);
+  return std::min<int64_t>((n + 7) / 8, waves / items) * 8;
+}
+
+// waves of a launch: teams of eight particles each, then 64 particles each
+unsigned moment_waves(int64_t n, int64_t heavy, int64_t items) {
+  const int64_t rest = std::max<int64_t>(n - heavy, 0);
+  return (unsigned)((heavy / 8 + (rest + 63) / 64) * items);
+}
+
 // transient -> trajectories (-> downsampling and statistics when stats_dev)
 int moment_run(abc_ctx* c, int model, int64_t n, const double* theta_dev, int64_t ld,
                const MomCfgDev& m, double* out_dev, int64_t* steps_dev, double* stats_dev) {
@@ -1574,14 +1594,14 @@ int moment_run(abc_ctx* c, int model, int64_t n, const double* theta_dev, int64_
   hipLaunchKernelGGL(moment_order_kernel, dim3(1), dim3(ABC_MOM_ORDER_WG), 0, c->stream, n, key,
                      ord_map);
   hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(n, 256)), dim3(256), 0, c->stream, cost, n);
-  if (m.method == 1)
-    hipLaunchKernelGGL(moment_cyclemap_kernel<1>, dim3((unsigned)((n + 63) / 64 * 10)), dim3(64),
-                       0, c->stream, m, model, n, theta_dev, ld, ord_map, P<double>(c->mmap), cost,
-                       steps);
-  else
-    hipLaunchKernelGGL(moment_cyclemap_kernel<0>, dim3((unsigned)((n + 63) / 64 * 10)), dim3(64),
-                       0, c->stream, m, model, n, theta_dev, ld, ord_map, P<double>(c->mmap), cost,
-                       steps);
+  const int64_t hc = m.method == 1 ? moment_heavy(n, 10) : 0;
+  const unsigned wc = moment_waves(n, hc, 10);
+  auto cyclemap = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(wc), dim3(64), 0, c->stream, m, model, n, theta_dev, ld, ord_map,
+                       hc, P<double>(c->mmap), cost, steps);
+  };
+  if (m.method == 1) cyclemap(moment_cyclemap_kernel<1>);
+  else cyclemap(moment_cyclemap_kernel<0>);
   HIPCHK(c, hipGetLastError());
   hipLaunchKernelGGL(moment_order_kernel, dim3(1), dim3(ABC_MOM_ORDER_WG), 0, c->stream, n, cost,
                      ord);
@@ -1589,16 +1609,16 @@ int moment_run(abc_ctx* c, int model, int64_t n, const double* theta_dev, int64_
   hipLaunchKernelGGL(moment_transient_kernel, dim3(grid1(n, 64)), dim3(64), 0, c->stream, m, n,
                      P<double>(c->mmap), P<double>(c->mss));
   HIPCHK(c, hipGetLastError());
-  // one wave per (group of 64 ordered particles, condition x age item)
-  const int64_t waves = (n + 63) / 64 * (int64_t)m.n_conds * m.n_ages;
-  if (m.method == 1)
-    hipLaunchKernelGGL(moment_traj_kernel<1>, dim3((unsigned)waves), dim3(64), 0, c->stream, m,
-                       model, n, theta_dev, ld, P<double>(c->mss), P<double>(c->mmap), ord,
-                       out_dev, steps);
-  else
-    hipLaunchKernelGGL(moment_traj_kernel<0>, dim3((unsigned)waves), dim3(64), 0, c->stream, m,
-                       model, n, theta_dev, ld, P<double>(c->mss), P<double>(c->mmap), ord,
-                       out_dev, steps);
+  // one wave per (group of ordered particles, condition x age item)
+  const int64_t items = (int64_t)m.n_conds * m.n_ages;
+  const int64_t ht = m.method == 1 ? moment_heavy(n, items) : 0;
+  const unsigned wt = moment_waves(n, ht, items);
+  auto traj = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(wt), dim3(64), 0, c->stream, m, model, n, theta_dev, ld,
+                       P<double>(c->mss), P<double>(c->mmap), ord, ht, out_dev, steps);
+  };
+  if (m.method == 1) traj(moment_traj_kernel<1>);
+  else traj(moment_traj_kernel<0>);
   HIPCHK(c, hipGetLastError());
   if (stats_dev) {
     hipLaunchKernelGGL(moment_stats_kernel, dim3(grid1(n, 64)), dim3(64), 0, c->stream, m, n,

@@ -192,7 +192,7 @@ struct MomCfgDev {
 template <int METHOD>
 __global__ void moment_cyclemap_kernel(MomCfgDev cfg, int model, int64_t n,
                                        const double* theta, int64_t ld, const int32_t* order,
-                                       double* maps, unsigned long long* cost,
+                                       int64_t heavy, double* maps, unsigned long long* cost,
                                        unsigned long long* steps);
 __global__ void moment_key_kernel(MomCfgDev cfg, int model, int64_t n, const double* theta,
                                   int64_t ld, unsigned long long* cost);
@@ -205,7 +205,8 @@ __global__ void moment_transient_kernel(MomCfgDev cfg, int64_t n, const double* 
 template <int METHOD>
 __global__ void moment_traj_kernel(MomCfgDev cfg, int model, int64_t n,
                                    const double* theta, int64_t ld, const double* ss,
-                                   const double* maps, const int32_t* order, double* out,
+                                   const double* maps, const int32_t* order, int64_t heavy,
+                                   double* out,
                                    unsigned long long* steps);
 __global__ void moment_stats_kernel(MomCfgDev cfg, int64_t n, double* mom,
                                     double* stats);

@@ -25,7 +25,8 @@
 // vector) integrates the 10 cycle maps that fix the affine cycle map;
 // moment_transient_kernel: one lane per particle finds the periodic state
 // from it.  moment_traj_kernel: one lane
-// per (particle, condition, age) integrates that state from t0 to the age;
+// per (particle, condition, age) integrates that state from t0 to the age
+// (a team of eight lanes instead of one for the costliest particles, method 1);
 // the items of a particle are adjacent, so the lanes of a wavefront share
 // their rates (and their stiffness, which sets the step count).
 // moment_stats_kernel: one lane per particle downsamples the moments and forms
@@ -117,14 +118,25 @@ ABC_DEV Piece make_piece(const Particle& P, const MomCfgDev& cfg, double texp, d
   return pc;
 }
 
+// The cycle length as a divisor.  a / T with a in [0, T] by four operations
+// (div_by: correctly rounded) while T lies well inside the exponent range, by a
+// division otherwise.  (A quotient too small for div_by is lost against the 1
+// it is added to.)
+struct Cycle {
+  double T;
+  Divisor d;
+  bool fast;
+};
+ABC_DEV Cycle cycle_of(double T) { return Cycle{T, divisor_of(T), T > 0x1p-100 && T < 0x1p100}; }
+
 // rates at time t inside the piece: alpha carries the size scaling 1 + a/T
-ABC_DEV void rates(const Piece& pc, const Particle& P, double cycle, double t, double* p) {
+ABC_DEV void rates(const Piece& pc, const Particle& P, const Cycle& cyc, double t, double* p) {
   p[0] = pc.base[0];
   p[1] = pc.base[1];
   double al = pc.base[2];
   if (P.scaling) {
     const double a = t - pc.cs;
-    al = al * (1.0 + a / cycle);
+    al = al * (1.0 + (cyc.fast ? div_by(a, cyc.d.y, cyc.d.zh, cyc.d.zl) : a / cyc.T));
   }
   p[2] = al;
   p[3] = pc.base[3];
@@ -143,7 +155,7 @@ ABC_DEV void rhs(const double* p, double lam, const double* y, double* dy) {
   dy[8] = p[2] * lam * y[0] + p[3] * y[2] + 2 * p[2] * lam * y[5] - 2 * p[3] * y[8];
 }
 
-ABC_DEV void eval(const Piece& pc, const Particle& P, double cycle, double t, const double* y,
+ABC_DEV void eval(const Piece& pc, const Particle& P, const Cycle& cycle, double t, const double* y,
                   double* dy) {
   double p[4];
   rates(pc, P, cycle, t, p);
@@ -156,7 +168,8 @@ ABC_DEV int64_t dopri_piece(const Piece& pc, const Particle& P, const MomCfgDev&
                             double b, double* y, const LogEntry* ltab) {
   const double len = b - a;
   if (len <= 0) return 0;
-  const double cyc = cfg.cycle, rtol = cfg.rtol, atol = cfg.atol;
+  const Cycle cyc = cycle_of(cfg.cycle);
+  const double rtol = cfg.rtol, atol = cfg.atol;
   double t = a;
   double h = len < 1e-2 ? len : 1e-2;
   double k1[9], k2[9], k3[9], k4[9], k5[9], k6[9], k7[9], yt[9], yn[9];
@@ -311,10 +324,11 @@ ABC_DEV int64_t egb_piece(const Piece& pc, const Particle& P, const MomCfgDev& c
   constexpr int Z[5] = {1, 2, 6, 7, 8};
   const double len = b - a;
   if (len <= 0) return 0;
-  const double cyc = cfg.cycle, rtol = cfg.rtol, atol = cfg.atol;
+  const Cycle cyc = cycle_of(cfg.cycle);
+  const double rtol = cfg.rtol, atol = cfg.atol;
   double p[4];
   rates(pc, P, cyc, a, p);
-  const double al1 = P.scaling ? pc.base[2] / cyc : 0.0;
+  const double al1 = P.scaling ? pc.base[2] / cyc.T : 0.0;
   GBlock q;
   gb_setup(q, p, al1, pc.lam, y);
   double t = a;
@@ -410,9 +424,10 @@ ABC_DEV int64_t egb_piece(const Piece& pc, const Particle& P, const MomCfgDev& c
 // at the window edges texp, texp + pulse.  The edges are generated in
 // ascending order (a sorted merge of the grid with the two window edges);
 // coincident edges give empty pieces, which are skipped.
-template <int METHOD>
-ABC_DEV int64_t moment_solve(const Particle& P, const MomCfgDev& cfg, double texp, double pulse,
-                             double tmin, double tmax, double* y, const LogEntry* ltab) {
+// piece(pc, a, b) integrates one piece and returns its steps.
+template <class Integrate>
+ABC_DEV int64_t moment_pieces(const Particle& P, const MomCfgDev& cfg, double texp, double pulse,
+                              double tmin, double tmax, Integrate piece) {
   const double h = cfg.cycle / cfg.n_steps;
   double k = floor(tmin / h) + 1.0;
   const double we = texp + pulse;
@@ -441,13 +456,21 @@ ABC_DEV int64_t moment_solve(const Particle& P, const MomCfgDev& cfg, double tex
     if (b > a) {
       const double tb = 0.5 * (a + b);
       const Piece pc = make_piece(P, cfg, texp, pulse, tb);
-      steps += METHOD == 1 ? egb_piece(pc, P, cfg, a, b, y, ltab)
-                           : dopri_piece(pc, P, cfg, a, b, y, ltab);
+      steps += piece(pc, a, b);
       a = b;
     }
     if (src < 0) break;
   }
   return steps;
+}
+
+template <int METHOD>
+ABC_DEV int64_t moment_solve(const Particle& P, const MomCfgDev& cfg, double texp, double pulse,
+                             double tmin, double tmax, double* y, const LogEntry* ltab) {
+  return moment_pieces(P, cfg, texp, pulse, tmin, tmax, [&](const Piece& pc, double a, double b) {
+    return METHOD == 1 ? egb_piece(pc, P, cfg, a, b, y, ltab)
+                       : dopri_piece(pc, P, cfg, a, b, y, ltab);
+  });
 }
 
 // binomial partitioning at division (model.jl:98-111)
@@ -461,6 +484,202 @@ ABC_DEV void periodic_boundary(const double* e, double* v) {
   v[7] = e[7] / 4;
   v[1] = e[1] / 2;
   v[2] = e[2] / 2;
+}
+
+// ---- method 1 by a team of eight lanes: one integration with a shorter chain.
+// Of the about 1,300 to 2,000 instructions of a step (by how many of the
+// exponential integrals take the series), more than half evaluate the gene
+// block at the five stage times, which does not depend on the other moments:
+// lane r < 5 does it for stage r + 2.  Lane 0 then carries E u and Var u, lane 1
+// E l and Var l, lane 2 Cov ul; every lane takes the same step decisions.  Each
+// value is formed by the operations of egb_piece in the same order, so the
+// results and the steps are the same bits.  About 600 instructions and 4,600
+// cycles a step against 2,000 and 13,700 by one lane; 503 particles of model 3
+// (27,665 trajectories, the machine mostly idle): 96 -> 36 ms, 4,096 of model 4:
+// 72 -> 43 ms.
+constexpr int kTeam = 8, kTeams = 64 / kTeam;
+
+// what a stage time contributes to the five right-hand sides
+struct Forcing {
+  double f[5];  // alpha (1 - lam) E g, alpha lam E g, the Cov g terms of Var u, Cov ul, Var l
+};
+
+ABC_DEV Forcing forcing_of(const double* p, double lam, const double* y) {
+  Forcing o;
+  o.f[0] = (1 - lam) * p[2] * y[0];
+  o.f[1] = lam * p[2] * y[0];
+  o.f[2] = 2 * p[2] * (1 - lam) * y[4];
+  o.f[3] = p[2] * lam * y[4] + p[2] * (1 - lam) * y[5];
+  o.f[4] = 2 * p[2] * lam * y[5];
+  return o;
+}
+
+// a lane's share of the state: the gene block (every lane) and its moments
+struct TeamState {
+  double g[9];  // entries 0, 3, 4, 5
+  double m, v;  // lane 0: E u, Var u; lane 1: E l, Var l; lane 2: -, Cov ul; others zero
+};
+
+struct TeamLane {
+  int r;            // lane within the team
+  int base;         // the team's first lane of the wave
+  double (*F)[5];   // the team's stage forcings in LDS
+};
+
+ABC_DEV int64_t egb_piece_team(const Piece& pc, const Particle& P, const MomCfgDev& cfg, double a,
+                               double b, TeamState& S, const TeamLane& L, const LogEntry* ltab) {
+  const double len = b - a;
+  if (len <= 0) return 0;
+  const Cycle cyc = cycle_of(cfg.cycle);
+  const double rtol = cfg.rtol, atol = cfg.atol;
+  const bool first = L.r < 2, second = L.r < 3;  // lanes with a mean, with a (co)variance
+  // this lane's two forcings
+  const int im = L.r == 0 ? 0 : (L.r == 1 ? 1 : 3), iv = L.r == 0 ? 2 : 4;
+  const double cr = L.r == 0 ? kC2 : (L.r == 1 ? kC3 : (L.r == 2 ? kC4 : (L.r == 3 ? kC5 : 1.0)));
+  double p[4];
+  rates(pc, P, cyc, a, p);
+  const double al1 = P.scaling ? pc.base[2] / cyc.T : 0.0;
+  GBlock q;
+  gb_setup(q, p, al1, pc.lam, S.g);
+  const double ga = p[3], ga2 = 2 * p[3];
+  auto dmean = [&](double f, double m) { return first ? f - ga * m : 0.0; };
+  auto dvar = [&](double f, double g, double m, double v) {
+    const double s = first ? (f + ga * m) + g : f;
+    return second ? s - ga2 * v : 0.0;
+  };
+  double t = a;
+  double h = len < 1e-2 ? len : 1e-2;
+  double ys[9], m = S.m, v = S.v;
+  double km[8], kv[8];
+  int64_t steps = 0;
+  {
+    gb_eval(q, t - a, ys);
+    const Forcing f0 = forcing_of(p, pc.lam, ys);
+    const double fm = im == 0 ? f0.f[0] : (im == 1 ? f0.f[1] : f0.f[3]);
+    const double fv = iv == 2 ? f0.f[2] : f0.f[4];
+    km[1] = dmean(fm, m);
+    kv[1] = dvar(fm, fv, m, v);
+  }
+  while (t < b) {
+    if (t + h > b) h = b - t;
+    {
+      const double ts = t + cr * h;
+      gb_eval(q, ts - a, ys);
+      rates(pc, P, cyc, ts, p);
+      const Forcing f = forcing_of(p, pc.lam, ys);
+      if (L.r < 5) {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) L.F[L.r][i] = f.f[i];
+      }
+    }
+    // the team is in one wave: its LDS accesses complete in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    double fm[7], fv[7];
+#pragma unroll
+    for (int i = 2; i < 7; ++i) {
+      fm[i] = L.F[i - 2][im];
+      fv[i] = L.F[i - 2][iv];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    double xm, xv;
+    xm = m + h * (kA21 * km[1]);
+    xv = v + h * (kA21 * kv[1]);
+    km[2] = dmean(fm[2], xm);
+    kv[2] = dvar(fm[2], fv[2], xm, xv);
+    xm = m + h * (kA31 * km[1] + kA32 * km[2]);
+    xv = v + h * (kA31 * kv[1] + kA32 * kv[2]);
+    km[3] = dmean(fm[3], xm);
+    kv[3] = dvar(fm[3], fv[3], xm, xv);
+    xm = m + h * (kA41 * km[1] + kA42 * km[2] + kA43 * km[3]);
+    xv = v + h * (kA41 * kv[1] + kA42 * kv[2] + kA43 * kv[3]);
+    km[4] = dmean(fm[4], xm);
+    kv[4] = dvar(fm[4], fv[4], xm, xv);
+    xm = m + h * (kA51 * km[1] + kA52 * km[2] + kA53 * km[3] + kA54 * km[4]);
+    xv = v + h * (kA51 * kv[1] + kA52 * kv[2] + kA53 * kv[3] + kA54 * kv[4]);
+    km[5] = dmean(fm[5], xm);
+    kv[5] = dvar(fm[5], fv[5], xm, xv);
+    xm = m + h * (kA61 * km[1] + kA62 * km[2] + kA63 * km[3] + kA64 * km[4] + kA65 * km[5]);
+    xv = v + h * (kA61 * kv[1] + kA62 * kv[2] + kA63 * kv[3] + kA64 * kv[4] + kA65 * kv[5]);
+    km[6] = dmean(fm[6], xm);
+    kv[6] = dvar(fm[6], fv[6], xm, xv);
+    const double nm = m + h * (kB1 * km[1] + kB3 * km[3] + kB4 * km[4] + kB5 * km[5] + kB6 * km[6]);
+    const double nv = v + h * (kB1 * kv[1] + kB3 * kv[3] + kB4 * kv[4] + kB5 * kv[5] + kB6 * kv[6]);
+    km[7] = dmean(fm[6], nm);
+    kv[7] = dvar(fm[6], fv[6], nm, nv);
+    double err = 0.0;
+    {
+      const double em = h * (kE1 * km[1] + kE3 * km[3] + kE4 * km[4] + kE5 * km[5] + kE6 * km[6] +
+                             kE7 * km[7]);
+      const double ev = h * (kE1 * kv[1] + kE3 * kv[3] + kE4 * kv[4] + kE5 * kv[5] + kE6 * kv[6] +
+                             kE7 * kv[7]);
+      const double rm = fabs(em) / (atol + rtol * fmax(fabs(m), fabs(nm)));
+      const double rv = fabs(ev) / (atol + rtol * fmax(fabs(v), fabs(nv)));
+      if (rm > err) err = rm;
+      if (rv > err) err = rv;
+#pragma unroll
+      for (int o = 1; o < kTeam; o <<= 1) {
+        const double x = __shfl_xor(err, o);
+        if (x > err) err = x;
+      }
+    }
+    steps++;
+    if (err <= 1.0) {
+      t += h;
+      m = nm;
+      v = nv;
+      km[1] = km[7];
+      kv[1] = kv[7];
+      S.g[0] = ys[0];  // at t on the lanes from 4 on
+      S.g[3] = ys[3];
+      S.g[4] = ys[4];
+      S.g[5] = ys[5];
+      double fac = err == 0.0 ? 5.0 : 0.9 * ex_core(-0.2 * ln(err, ltab));
+      if (fac > 5.0) fac = 5.0;
+      h *= fac;
+    } else {
+      double fac = 0.9 * ex_core(-0.2 * ln(err, ltab));
+      if (fac < 0.2) fac = 0.2;
+      h *= fac;
+    }
+    if (h < 1e-14 * (fabs(t) + 1.0)) h = 1e-14 * (fabs(t) + 1.0);
+  }
+  S.m = m;
+  S.v = v;
+  S.g[0] = __shfl(S.g[0], L.base + 4);
+  S.g[3] = __shfl(S.g[3], L.base + 4);
+  S.g[4] = __shfl(S.g[4], L.base + 4);
+  S.g[5] = __shfl(S.g[5], L.base + 4);
+  return steps;
+}
+
+ABC_DEV int64_t moment_solve_team(const Particle& P, const MomCfgDev& cfg, double texp,
+                                  double pulse, double tmin, double tmax, TeamState& S,
+                                  const TeamLane& L, const LogEntry* ltab) {
+  return moment_pieces(P, cfg, texp, pulse, tmin, tmax, [&](const Piece& pc, double a, double b) {
+    return egb_piece_team(pc, P, cfg, a, b, S, L, ltab);
+  });
+}
+
+// the nine moments on every lane of the team
+ABC_DEV void team_gather(const TeamState& S, const TeamLane& L, double* y) {
+  y[0] = S.g[0];
+  y[1] = __shfl(S.m, L.base);
+  y[2] = __shfl(S.m, L.base + 1);
+  y[3] = S.g[3];
+  y[4] = S.g[4];
+  y[5] = S.g[5];
+  y[6] = __shfl(S.v, L.base);
+  y[7] = __shfl(S.v, L.base + 2);
+  y[8] = __shfl(S.v, L.base + 1);
+}
+
+ABC_DEV void team_scatter(const double* y, const TeamLane& L, TeamState& S) {
+  S.g[0] = y[0];
+  S.g[3] = y[3];
+  S.g[4] = y[4];
+  S.g[5] = y[5];
+  S.m = L.r == 0 ? y[1] : (L.r == 1 ? y[2] : 0.0);
+  S.v = L.r == 0 ? y[6] : (L.r == 1 ? y[8] : (L.r == 2 ? y[7] : 0.0));
 }
 
 template <int METHOD>
@@ -488,20 +707,46 @@ ABC_DEV Particle particle_of(int model, const MomCfgDev& cfg, const double* thet
 // Column c of particle p (c = 0 the zero state, c = 1 + i unit vector i) goes
 // to maps[(p * 10 + c) * 9 + r]; the transient rules below need nothing else,
 // so a particle's longest chain is one cycle whatever its iterations.
-// Wave w integrates column w % 10 for the 64 particles order[64 (w / 10) ..]
-// (an order by predicted cost) and adds each integration's steps to cost[p].
+// A wave integrates one column for 64 consecutive particles of order (by
+// predicted cost), or with teams for 8 of its first `heavy` particles, and adds
+// each integration's steps to cost[p].
 template <int METHOD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void moment_cyclemap_kernel(
     const MomCfgDev cfg, int model, int64_t n, const double* __restrict__ theta, int64_t ld,
-    const int32_t* __restrict__ order, double* __restrict__ maps,
+    const int32_t* __restrict__ order, int64_t heavy, double* __restrict__ maps,
     unsigned long long* __restrict__ cost, unsigned long long* __restrict__ steps) {
   __shared__ LogEntry ltab[ABC_LOG_N];
+  __shared__ double tf[METHOD == 1 ? kTeams : 1][5][5];
   load_log_table(ltab);
   __syncthreads();
-  const int64_t w = blockIdx.x;  // 64 lanes per workgroup
+  int64_t w = blockIdx.x;  // one wave per workgroup
+  const int64_t wt = heavy / kTeams * 10;
+  if (METHOD == 1 && w < wt) {  // teams of the first `heavy` particles
+    const int64_t g = w / 10;
+    const int col = (int)(w - g * 10);
+    const int team = threadIdx.x / kTeam;
+    const TeamLane L{(int)threadIdx.x % kTeam, team * kTeam, tf[team]};
+    const int64_t i = g * kTeams + team;
+    if (i >= n) return;
+    const int64_t p = order[i];
+    const Particle P = particle_of(model, cfg, theta, ld, p);
+    double y[9];
+    for (int k = 0; k < 9; ++k) y[k] = (col > 0 && k == col - 1) ? 1.0 : 0.0;
+    TeamState S{};
+    team_scatter(y, L, S);
+    const int64_t st = moment_solve_team(P, cfg, -1.0, 0.1, 0.0, cfg.cycle, S, L, ltab);
+    team_gather(S, L, y);
+    if (L.r != 0) return;
+    double* o = maps + (p * 10 + col) * 9;
+    for (int k = 0; k < 9; ++k) o[k] = y[k];
+    atomicAdd(cost + p, (unsigned long long)st);
+    if (steps) atomicAdd(steps + p, (unsigned long long)st);
+    return;
+  }
+  w -= wt;
   const int64_t g = w / 10;
   const int col = (int)(w - g * 10);
-  const int64_t i = g * 64 + threadIdx.x;
+  const int64_t i = heavy + g * 64 + threadIdx.x;
   if (i >= n) return;
   const int64_t p = order[i];
   const Particle P = particle_of(model, cfg, theta, ld, p);
@@ -669,9 +914,9 @@ __global__ __launch_bounds__(64) void moment_transient_kernel(const MomCfgDev cf
 
 // trajectories (model.jl:146-174) for item (particle, condition, age): out
 // column (cond * n_ages + age) * 5 + {mean_u, mean_l, var_u, cov_ul, var_l}.
-// Wave w takes one (condition, age) item for the 64 particles
-// order[64 g .. 64 g + 63], g = w / items, so its lanes share the item's
-// cycle structure and have similar step counts.
+// A wave takes one (condition, age) item for 64 consecutive particles of order
+// (with teams: 8 of its first `heavy`), so its lanes share the item's cycle
+// structure and have similar step counts.
 // A whole cycle that starts on a cycle boundary and does not meet the
 // labelling window has the rates of [0, T] shifted by whole cycles and no
 // labelling, so it is the particle's affine cycle map, applied from maps.
@@ -683,16 +928,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void mo
                                                           const double* __restrict__ ss,
                                                           const double* __restrict__ maps,
                                                           const int32_t* __restrict__ order,
+                                                          int64_t heavy,
                                                           double* __restrict__ out,
                                                           unsigned long long* __restrict__ steps) {
   __shared__ LogEntry ltab[ABC_LOG_N];
+  __shared__ double tf[METHOD == 1 ? kTeams : 1][5][5];
   load_log_table(ltab);
   __syncthreads();
   const int per = cfg.n_conds * cfg.n_ages;
-  const int64_t w = blockIdx.x;  // 64 lanes per workgroup
+  int64_t w = blockIdx.x;  // one wave per workgroup
+  const int64_t wt = heavy / kTeams * per;
+  const bool by_team = METHOD == 1 && w < wt;  // teams of the first `heavy` particles
+  if (!by_team) w -= wt;
   const int64_t g = w / per;
   const int r = (int)(w - g * per);
-  const int64_t i = g * 64 + threadIdx.x;
+  const int team = threadIdx.x / kTeam;
+  const int64_t i = by_team ? g * kTeams + team : heavy + g * 64 + threadIdx.x;
   if (i >= n) return;
   const int64_t p = order[i];
   const int j = r / cfg.n_ages, ai = r - j * cfg.n_ages;
@@ -702,6 +953,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void mo
   const int nsols = (age > 0 && age < T) ? (int)floor((age - t0) / T) + 1 : (int)floor((age - t0) / T);
   const double we = texp + pulse;
   const double* mp = maps + p * 90;
+  const TeamLane L{(int)threadIdx.x % kTeam, team * kTeam, tf[by_team ? team : 0]};
+  TeamState S{};
   double y[9], tmp[9];
   for (int i = 0; i < 9; ++i) y[i] = ss[p + (int64_t)i * n];
   double tau = t0;
@@ -721,11 +974,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void mo
         tmp[r] = acc;
       }
       for (int i = 0; i < 9; ++i) y[i] = tmp[i];
+    } else if (by_team) {  // y is the same on every lane of the team
+      team_scatter(y, L, S);
+      st += moment_solve_team(P, cfg, texp, pulse, tau, tf, S, L, ltab);
+      team_gather(S, L, y);
     } else {
       st += moment_solve<METHOD>(P, cfg, texp, pulse, tau, tf, y, ltab);
     }
     tau = tf;
   }
+  if (by_team && L.r != 0) return;
   double* o = out + p + (int64_t)r * 5 * n;
   o[0] = y[1];
   o[n] = y[2];
@@ -809,14 +1067,14 @@ __global__ __launch_bounds__(64) void moment_stats_kernel(const MomCfgDev cfg,
 // one instantiation per integration method (cfg.method), so that each has its
 // own register allocation
 template __global__ void moment_cyclemap_kernel<0>(MomCfgDev, int, int64_t, const double*, int64_t,
-                                                   const int32_t*, double*, unsigned long long*,
-                                                   unsigned long long*);
+                                                   const int32_t*, int64_t, double*,
+                                                   unsigned long long*, unsigned long long*);
 template __global__ void moment_cyclemap_kernel<1>(MomCfgDev, int, int64_t, const double*, int64_t,
-                                                   const int32_t*, double*, unsigned long long*,
-                                                   unsigned long long*);
+                                                   const int32_t*, int64_t, double*,
+                                                   unsigned long long*, unsigned long long*);
 template __global__ void moment_traj_kernel<0>(MomCfgDev, int, int64_t, const double*, int64_t,
                                                const double*, const double*, const int32_t*,
-                                               double*, unsigned long long*);
+                                               int64_t, double*, unsigned long long*);
 template __global__ void moment_traj_kernel<1>(MomCfgDev, int, int64_t, const double*, int64_t,
                                                const double*, const double*, const int32_t*,
-                                               double*, unsigned long long*);
+                                               int64_t, double*, unsigned long long*);
