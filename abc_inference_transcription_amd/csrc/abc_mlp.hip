@@ -33,7 +33,24 @@ enum { EPI_F32 = 0, EPI_SILU = 1, EPI_DSILU = 2 };
 // (+8 bf16 of padding against bank conflicts)
 constexpr int BK = 64, LDSK = BK + 8;
 
-__device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + __expf(-z)); }
+// s = 1 / (1 + e^-z) of four values.  The reciprocals of x = 1 + e^-z >= 1 are
+// correctly rounded without the division sequence: the hardware's reciprocal
+// and one Newton step give the division's bits for every x in [1, 2^126)
+// (compared for all of them on gfx950); beyond, where the reciprocal is
+// subnormal or x infinite, all four divide.
+__device__ __forceinline__ void sigm4(const float* z, float* s) {
+  float x[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    x[q] = 1.0f + __expf(-z[q]);
+    const float r = __builtin_amdgcn_rcpf(x[q]);
+    s[q] = fmaf(fmaf(-x[q], r, 1.0f), r, r);
+  }
+  if (fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])) >= 0x1p126f) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) s[q] = 1.0f / x[q];
+  }
+}
 
 // 256 threads, workgroup tile BM x BN (BM 128 or 64), wave tile BM/2 x BN/2
 // (2 x 2 waves).  blockIdx.z selects a K chunk [z*K, (z+1)*K) of rows with
@@ -129,6 +146,13 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
       const int mb = m0 + wm * WM + r4 * 16 + (lane >> 4) * 4;
       const int n = n0 + wn * WN + cb * 16 + (lane & 15);
       bf16x4 tv;
+      float z[4], s[4];
+      if (EPI != EPI_F32) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          z[q] = EPI == EPI_SILU ? acc[r4][cb][q] + bias[n] : Zprev[(size_t)(mb + q) * N + n];
+        sigm4(z, s);
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int m = mb + q;
@@ -138,15 +162,12 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
           if (bias) v += bias[n];
           Cf[o] = v;
         } else if (EPI == EPI_SILU) {
-          const float z = v + bias[n];
-          Zout[o] = z;
-          const bf16 h = (bf16)(z * sigm(z));
+          Zout[o] = z[q];
+          const bf16 h = (bf16)(z[q] * s[q]);
           Cb[o] = h;
           tv[q] = h;
         } else {
-          const float z = Zprev[o];
-          const float s = sigm(z);
-          const bf16 d = (bf16)(v * (s * (1.0f + z * (1.0f - s))));
+          const bf16 d = (bf16)(v * (s[q] * (1.0f + z[q] * (1.0f - s[q]))));
           Cb[o] = d;
           tv[q] = d;
         }
@@ -270,48 +291,130 @@ struct LayerDesc {
   int64_t b_off;    // offset of b (out)
 };
 
-// Adam on the flat FP32 parameters; refreshes the bf16 copies W (out x in)
-// and W^T (in x out) of every weight.
-__global__ void adam_kernel(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                            const float* __restrict__ g, int64_t n, float lr, float b1, float b2,
-                            float eps, float wd, float c1, float c2, const LayerDesc* __restrict__ L,
-                            int nl, const int64_t* __restrict__ bf_off, bf16* __restrict__ Wb,
-                            bf16* __restrict__ WbT) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  float gg = g[p];
-  const float mm = b1 * m[p] + (1.0f - b1) * gg;
-  const float vv = b2 * v[p] + (1.0f - b2) * gg * gg;
-  m[p] = mm;
-  v[p] = vv;
-  float ww = w[p];
-  ww -= lr * ((mm / c1) / (sqrtf(vv / c2) + eps) + wd * ww);
-  w[p] = ww;
+// place of weight (o, i) of an out x in layer in the fragment-ordered copy: the
+// 16 x 32 MFMA operand tiles (o / 16, i / 32), each as its 64 lanes' 16 bytes
+__device__ __forceinline__ int64_t frag_at(int o, int i, int in) {
+  return ((int64_t)(o >> 4) * in + (i & ~31)) * 16 + ((o & 15) + ((i >> 3) & 3) * 16) * 8 + (i & 7);
+}
+
+// One workgroup per 64 x 64 tile of a layer's weights (dims.x of them in all, in
+// layer order), then one per 256 biases: tile and layer of workgroup `blk`.
+struct TilePos {
+  int layer, o0, i0;  // layer < 0: biases, o0 the first of the 256 (over all layers)
+};
+__device__ __forceinline__ TilePos tile_pos(int blk, const LayerDesc* __restrict__ L, int nl) {
   for (int l = 0; l < nl; ++l) {
-    const int64_t sz = (int64_t)L[l].in * L[l].out;
-    if (p >= L[l].w_off && p < L[l].w_off + sz) {
-      const int64_t e = p - L[l].w_off;
-      const int o = (int)(e / L[l].in), i = (int)(e % L[l].in);
-      Wb[bf_off[l] + e] = (bf16)ww;
-      WbT[bf_off[l] + (int64_t)i * L[l].out + o] = (bf16)ww;
+    const int ti = L[l].in / 64, t = L[l].out / 64 * ti;
+    if (blk < t) return TilePos{l, blk / ti * 64, blk % ti * 64};
+    blk -= t;
+  }
+  return TilePos{-1, blk * 256, 0};
+}
+
+// bias q (over all layers) as an index of the flat parameters, or -1
+__device__ __forceinline__ int64_t bias_at(int q, const LayerDesc* __restrict__ L, int nl) {
+  for (int l = 0; l < nl; ++l) {
+    if (q < L[l].out) return L[l].b_off + q;
+    q -= L[l].out;
+  }
+  return -1;
+}
+
+// the bf16 copies of a tile: v holds this thread's weights, v[j][e] that of
+// (o0 + j * 32 + tid / 8, i0 + (tid & 7) * 8 + e); W and its fragment order
+// take 16 bytes per 8 of them, W^T goes through LDS
+__device__ __forceinline__ void store_copies(const float (&v)[2][8], const TilePos& T,
+                                             const LayerDesc& L, int64_t off,
+                                             bf16* __restrict__ Wb, bf16* __restrict__ WbT,
+                                             bf16* __restrict__ Wf) {
+  __shared__ bf16 tile[64][64 + 8];  // [i][o]
+  const int ro = threadIdx.x >> 3, ri = (threadIdx.x & 7) * 8;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int o = T.o0 + j * 32 + ro, i = T.i0 + ri;
+    bf16x8 h;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      h[e] = (bf16)v[j][e];
+      tile[ri + e][j * 32 + ro] = h[e];
     }
+    *reinterpret_cast<bf16x8*>(Wb + off + (int64_t)o * L.in + i) = h;
+    *reinterpret_cast<bf16x8*>(Wf + off + frag_at(o, i, L.in)) = h;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int i = j * 32 + ro;
+    *reinterpret_cast<bf16x8*>(WbT + off + (int64_t)(T.i0 + i) * L.out + T.o0 + ri) =
+        *reinterpret_cast<const bf16x8*>(&tile[i][ri]);
   }
 }
 
-__global__ void refresh_bf16_kernel(const float* __restrict__ w, const LayerDesc* __restrict__ L,
-                                    int nl, const int64_t* __restrict__ bf_off,
-                                    bf16* __restrict__ Wb, bf16* __restrict__ WbT, int64_t n) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  for (int l = 0; l < nl; ++l) {
-    const int64_t sz = (int64_t)L[l].in * L[l].out;
-    if (p >= L[l].w_off && p < L[l].w_off + sz) {
-      const int64_t e = p - L[l].w_off;
-      const int o = (int)(e / L[l].in), i = (int)(e % L[l].in);
-      Wb[bf_off[l] + e] = (bf16)w[p];
-      WbT[bf_off[l] + (int64_t)i * L[l].out + o] = (bf16)w[p];
+// Adam on the flat FP32 parameters; refreshes the bf16 copies W (out x in), W^T
+// (in x out) and W in fragment order of every weight.  Bound by memory: 8
+// weights a thread in 16- and 32-byte pieces (a weight a thread with scattered
+// copies: 12.1 us for 0.9 million weights, 9.2 now).
+__global__ __launch_bounds__(256) void adam_kernel(
+    float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
+    const float* __restrict__ g, float lr, float b1, float b2, float eps, float wd, float c1,
+    float c2, const LayerDesc* __restrict__ L, int nl, const int64_t* __restrict__ bf_off,
+    bf16* __restrict__ Wb, bf16* __restrict__ WbT, bf16* __restrict__ Wf) {
+  auto step = [&](float gg, float& mp, float& vp, float ww) {
+    const float mm = b1 * mp + (1.0f - b1) * gg;
+    const float vv = b2 * vp + (1.0f - b2) * gg * gg;
+    mp = mm;
+    vp = vv;
+    return ww - lr * ((mm / c1) / (sqrtf(vv / c2) + eps) + wd * ww);
+  };
+  const TilePos T = tile_pos((int)blockIdx.x, L, nl);
+  if (T.layer < 0) {
+    const int64_t p = bias_at(T.o0 + (int)threadIdx.x, L, nl);
+    if (p >= 0) w[p] = step(g[p], m[p], v[p], w[p]);
+    return;
+  }
+  const LayerDesc D = L[T.layer];
+  float x[2][8];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int o = T.o0 + j * 32 + (threadIdx.x >> 3), i = T.i0 + (threadIdx.x & 7) * 8;
+    const int64_t p = D.w_off + (int64_t)o * D.in + i;
+#pragma unroll
+    for (int h = 0; h < 8; h += 4) {
+      f32x4 gm = *reinterpret_cast<const f32x4*>(g + p + h);
+      f32x4 mm = *reinterpret_cast<const f32x4*>(m + p + h);
+      f32x4 vv = *reinterpret_cast<const f32x4*>(v + p + h);
+      f32x4 ww = *reinterpret_cast<const f32x4*>(w + p + h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float a = mm[e], b = vv[e];
+        ww[e] = x[j][h + e] = step(gm[e], a, b, ww[e]);
+        mm[e] = a;
+        vv[e] = b;
+      }
+      *reinterpret_cast<f32x4*>(m + p + h) = mm;
+      *reinterpret_cast<f32x4*>(v + p + h) = vv;
+      *reinterpret_cast<f32x4*>(w + p + h) = ww;
     }
   }
+  store_copies(x, T, D, bf_off[T.layer], Wb, WbT, Wf);
+}
+
+// the bf16 copies of every weight (launch: the weight tiles)
+__global__ __launch_bounds__(256) void refresh_bf16_kernel(
+    const float* __restrict__ w, const LayerDesc* __restrict__ L, int nl,
+    const int64_t* __restrict__ bf_off, bf16* __restrict__ Wb, bf16* __restrict__ WbT,
+    bf16* __restrict__ Wf) {
+  const TilePos T = tile_pos((int)blockIdx.x, L, nl);
+  if (T.layer < 0) return;
+  const LayerDesc D = L[T.layer];
+  float x[2][8];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      x[j][e] = w[D.w_off + (int64_t)(T.o0 + j * 32 + (threadIdx.x >> 3)) * D.in + T.i0 +
+                  (threadIdx.x & 7) * 8 + e];
+  store_copies(x, T, D, bf_off[T.layer], Wb, WbT, Wf);
 }
 
 __global__ void zero_f32_kernel(float* __restrict__ p, int64_t n) {
@@ -326,6 +429,131 @@ __global__ void gather_out_kernel(const float* __restrict__ O, int Bn, int ns, i
   if (q >= (int64_t)Bn * 2 * ns) return;
   const int b = (int)(q / (2 * ns)), k = (int)(q % (2 * ns));
   y[q] = O[(size_t)b * out_pad + k];
+}
+
+// The whole network on 16 RT rows per workgroup of eight waves, for inference:
+// the activations stay in LDS from the features to the outputs and the weights
+// come from the L2 once per workgroup, so a call is one launch and writes
+// nothing but its outputs (layer by layer it wrote, per row and unit, the
+// training step's pre-activation and two copies of the activation).  Wave w
+// makes features [w, w + 1) * width / 8 of a layer: W fragments are the MFMA's
+// rows and activations its columns, so a lane ends up with four consecutive
+// features of one row, one 8-byte LDS store.  A layer's outputs are all in
+// registers before the first replaces an input.  Every output sums its K in the
+// order of gemm_nt_kernel, 32 at a time: the same bits.
+// Bound by the L2 reads of the weights (1.7 MB a workgroup at width 512) and
+// the activations' exponentials and reciprocals.  40,000 rows, 23 -> 4 x 512 ->
+// 180: 395 -> 128 us, 77 rows 57 -> 38 us.
+constexpr int kInferPad = 8;  // bf16 of padding per LDS row
+template <int RT, int FT>
+__global__ __launch_bounds__(512) void infer_kernel(const float* __restrict__ x, int64_t n, int n_in,
+                                                    const LayerDesc* __restrict__ layers, int depth,
+                                                    const int64_t* __restrict__ bf_off,
+                                                    const bf16* __restrict__ Wf,
+                                                    const float* __restrict__ w, int n_out,
+                                                    int vec4, float* __restrict__ y) {
+  extern __shared__ bf16 act[];
+  constexpr int W = 128 * FT, D = 2;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t r0 = (int64_t)blockIdx.x * (16 * RT);
+  const int in_pad = layers[0].in;
+  const int S = (in_pad > W ? in_pad : W) + kInferPad;
+  for (int q = threadIdx.x; q < 16 * RT * in_pad; q += 512) {
+    const int r = q / in_pad, k = q - r * in_pad;
+    act[r * S + k] = (bf16)(r0 + r < n && k < n_in ? x[(r0 + r) * n_in + k] : 0.0f);
+  }
+  __syncthreads();
+  const int li = lane & 15, kq = (lane >> 4) * 8;
+  // acc[t][r]: features f0 + 16 t .. of a layer with K inputs, rows 16 r ..
+  auto product = [&](const bf16* Wl, int K, int f0, auto& acc) {
+    constexpr int T = sizeof(acc) / sizeof(acc[0]);
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16* wp = Wl + (size_t)(f0 / 16) * K * 16 + lane * 8;  // tile t, step k: + (t K + k) * 16
+    // weights D steps of 32 ahead: an L2 read takes longer than a step's MFMAs
+    bf16x8 a[D][T];
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        if (32 * d < K)
+          a[d][t] = *reinterpret_cast<const bf16x8*>(wp + (size_t)(t * K + 32 * d) * 16);
+    for (int k0 = 0; k0 < K; k0 += 32 * D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int k = k0 + 32 * d;
+        if (k >= K) break;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const bf16x8 b = *reinterpret_cast<const bf16x8*>(act + (16 * r + li) * S + k + kq);
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+            acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b, acc[t][r], 0, 0, 0);
+        }
+        const int kn = k + 32 * D;
+        if (kn < K)
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+            a[d][t] = *reinterpret_cast<const bf16x8*>(wp + (size_t)(t * K + kn) * 16);
+      }
+    }
+  };
+  for (int l = 0; l < depth; ++l) {
+    const LayerDesc L = layers[l];
+    const int f0 = wave * (16 * FT);
+    f32x4 acc[FT][RT];
+    product(Wf + bf_off[l], L.in, f0, acc);
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < FT; ++t) {
+      const int f = f0 + 16 * t + (lane >> 4) * 4;
+      float bias[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bias[q] = w[L.b_off + f + q];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        bf16x4 h;
+        float z[4], s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) z[q] = acc[t][r][q] + bias[q];
+        sigm4(z, s);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[q] = (bf16)(z[q] * s[q]);
+        *reinterpret_cast<bf16x4*>(act + (16 * r + li) * S + f) = h;
+      }
+    }
+    __syncthreads();
+  }
+  // the output layer, 32 features per wave at a time (its padding ends on one)
+  const LayerDesc L = layers[depth];
+  for (int f0 = wave * 32; f0 < n_out; f0 += 256) {
+    f32x4 acc[2][RT];
+    product(Wf + bf_off[depth], L.in, f0, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int f = f0 + 16 * t + (lane >> 4) * 4;
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const int64_t row = r0 + 16 * r + li;
+        if (row >= n) continue;
+        if (vec4 && f < n_out) {
+          float4 v;
+          v.x = acc[t][r][0] + w[L.b_off + f];
+          v.y = acc[t][r][1] + w[L.b_off + f + 1];
+          v.z = acc[t][r][2] + w[L.b_off + f + 2];
+          v.w = acc[t][r][3] + w[L.b_off + f + 3];
+          *reinterpret_cast<float4*>(y + row * n_out + f) = v;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (f + q < n_out) y[row * n_out + f + q] = acc[t][r][q] + w[L.b_off + f + q];
+        }
+      }
+    }
+  }
 }
 
 int g1(int64_t n, int b) { return (int)((n + b - 1) / b); }
@@ -506,12 +734,13 @@ struct abc_mlp {
   int tile_rows = 0;  // GEMM workgroup rows: 0 = by shape, else 64 or 128
   int tile_cols = 0;  // GEMM workgroup columns: 0 = by shape, else 64 or 128
   int64_t n_par = 0, n_bf = 0;
+  int w_tiles = 0, n_bias = 0;  // 64 x 64 weight tiles and biases over all layers
   std::vector<LayerDesc> layers;
   std::vector<int64_t> bf_off;
   LayerDesc* d_layers = nullptr;
   int64_t* d_bf_off = nullptr;
   float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
-  bf16 *Wb = nullptr, *WbT = nullptr;
+  bf16 *Wb = nullptr, *WbT = nullptr, *Wf = nullptr;  // Wf: fragment order
   // activations (max_batch rows, padded to 128)
   bf16 *X = nullptr, *XT = nullptr;
   std::vector<float*> Z;
@@ -610,6 +839,45 @@ int forward(abc_mlp* p, int64_t Bn, const float* x_dev) {
   return ABC_OK;
 }
 
+// One launch for all n rows where a layer's outputs fit a workgroup's registers
+// and LDS (width up to 512); false: not launched.  Rows per workgroup: 16 while
+// those give at most one workgroup per CU, 32 up to two, 64 above, two of which
+// share a CU and overlap one's MFMAs with the other's activations (with 128, one
+// a CU, they do not).  16 / 32 / 64 / 128 rows, us: n = 77 39 / 43 / 60 / 86, 8,192
+// 60 / 51 / 65 / 96, 16,384 97 / 70 / 69 / 101, 40,000 212 / 143 / 131 / 186.
+template <int RT, int FT>
+bool infer_launch(abc_mlp* p, int64_t n, const float* x, float* y) {
+  const size_t lds = (size_t)16 * RT * ((size_t)std::max(p->in_pad, 128 * FT) + kInferPad) * 2;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(infer_kernel<RT, FT>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  hipLaunchKernelGGL((infer_kernel<RT, FT>), dim3((unsigned)((n + 16 * RT - 1) / (16 * RT))),
+                     dim3(512), lds, p->stream, x, n, p->n_in, p->d_layers, p->depth, p->d_bf_off,
+                     p->Wf, p->w, p->n_out,
+                     (int)(p->n_out % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0), y);
+  return true;
+}
+
+template <int FT>
+bool infer_width(abc_mlp* p, int64_t n, const float* x, float* y) {
+  if (n <= 4096) return infer_launch<1, FT>(p, n, x, y);
+  if (n <= 16384) return infer_launch<2, FT>(p, n, x, y);
+  return infer_launch<4, FT>(p, n, x, y);
+}
+
+bool infer(abc_mlp* p, int64_t n, const float* x, float* y) {
+  if (n > (int64_t)1 << 30) return false;
+  switch (p->width) {
+    case 128: return infer_width<1>(p, n, x, y);
+    case 256: return infer_width<2>(p, n, x, y);
+    case 384: return infer_width<3>(p, n, x, y);
+    case 512: return infer_width<4>(p, n, x, y);
+    default: return false;
+  }
+}
+
 // fwd + loss + bwd into p->g; loss (mean NLL) accumulated in p->loss
 int grad(abc_mlp* p, int64_t Bn, const float* x_dev, const float* t_dev) {
   int rc = forward(p, Bn, x_dev);
@@ -694,7 +962,7 @@ int32_t abc_mlp_create(abc_mlp** out, int32_t device, int32_t n_in, int32_t widt
     if (ok && hipMalloc((void**)ptr, bytes) != hipSuccess) ok = false;
   };
   A(&p->w, 4 * off); A(&p->m, 4 * off); A(&p->v, 4 * off); A(&p->g, 4 * off);
-  A(&p->Wb, 2 * boff); A(&p->WbT, 2 * boff);
+  A(&p->Wb, 2 * boff); A(&p->WbT, 2 * boff); A(&p->Wf, 2 * boff);
   A(&p->d_layers, sizeof(LayerDesc) * p->layers.size());
   A(&p->d_bf_off, sizeof(int64_t) * p->bf_off.size());
   A(&p->X, 2 * Bp * p->in_pad); A(&p->XT, 2 * Bp * p->in_pad);
@@ -720,8 +988,12 @@ int32_t abc_mlp_create(abc_mlp** out, int32_t device, int32_t n_in, int32_t widt
     abc_mlp_destroy(p);
     return ABC_E_HIP;
   }
-  hipLaunchKernelGGL(refresh_bf16_kernel, dim3(g1(off, 256)), dim3(256), 0, p->stream, p->w,
-                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, off);
+  for (const LayerDesc& L : p->layers) {
+    p->w_tiles += (L.in / 64) * (L.out / 64);
+    p->n_bias += L.out;
+  }
+  hipLaunchKernelGGL(refresh_bf16_kernel, dim3(p->w_tiles), dim3(256), 0, p->stream, p->w,
+                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf);
   if (hipStreamSynchronize(p->stream) != hipSuccess) { abc_mlp_destroy(p); return ABC_E_HIP; }
   *out = p;
   return ABC_OK;
@@ -730,7 +1002,7 @@ int32_t abc_mlp_create(abc_mlp** out, int32_t device, int32_t n_in, int32_t widt
 int32_t abc_mlp_destroy(abc_mlp* p) {
   if (!p) return ABC_OK;
   if (p->stream) hipStreamSynchronize(p->stream);
-  void* bufs[] = {p->w, p->m, p->v, p->g, p->Wb, p->WbT, p->d_layers, p->d_bf_off, p->X, p->XT,
+  void* bufs[] = {p->w, p->m, p->v, p->g, p->Wb, p->WbT, p->Wf, p->d_layers, p->d_bf_off, p->X, p->XT,
                   p->O, p->dA, p->dAT, p->dB, p->dBT, p->loss, p->splitk_ws};
   for (void* b : bufs)
     if (b) hipFree(b);
@@ -789,14 +1061,18 @@ int32_t abc_mlp_set_params(abc_mlp* p, const float* host) {
   if (!p || !host) return ABC_E_ARG;
   MCHK(p, hipStreamSynchronize(p->stream));
   MCHK(p, hipMemcpy(p->w, host, 4 * p->n_par, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(refresh_bf16_kernel, dim3(g1(p->n_par, 256)), dim3(256), 0, p->stream, p->w,
-                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->n_par);
+  hipLaunchKernelGGL(refresh_bf16_kernel, dim3(p->w_tiles), dim3(256), 0, p->stream, p->w,
+                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf);
   MCHK(p, hipStreamSynchronize(p->stream));
   return ABC_OK;
 }
 
 int32_t abc_mlp_forward_dev(abc_mlp* p, int64_t n, const float* x_dev, float* y_dev) {
   if (!p || n < 0 || (n > 0 && (!x_dev || !y_dev))) return ABC_E_ARG;
+  if (n > 0 && infer(p, n, x_dev, y_dev)) {
+    MCHK(p, hipGetLastError());
+    return ABC_OK;
+  }
   for (int64_t o = 0; o < n; o += p->max_batch) {
     const int64_t b = std::min<int64_t>(p->max_batch, n - o);
     int rc = forward(p, b, x_dev + o * p->n_in);
@@ -828,9 +1104,9 @@ int32_t abc_mlp_train_step_dev(abc_mlp* p, int64_t n, const float* x_dev, const 
   p->step++;
   const float c1 = 1.0f - std::pow(beta1, (float)p->step);
   const float c2 = 1.0f - std::pow(beta2, (float)p->step);
-  hipLaunchKernelGGL(adam_kernel, dim3(g1(p->n_par, 256)), dim3(256), 0, p->stream, p->w, p->m,
-                     p->v, p->g, p->n_par, lr, beta1, beta2, eps, weight_decay, c1, c2,
-                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT);
+  hipLaunchKernelGGL(adam_kernel, dim3(p->w_tiles + g1(p->n_bias, 256)), dim3(256), 0, p->stream,
+                     p->w, p->m, p->v, p->g, lr, beta1, beta2, eps, weight_decay, c1, c2,
+                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf);
   if (loss_dev_or_null)
     MCHK(p, hipMemcpyAsync(loss_dev_or_null, p->loss, 4, hipMemcpyDeviceToDevice, p->stream));
   MCHK(p, hipGetLastError());
