@@ -1896,9 +1896,11 @@ int data_meta(abc_ctx* c, int64_t G, int64_t n, int32_t nc, const int32_t* age, 
   return ABC_OK;
 }
 
-// the kernel over every gene, in launches whose resample scratch stays near 1 GiB
+// the kernel over every gene, in launches whose resample scratch stays near 1 GiB;
+// check: a count of 2^20 or more is an error in any cell, not only in those summed
 int data_run(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t* l, int32_t nc,
-             int32_t J, int64_t np, int64_t nch, int32_t n_boot, uint64_t seed, double* out) {
+             int32_t J, int64_t np, int64_t nch, int32_t n_boot, uint64_t seed, double* out,
+             bool check) {
   int rc;
   const int64_t K1 = 4 * nc + 3 * J;
   // families of at most ABC_DATA_SORTED_MAX cells: each gene's cells packed in
@@ -1920,10 +1922,15 @@ int data_run(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t
   if ((rc = ensure(c, c->dboot, (size_t)(chunk * n_boot * K1) * sizeof(double)))) return rc;
   if ((rc = ensure(c, c->dpt, sizeof(double) * (size_t)(chunk * K1)))) return rc;
   if ((rc = ensure(c, c->dflag, sizeof(unsigned long long)))) return rc;
-  if (sorted && slots > 0 && (rc = ensure(c, c->dxs, sizeof(unsigned long long) * (size_t)(chunk * slots))))
-    return rc;
+  // the packed cells and, after them, the largest u + l of each 64
+  if (sorted && (rc = ensure(c, c->dxs, (size_t)chunk * (size_t)(slots * 8 + slots / 16)))) return rc;
+  uint32_t* xmax = reinterpret_cast<uint32_t*>(P<unsigned long long>(c->dxs) + chunk * slots);
   unsigned long long* flag = P<unsigned long long>(c->dflag);
   hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream, flag, (int64_t)1);
+  if (check && n > 0)
+    hipLaunchKernelGGL(data_check_kernel,
+                       dim3((unsigned)std::min<int64_t>((G * n + 255) / 256, 2048)), dim3(256), 0,
+                       c->stream, G * n, u, l, reinterpret_cast<unsigned int*>(flag));
   const int32_t* m = P<int32_t>(c->dmeta);
   const int32_t* perm = P<int32_t>(c->dsort);
   for (int64_t g0 = 0; g0 < G; g0 += chunk) {
@@ -1934,19 +1941,23 @@ int data_run(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t
                            dim3((unsigned)((cnt * (slots / ABC_DATA_WG) + 7) / 8 * 8)),
                            dim3(ABC_DATA_WG), 0, c->stream, n, u, l, g0, m + 2 * n, np,
                            m + 2 * n + np, nch, perm, perm + total, slots, cnt,
-                           P<unsigned long long>(c->dxs), reinterpret_cast<unsigned int*>(flag));
+                           P<unsigned long long>(c->dxs), xmax,
+                           reinterpret_cast<unsigned int*>(flag));
       HIPCHK(c, hipGetLastError());
       const int spb = ABC_DATA_SETS_PER_WG;
       const int nsb = (n_boot + 1 + spb - 1) / spb;
       const int64_t items = cnt * nsb;
-      hipLaunchKernelGGL(data_stats_sorted_kernel, dim3((unsigned)((items + 7) / 8 * 8)),
-                         dim3(ABC_DATA_WG),
-                         (size_t)((mmax + 1) / 2 > 0 ? (mmax + 1) / 2 : 1) * sizeof(uint32_t),
-                         c->stream, cnt, nsb, g0, P<unsigned long long>(c->dxs), slots, n, np, nch,
-                         nc, J, P<double>(c->dw), n_boot, spb, (uint32_t)seed,
-                         (uint32_t)(seed >> 32) ^ 0x2545F491u, P<double>(c->dpt),
-                         P<double>(c->dboot));
-      HIPCHK(c, hipGetLastError());
+      const size_t lds = data_sorted_lds(mmax);
+      // every gene is one instantiation's: by its counts, which only the device knows
+      for (int small = 1; small >= 0; --small) {
+        hipLaunchKernelGGL(small ? data_stats_sorted_kernel<true> : data_stats_sorted_kernel<false>,
+                           dim3((unsigned)((items + 7) / 8 * 8)), dim3(ABC_DATA_WG), lds, c->stream,
+                           cnt, nsb, g0, P<unsigned long long>(c->dxs), slots, xmax, n, np, nch, nc,
+                           J, P<double>(c->dw), n_boot, spb, (uint32_t)seed,
+                           (uint32_t)(seed >> 32) ^ 0x2545F491u, P<double>(c->dpt),
+                           P<double>(c->dboot));
+        HIPCHK(c, hipGetLastError());
+      }
       hipLaunchKernelGGL(data_se_kernel, dim3(grid1(cnt * K1, 256)), dim3(256), 0, c->stream, G,
                          g0, cnt, nc, J, n_boot, P<double>(c->dpt), P<double>(c->dboot), out);
     } else
@@ -1981,7 +1992,7 @@ int32_t abc_data_stats_dev(abc_ctx* c, int64_t n_genes, int64_t n_cells, const u
   if ((n_cells > 0 && (!u_dev || !l_dev)) || !out_dev)
     return fail(c, ABC_E_ARG, "u, l and out are required");
   return data_run(c, n_genes, n_cells, u_dev, l_dev, n_clusters, n_conds, n_pulse, n_chase, n_boot,
-                  seed, out_dev);
+                  seed, out_dev, false);
 }
 
 int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint32_t* u,
@@ -1997,8 +2008,6 @@ int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint3
   if (n_genes == 0) return ABC_OK;
   if ((n_cells > 0 && (!u || !l)) || !out) return fail(c, ABC_E_ARG, "u, l and out are required");
   const size_t nu = (size_t)n_genes * (size_t)n_cells;
-  for (size_t i = 0; i < nu; ++i)
-    if ((u[i] | l[i]) >= (1u << 20)) return fail(c, ABC_E_ARG, "counts must be below 2^20");
   const size_t K = (size_t)(8 * n_clusters + 6 * n_conds);
   if ((rc = ensure(c, c->du, sizeof(uint32_t) * (nu > 0 ? nu : 1)))) return rc;
   if ((rc = ensure(c, c->dl, sizeof(uint32_t) * (nu > 0 ? nu : 1)))) return rc;
@@ -2008,7 +2017,7 @@ int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint3
     HIPCHK(c, hipMemcpyAsync(c->dl.p, l, sizeof(uint32_t) * nu, hipMemcpyHostToDevice, c->stream));
   }
   rc = data_run(c, n_genes, n_cells, P<uint32_t>(c->du), P<uint32_t>(c->dl), n_clusters, n_conds,
-                n_pulse, n_chase, n_boot, seed, P<double>(c->dout));
+                n_pulse, n_chase, n_boot, seed, P<double>(c->dout), true);
   if (rc) return rc;
   HIPCHK(c, hipMemcpyAsync(out, c->dout.p, sizeof(double) * (size_t)n_genes * K,
                            hipMemcpyDeviceToHost, c->stream));

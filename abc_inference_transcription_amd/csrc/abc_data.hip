@@ -32,6 +32,8 @@
 // data_stats_sorted_kernel, which counts the draws per cell first and spreads
 // a gene's sets over several workgroups, and data_se_kernel; both paths give
 // the same integers and so the same bits.
+#include <type_traits>
+
 #include "abc_device.h"
 #include "abc_kernels.h"
 
@@ -43,14 +45,6 @@ namespace {
 ABC_DEV int64_t pos_of(const u4& w, int h, int64_t m) {
   const uint64_t u = h == 0 ? ((uint64_t)w.y << 32 | w.x) : ((uint64_t)w.w << 32 | w.z);
   return (int64_t)__umul64hi(u, (uint64_t)m);
-}
-
-// the same for m < 2^32: with u = hi 2^32 + lo, floor(u m / 2^64) =
-// floor((hi m + floor(lo m / 2^32)) / 2^32), since the low word of lo m
-// cannot carry the sum past a multiple of 2^64
-ABC_DEV uint32_t pos_of32(const u4& w, int h, uint32_t m) {
-  const uint32_t lo = h == 0 ? w.x : w.z, hi = h == 0 ? w.y : w.w;
-  return (uint32_t)(((uint64_t)hi * m + __umulhi(lo, m)) >> 32);
 }
 
 // (n Sxy - Sx Sy) / (n (n - 1)) from exact 128-bit products
@@ -288,14 +282,17 @@ __global__ __launch_bounds__(ABC_DATA_WG) void data_stats_kernel(
 }
 
 // Each family's cells of one gene as one 64-bit word per cell: bits 0-19 u,
-// 20-39 l, 40-55 the cell's position in the family (its draw counter), 56-63
-// its group + 1 (0: a cell in no group, or padding).  Per gene the families
-// follow one another (pulse, chase, all cells by condition, all cells by
-// (condition, cluster)), each in ceil(m / 256) * 256 slots, transposed: slot
-// j * 256 + t holds sorted position t * ceil(m / 256) + j, so that lane t of
-// data_stats_sorted_kernel walks a contiguous run of the sorted cells while
-// the 256 lanes read 256 consecutive words.  A count of 2^20 or more in a
-// cell with a group sets *bad_out (the same cells the data's own set sums).
+// 32-51 l, 20-31 and 52-55 twice the cell's position in the family (the byte
+// of its 16-bit draw counter, low 12 and high 4 bits), 56-63 its group + 1 (0:
+// a cell in no group, or padding).  Per gene the families follow one another
+// (pulse, chase, all cells by condition, all cells by (condition, cluster)),
+// each in ceil(m / 256) * 256 slots, transposed: slot j * 256 + t holds sorted
+// position t * ceil(m / 256) + j, so that lane t of data_stats_sorted_kernel
+// walks a contiguous run of the sorted cells while the 256 lanes read 256
+// consecutive words.  The largest u + l of each 64 slots goes to xmax (one
+// address per gene and an atomic per wave took 0.6 ms more).  A count of 2^20
+// or more in a cell with a group sets *bad_out (the same cells the data's own
+// set sums).
 // Workgroup L packs block (item % (slots / 256)) of gene item / (slots /
 // 256), item = (L % 8) * (gridDim.x / 8) + L / 8, so that one XCD reads
 // each gene's counts.
@@ -303,7 +300,8 @@ __global__ __launch_bounds__(256) void data_pack_kernel(
     int64_t n, const uint32_t* __restrict__ u, const uint32_t* __restrict__ l, int64_t g0,
     const int32_t* __restrict__ pulse, int64_t np, const int32_t* __restrict__ chase, int64_t nch,
     const int32_t* __restrict__ perm, const int32_t* __restrict__ grp, int64_t slots,
-    int64_t genes, unsigned long long* __restrict__ xs, unsigned int* __restrict__ bad_out) {
+    int64_t genes, unsigned long long* __restrict__ xs, uint32_t* __restrict__ xmax,
+    unsigned int* __restrict__ bad_out) {
   const int64_t item = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int64_t nblk = slots / 256;
   if (item >= genes * nblk) return;
@@ -317,6 +315,7 @@ __global__ __launch_bounds__(256) void data_pack_kernel(
   else { f = 3; at = s - 256 * (c0 + c1 + c2); m = n; base = np + nch + n; cf = c2; }
   const int64_t k = (at & 255) * cf + (at >> 8);
   unsigned long long word = 0ull;
+  uint32_t sum = 0;
   if (k < m) {
     const int gk = grp[base + k];
     if (gk >= 0) {
@@ -325,12 +324,28 @@ __global__ __launch_bounds__(256) void data_pack_kernel(
       const uint32_t x0 = u[g * n + i], x1 = l[g * n + i];
       if ((x0 | x1) >= (1u << 20)) atomicOr(bad_out, 1u);
       else
-        word = (unsigned long long)x0 | (unsigned long long)x1 << 20 |
-               (unsigned long long)pos << 40 | (unsigned long long)(gk + 1) << 56;
+        word = (unsigned long long)x0 | (unsigned long long)x1 << 32 |
+               (unsigned long long)((2 * pos) & 0xFFF) << 20 |
+               (unsigned long long)((2 * pos) >> 12) << 52 | (unsigned long long)(gk + 1) << 56;
+      if ((x0 | x1) < (1u << 20)) sum = x0 + x1;
     }
   }
   xs[gl * slots + s] = word;
+  for (int o = 32; o > 0; o >>= 1) sum = max(sum, (uint32_t)__shfl_xor((int)sum, o));
+  if ((threadIdx.x & 63) == 0) xmax[(gl * slots + s) / 64] = sum;
 }
+
+// *bad_out |= 1 if a count of u or l is 2^20 or more
+__global__ __launch_bounds__(256) void data_check_kernel(int64_t n, const uint32_t* __restrict__ u,
+                                                         const uint32_t* __restrict__ l,
+                                                         unsigned int* __restrict__ bad_out) {
+  uint32_t x = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    x |= u[i] | l[i];
+  if (x >= (1u << 20)) atomicOr(bad_out, 1u);
+}
+
+size_t data_sorted_lds(int64_t mm) { return (size_t)((mm + 3) / 4 * 8) + sizeof(DataLds); }
 
 // The same statistics for genes whose families hold at most
 // ABC_DATA_SORTED_MAX cells, with the sets spread over workgroups: gene g0 +
@@ -346,19 +361,40 @@ __global__ __launch_bounds__(256) void data_pack_kernel(
 // count-weighted values in registers and adds them to the group's sums
 // where its run changes group.  The integer sums are those of
 // data_stats_kernel, regrouped, so the statistics are identical.
-// data_se_kernel then forms the standard errors.  Eight waves per SIMD
-// (64 VGPRs): the values spilled are kept per set, outside the draw and cell loops.
+// data_se_kernel then forms the standard errors.
+// SMALL: the genes whose largest u + l, squared, times the largest family's
+// cells is below 2^32 (u + l up to 889 at 5,422 cells: nearly every gene of
+// such data), so that every sum of a lane's run fits 32 bits and a term is one
+// 24-bit multiply-add; the other genes are summed in 64 bits.  Which kind a
+// gene is, only the device knows (xmax, of data_pack_kernel), so both are
+// launched and each leaves the other's genes at once (33 us for 3,419 genes).
+// VALU issue bounds it: a Philox block and two position products per two
+// draws, 21 multiplies of a quarter of the rate and about 40 other
+// instructions, then 9 to 16 per cell walked (25 to 45 in 64 bits).  3,419
+// genes of 5,422 cells, 100 resamples: 10.7 ms (12.6 with every sum in 64
+// bits and both words of each position product), of the 9.9 ms that the
+// 5.6e9 draws and cells take at that count.
+template <bool SMALL>
 __global__ __launch_bounds__(ABC_DATA_WG) __attribute__((amdgpu_waves_per_eu(8))) void
 data_stats_sorted_kernel(
     int64_t genes, int nsb, int64_t g0, const unsigned long long* __restrict__ xs, int64_t slots,
-    int64_t n, int64_t np, int64_t nch, int nc, int J, const double* __restrict__ w_point,
-    int n_boot, int spb, uint32_t k0, uint32_t k1, double* __restrict__ pt,
-    double* __restrict__ boot) {
-  extern __shared__ uint32_t mult_sh[];  // two 16-bit counters per word
-  __shared__ DataLds S;
+    const uint32_t* __restrict__ xmax, int64_t n, int64_t np, int64_t nch, int nc, int J,
+    const double* __restrict__ w_point, int n_boot, int spb, uint32_t k0, uint32_t k1,
+    double* __restrict__ pt, double* __restrict__ boot) {
+  // two 16-bit counters per word, at LDS address 0, then the sums (data_sorted_lds)
+  extern __shared__ __attribute__((aligned(16))) uint32_t mult_sh[];
   const int64_t item = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (item >= genes * nsb) return;  // the whole workgroup: padding to a multiple of 8
   const int64_t gl = item / nsb;  // gene within this launch
+  const int64_t mm = n > np ? (n > nch ? n : nch) : (np > nch ? np : nch);
+  DataLds& S = *reinterpret_cast<DataLds*>(mult_sh + (mm + 3) / 4 * 2);
+  bool over = false;
+  for (int64_t i = threadIdx.x; i < slots / 64; i += ABC_DATA_WG) {
+    const unsigned long long x = xmax[gl * (slots / 64) + i];
+    over = over || x * x * (unsigned long long)mm >= (1ull << 32);
+  }
+  if ((__syncthreads_or(over) == 0) != SMALL) return;  // the whole workgroup
+  using Sum = typename std::conditional<SMALL, uint32_t, unsigned long long>::type;
   const int64_t g = g0 + gl;
   const int tid = threadIdx.x;
   const unsigned long long* xg = xs + gl * slots;
@@ -366,6 +402,8 @@ data_stats_sorted_kernel(
   double* bg = boot + (size_t)gl * (size_t)n_boot * (size_t)K1;
   const int s_lo = (int)(item - gl * nsb) * spb;
   const int s_hi = s_lo + spb < n_boot + 1 ? s_lo + spb : n_boot + 1;
+  unsigned char* mult_b = reinterpret_cast<unsigned char*>(mult_sh);
+  typedef unsigned short __attribute__((may_alias)) half_word;
   for (int set = s_lo; set < s_hi; ++set) {
     const int b = set - 1;
     for (int i = tid; i < 2 * 3 * MC + 3 * MJ + 6 * MJ * MC; i += ABC_DATA_WG) {
@@ -373,87 +411,125 @@ data_stats_sorted_kernel(
       else if (i < 2 * 3 * MC + 3 * MJ) (&S.rat[0][0])[i - 2 * 3 * MC] = 0ull;
       else (&S.cor[0][0][0])[i - 2 * 3 * MC - 3 * MJ] = 0ull;
     }
-    int64_t fb = 0;  // the family's first slot
+    const unsigned long long* xf = xg + tid;  // the family's first slot of this lane
     // unrolled: each family's cell walk is compiled with its own sums and no
     // branch on the family per cell
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
-      const int64_t m = f == 0 ? np : (f == 1 ? nch : n);
-      const int64_t cf = (m + ABC_DATA_WG - 1) / ABC_DATA_WG;
+      const uint32_t m = (uint32_t)(f == 0 ? np : (f == 1 ? nch : n));
+      const uint32_t cf = (m + ABC_DATA_WG - 1) / ABC_DATA_WG;
+      // the data themselves: every cell once
+      for (uint32_t i = tid; 2 * i < m; i += ABC_DATA_WG) mult_sh[i] = b < 0 ? 0x10001u : 0u;
       if (b >= 0) {
-        for (int64_t i = tid; 2 * i < m; i += ABC_DATA_WG) mult_sh[i] = 0u;
         __syncthreads();
-        for (int64_t q = tid; 2 * q < m; q += ABC_DATA_WG) {
-          const u4 w = philox((uint32_t)q, (uint32_t)b, (uint32_t)g, (uint32_t)f, k0, k1);
-          const uint32_t p0 = pos_of32(w, 0, (uint32_t)m);
-          atomicAdd(&mult_sh[p0 >> 1], 1u << (16 * (p0 & 1)));
-          if (2 * q + 1 < m) {
-            const uint32_t p1 = pos_of32(w, 1, (uint32_t)m);
-            atomicAdd(&mult_sh[p1 >> 1], 1u << (16 * (p1 & 1)));
-          }
+        // a position is the high word of hi m + floor(lo m / 2^32): that of
+        // hi m alone unless its low word is within m of a carry
+        auto count = [&](uint32_t lo, uint32_t hi) {
+          uint64_t pr = (uint64_t)hi * m;
+          if ((uint32_t)pr > ~m) pr += __umulhi(lo, m);
+          uint32_t p = (uint32_t)(pr >> 32);
+          asm("" : "+v"(p));  // formed as a 64-bit shift otherwise, for one more instruction
+          atomicAdd(&mult_sh[p >> 1], 1u << ((p << 4) & 31u));
+        };
+        uint32_t q = tid;
+        for (; q < m / 2; q += ABC_DATA_WG) {
+          const u4 w = philox(q, (uint32_t)b, (uint32_t)g, (uint32_t)f, k0, k1);
+          count(w.x, w.y);
+          count(w.z, w.w);
+        }
+        if (2 * q + 1 == m) {  // the last draw of an odd number
+          const u4 w = philox(q, (uint32_t)b, (uint32_t)g, (uint32_t)f, k0, k1);
+          count(w.x, w.y);
         }
       }
       __syncthreads();
-      int cur = -1;
-      unsigned long long a0 = 0, a1 = 0, a2 = 0, a3 = 0, a4 = 0, a5 = 0;
+      int cur = 0;  // group + 1
+      Sum a0 = 0, a1 = 0, a2 = 0, a3 = 0, a4 = 0, a5 = 0;
       auto flush = [&]() {
-        if (cur < 0 || a0 == 0ull) return;
+        if (cur == 0 || a0 == 0) return;
+        const int gr = cur - 1;
+        auto add = [](unsigned long long* p, Sum v) { atomicAdd(p, (unsigned long long)v); };
         if (f < 2) {
-          atomicAdd(&S.ccp[f][0][cur], a0);
-          atomicAdd(&S.ccp[f][1][cur], a1);
-          atomicAdd(&S.ccp[f][2][cur], a2);
+          add(&S.ccp[f][0][gr], a0);
+          add(&S.ccp[f][1][gr], a1);
+          add(&S.ccp[f][2][gr], a2);
         } else if (f == 2) {
-          atomicAdd(&S.rat[0][cur], a0);
-          atomicAdd(&S.rat[1][cur], a1);
-          atomicAdd(&S.rat[2][cur], a2);
+          add(&S.rat[0][gr], a0);
+          add(&S.rat[1][gr], a1);
+          add(&S.rat[2][gr], a2);
         } else {
-          const int j = cur / nc, c = cur - (cur / nc) * nc;
-          atomicAdd(&S.cor[0][j][c], a0);
-          atomicAdd(&S.cor[1][j][c], a1);
-          atomicAdd(&S.cor[2][j][c], a2);
-          atomicAdd(&S.cor[3][j][c], a3);
-          atomicAdd(&S.cor[4][j][c], a4);
-          atomicAdd(&S.cor[5][j][c], a5);
+          const int j = gr / nc, c = gr - (gr / nc) * nc;
+          add(&S.cor[0][j][c], a0);
+          add(&S.cor[1][j][c], a1);
+          add(&S.cor[2][j][c], a2);
+          add(&S.cor[3][j][c], a3);
+          add(&S.cor[4][j][c], a4);
+          add(&S.cor[5][j][c], a5);
         }
       };
-      const unsigned long long* xf = xg + fb + tid;
-      for (int64_t j = 0; j < cf; ++j) {
-        const unsigned long long v = xf[j * ABC_DATA_WG];
-        const int gk = (int)(v >> 56) - 1;
+      unsigned long long next = cf > 0 ? xf[0] : 0ull;
+      for (uint32_t j = 0; j < cf; ++j) {
+        const unsigned long long v = next;
+        next = xf[(size_t)(j + 1 < cf ? j + 1 : j) * ABC_DATA_WG];
+        const uint32_t vl = (uint32_t)v, vh = (uint32_t)(v >> 32);
+        const int gk = (int)(vh >> 24);
         if (gk != cur) {
           flush();
           cur = gk;
-          a0 = a1 = a2 = a3 = a4 = a5 = 0ull;
+          a0 = a1 = a2 = a3 = a4 = a5 = 0;
         }
-        if (gk < 0) continue;
-        const uint32_t pos = (uint32_t)(v >> 40) & 0xFFFFu;
-        const uint32_t mult = b < 0 ? 1u : (mult_sh[pos >> 1] >> (16 * (pos & 1))) & 0xFFFFu;
-        if (mult == 0u) continue;
-        const unsigned long long x0 = v & 0xFFFFFull, x1 = (v >> 20) & 0xFFFFFull;
-        const unsigned long long mm = mult;
-        a0 += mm;
-        if (f < 2) {
-          const unsigned long long x = x0 + x1;
-          a1 += mm * x;
-          a2 += mm * (x * x);
+        const uint32_t at = (vl >> 20) | ((vh >> 8) & 0xF000u);
+        // cells in no group are summed too and never flushed
+        const uint32_t mult = *reinterpret_cast<const half_word*>(mult_b + at);
+        const uint32_t x0 = vl & 0xFFFFFu, x1 = vh & 0xFFFFFu;
+        a0 += mult;
+        if (SMALL) {
+          if (f < 2) {
+            const uint32_t x = x0 + x1, t = __umul24(mult, x);
+            a1 += t;
+            a2 += __umul24(t, x);
+          } else {
+            const uint32_t t0 = __umul24(mult, x0), t1 = __umul24(mult, x1);
+            a1 += t0;
+            a2 += t1;
+            if (f == 3) {
+              a3 += __umul24(t0, x0);
+              a4 += __umul24(t1, x1);
+              a5 += __umul24(t0, x1);
+            }
+          }
         } else {
-          a1 += mm * x0;
-          a2 += mm * x1;
-          if (f == 3) {
-            a3 += mm * (x0 * x0);
-            a4 += mm * (x1 * x1);
-            a5 += mm * (x0 * x1);
+          const unsigned long long mm = mult;
+          if (f < 2) {
+            const unsigned long long x = x0 + x1;
+            a1 += (Sum)(mm * x);
+            a2 += (Sum)(mm * (x * x));
+          } else {
+            const unsigned long long y0 = x0, y1 = x1;
+            a1 += (Sum)(mm * y0);
+            a2 += (Sum)(mm * y1);
+            if (f == 3) {
+              a3 += (Sum)(mm * (y0 * y0));
+              a4 += (Sum)(mm * (y1 * y1));
+              a5 += (Sum)(mm * (y0 * y1));
+            }
           }
         }
       }
       flush();
       __syncthreads();
-      fb += cf * ABC_DATA_WG;
+      xf += (size_t)cf * ABC_DATA_WG;
     }
     finish_set(S, tid, b, nc, J, w_point, b < 0 ? pt + (size_t)gl * K1 : bg + (size_t)b * K1);
     __syncthreads();
   }
 }
+template __global__ void data_stats_sorted_kernel<true>(
+    int64_t, int, int64_t, const unsigned long long*, int64_t, const uint32_t*, int64_t, int64_t,
+    int64_t, int, int, const double*, int, int, uint32_t, uint32_t, double*, double*);
+template __global__ void data_stats_sorted_kernel<false>(
+    int64_t, int, int64_t, const unsigned long long*, int64_t, const uint32_t*, int64_t, int64_t,
+    int64_t, int, int, const double*, int, int, uint32_t, uint32_t, double*, double*);
 
 // Standard errors of data_stats_sorted_kernel's sets: one lane per (gene,
 // statistic) of the launch, the same sums in resample order as write_se.

@@ -226,9 +226,14 @@ __global__ void data_pack_kernel(int64_t n, const uint32_t* u, const uint32_t* l
                                  const int32_t* pulse, int64_t np, const int32_t* chase,
                                  int64_t nch, const int32_t* perm, const int32_t* grp,
                                  int64_t slots, int64_t genes, unsigned long long* xs,
-                                 unsigned int* bad_out);
+                                 uint32_t* xmax, unsigned int* bad_out);
+__global__ void data_check_kernel(int64_t n, const uint32_t* u, const uint32_t* l,
+                                  unsigned int* bad_out);
+size_t data_sorted_lds(int64_t mm);  // its LDS bytes, for families of up to mm cells
+template <bool SMALL>
 __global__ void data_stats_sorted_kernel(int64_t genes, int nsb, int64_t g0,
-                                         const unsigned long long* xs, int64_t slots, int64_t n,
+                                         const unsigned long long* xs, int64_t slots,
+                                         const uint32_t* xmax, int64_t n,
                                          int64_t np, int64_t nch, int nc, int J,
                                          const double* w_point, int n_boot, int spb, uint32_t k0,
                                          uint32_t k1, double* pt, double* boot);
