@@ -1269,7 +1269,8 @@ int screen_run(abc_ctx* c, abc_mlp* mlp, int64_t n, const float* x_dev, const fl
   rc = abc_mlp_forward_dev(mlp, n, x_dev, P<float>(c->sy));
   if (rc) return fail(c, rc, "surrogate forward failed");
   if ((rc = abc_mlp_synchronize(mlp))) return fail(c, rc, "surrogate forward failed");
-  hipLaunchKernelGGL(screen_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(score_dev ? screen_kernel<true> : screen_kernel<false>,
+                     dim3((unsigned)((n + ABC_SCREEN_PT - 1) / ABC_SCREEN_PT)), dim3(256), 0, c->stream,
                      P<float>(c->sy), n, A.E.K, mean_dev, sd_dev, (float)z, P<float>(c->wf),
                      P<double>(c->edata), A.G, P<double>(c->thr), (float)margin, A.E.clamp,
                      pass_dev, score_dev);

@@ -269,6 +269,8 @@ __global__ void gene_prep_kernel(const double* data, const double* se, int64_t G
                                  int64_t Gpad, __bf16* Bh, __bf16* Bl, double* cg, uint8_t* gflag,
                                  float* Wf, ErrGene* genes);
 // surrogate screen (abc_mlp.hip)
+#define ABC_SCREEN_PT 8  // particles per workgroup of screen_kernel
+template <bool SCORE>
 __global__ void screen_kernel(const float* y, int64_t n, int K, const float* mean, const float* sd,
                               float z, const float* Wf, const double* data, int64_t G,
                               const double* thr, float margin, double clamp, uint8_t* pass, float* score);

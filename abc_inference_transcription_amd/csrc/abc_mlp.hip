@@ -605,7 +605,33 @@ __global__ void targets_kernel(int64_t n, const double* __restrict__ stats, int 
 // with delta = d - E s.  A particle passes when E err - z sd err can reach a
 // gene's threshold (or when its prediction is not finite).  Genes whose data
 // are not finite have NaN errors and accept nobody.
-__global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y, int64_t n, int K,
+//
+// A workgroup holds the moments of PT particles in LDS; a lane scores genes g
+// and g + 256 against all of them.  A (particle, statistic, gene) term is 13
+// FP32 instructions, and one 16-byte and a quarter of a 16-byte LDS read serve
+// two: the reference expression
+//   4 delta delta c2 - 4 delta c3 + c4 - c2 c2  (16, four 4-byte LDS reads)
+// with the powers of two moved to c4 / 4, c2 c2 / 4 and 4 W^2, which changes no
+// bit while nothing overflows and no product is subnormal: moments and data
+// inside screen_safe's and SCREEN_BIG's ranges.  A workgroup that holds a
+// moment outside them, and a gene with such a datum, are scored with the
+// expression as it stands.  VALU issue bounds it: 40,000 particles, 2,000 genes,
+// 90 statistics in 2.0 ms with the moments and the normal integrals (2.5 ms
+// with 16 particles of one gene a lane and the expression as it stands; 7.2e9
+// terms of 13 instructions take 1.8 ms at the 3 cycles each that FP32
+// reaches).  500 particles: 0.28 ms for 1.04, as 8 particles a workgroup fill
+// more of the chip.  Four waves per SIMD: with five or six the sums spill (2.3
+// and 2.5 ms).
+#define SCREEN_BIG 0x1p30f
+ABC_DEV bool screen_safe(float e, float v2, float v3, float v4) {
+  // |delta| is 0 or at least 2^-44 then, and every product at least 2^-126
+  const float ae = fabsf(e), a3 = fabsf(v3);
+  return ae >= 0x1p-20f && ae <= SCREEN_BIG && v2 >= 0x1p-38f && v2 <= SCREEN_BIG &&
+         a3 >= 0x1p-80f && a3 <= 0x1p45f && v4 >= 0x1p-100f && v4 <= 0x1p60f;
+}
+
+template <bool SCORE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void screen_kernel(const float* __restrict__ y, int64_t n, int K,
                                                      const float* __restrict__ mean,
                                                      const float* __restrict__ sd, float z,
                                                      const float* __restrict__ Wf,
@@ -613,10 +639,10 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
                                                      const double* __restrict__ thr, float margin,
                                                      double clamp, uint8_t* __restrict__ pass,
                                                      float* __restrict__ score) {
-  constexpr int PT = 16;
-  __shared__ float e1[PT][ABC_MAX_STATS / 2], c2[PT][ABC_MAX_STATS / 2];
-  __shared__ float c3[PT][ABC_MAX_STATS / 2], c4[PT][ABC_MAX_STATS / 2];
-  __shared__ int hit[PT], bad[PT];
+  constexpr int PT = ABC_SCREEN_PT;
+  __shared__ float4 mo[ABC_MAX_STATS / 2][PT];  // E s, c2, c3, c4 (plain: c4 / 4)
+  __shared__ __attribute__((aligned(16))) float qv[ABC_MAX_STATS / 2][PT];  // c2 c2 / 4
+  __shared__ int hit[PT], bad[PT], general;
   __shared__ float s_sum[4][PT], s_max[4][PT];  // per wave: expected pairs, largest margin
   const double gx[7] = {-3.7504397177257425, -2.366759410734541, -1.1544053947399682, 0.0,
                         1.1544053947399682, 2.366759410734541, 3.7504397177257425};
@@ -628,12 +654,14 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
     hit[threadIdx.x] = (i0 + threadIdx.x < n) ? 0 : 1;
     bad[threadIdx.x] = 0;
   }
+  if (threadIdx.x == 0) general = 0;
   __syncthreads();
   for (int q = threadIdx.x; q < PT * K; q += blockDim.x) {
     const int p = q / K, k = q % K;
     const int64_t i = i0 + p;
-    double m1 = 0.0, v2 = 0.0, v3 = 0.0, v4 = 0.0;
+    double m1 = 1.0, v2 = 1.0, v3 = 1.0, v4 = 1.0;  // past n: anything in range
     if (i < n) {
+      m1 = v2 = v3 = v4 = 0.0;
       const double mu = y[i * 2 * K + k];
       const double lv = fmin(fmax((double)y[i * 2 * K + K + k], -12.0), 12.0);
       const double s = exp(0.5 * lv);
@@ -650,28 +678,38 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
       }
       if (!(fabs(m1) < 1e30) || !(v4 < 1e300)) hit[p] = bad[p] = 1;
     }
-    e1[p][k] = (float)m1;
-    c2[p][k] = (float)v2;
-    c3[p][k] = (float)v3;
-    c4[p][k] = (float)v4;
+    const float4 m = {(float)m1, (float)v2, (float)v3, (float)v4};
+    mo[k][p] = m;
+    qv[k][p] = m.y * m.y * 0.25f;
+    if (!screen_safe(m.x, m.y, m.z, m.w)) general = 1;  // benign race: every writer stores 1
   }
   __syncthreads();
+  const bool plain = general == 0;  // the whole workgroup
+  if (plain) {
+    for (int q = threadIdx.x; q < PT * K; q += blockDim.x) mo[q / PT][q % PT].w *= 0.25f;
+    __syncthreads();
+  }
   // per particle over this thread's genes: sum of P(err <= t) under the
   // Gaussian approximation, and the largest standardised margin (t - E) / sd
   float psum[PT], pmax[PT];
 #pragma unroll
   for (int p = 0; p < PT; ++p) { psum[p] = 0.f; pmax[p] = -HUGE_VALF; }
-  for (int64_t g = threadIdx.x; g < G; g += blockDim.x) {
-    const double tg = thr[g];
-    if (tg >= clamp) {  // every clamped error ties at the threshold: nobody may be skipped
-      for (int p = 0; p < PT; ++p) {
-        hit[p] = 1;
-        psum[p] += 1.f;
-        pmax[p] = HUGE_VALF;
+  auto finish = [&](float t, const float (&em)[PT], const float (&ev)[PT]) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p) {
+      const float sdv = sqrtf(ev[p]);
+      if (em[p] - z * sdv <= t) hit[p] = 1;  // benign race: every writer stores 1
+      if (SCORE) {
+        const float d = t - em[p];
+        const float u = sdv > 0.f ? d / sdv : (d >= 0.f ? HUGE_VALF : -HUGE_VALF);
+        psum[p] += normcdff(u);
+        pmax[p] = fmaxf(pmax[p], u);
       }
-      continue;
     }
-    const float t = (float)(tg * (1.0 + (double)margin));
+  };
+  // gene g by the expression as it stands
+  auto gene = [&](int64_t g, float t) {
+    const float back = plain ? 4.f : 1.f;  // c4 from mo
     float em[PT], ev[PT];
 #pragma unroll
     for (int p = 0; p < PT; ++p) { em[p] = 0.f; ev[p] = 0.f; }
@@ -681,25 +719,71 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
       const float w2 = w * w;
 #pragma unroll
       for (int p = 0; p < PT; ++p) {
-        const float dl = d - e1[p][k];
-        const float a = c2[p][k];
-        em[p] += w * (dl * dl + a);
-        ev[p] += w2 * fmaxf(4.f * dl * dl * a - 4.f * dl * c3[p][k] + c4[p][k] - a * a, 0.f);
+        const float4 m = mo[k][p];
+        const float dl = d - m.x;
+        em[p] += w * (dl * dl + m.y);
+        ev[p] += w2 * fmaxf(4.f * dl * dl * m.y - 4.f * dl * m.z + back * m.w - m.y * m.y, 0.f);
       }
     }
+    finish(t, em, ev);
+  };
+  for (int64_t g = threadIdx.x; g < G; g += 512) {
+    float t[2];
+    bool run[2];
 #pragma unroll
-    for (int p = 0; p < PT; ++p) {
-      const float sd = sqrtf(ev[p]);
-      if (em[p] - z * sd <= t) hit[p] = 1;  // benign race: every writer stores 1
-      if (score) {
-        const float d = t - em[p];
-        const float u = sd > 0.f ? d / sd : (d >= 0.f ? HUGE_VALF : -HUGE_VALF);
-        psum[p] += normcdff(u);
-        pmax[p] = fmaxf(pmax[p], u);
+    for (int h = 0; h < 2; ++h) {
+      const int64_t gh = g + 256 * h;
+      const double tg = gh < G ? thr[gh] : 0.0;
+      // a clamped threshold is every clamped error's: nobody may be skipped
+      run[h] = gh < G && !(tg >= clamp);
+      t[h] = (float)(tg * (1.0 + (double)margin));
+    }
+    float em0[PT], ev0[PT], em1[PT], ev1[PT], big = 0.f, big1 = 0.f;
+    const bool both = plain && (run[0] || run[1]);
+    if (both) {
+      const int64_t ga = run[0] ? g : g + 256, gb = run[1] ? g + 256 : g;
+#pragma unroll
+      for (int p = 0; p < PT; ++p) em0[p] = ev0[p] = em1[p] = ev1[p] = 0.f;
+      for (int k = 0; k < K; ++k) {
+        const float d0 = (float)data[ga + G * k], d1 = (float)data[gb + G * k];
+        const float w0 = Wf[ga + G * k], w1 = Wf[gb + G * k];
+        big = fmaxf(fmaxf(big, fabsf(d0)), w0);
+        big1 = fmaxf(fmaxf(big1, fabsf(d1)), w1);
+        const float x0 = 4.f * (w0 * w0), x1 = 4.f * (w1 * w1);
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+          const float4 m = mo[k][p];
+          const float q = qv[k][p];
+          const float a = d0 - m.x, b = d1 - m.x;
+          const float aa = a * a, bb = b * b;
+          em0[p] += w0 * (aa + m.y);
+          em1[p] += w1 * (bb + m.y);
+          ev0[p] += x0 * fmaxf(aa * m.y - a * m.z + m.w - q, 0.f);
+          ev1[p] += x1 * fmaxf(bb * m.y - b * m.z + m.w - q, 0.f);
+        }
       }
+    }
+#pragma unroll 1
+    for (int h = 0; h < 2 && g + 256 * h < G; ++h) {  // one copy of the code
+      if (!run[0]) {
+        for (int p = 0; p < PT; ++p) {
+          hit[p] = 1;
+          psum[p] += 1.f;
+          pmax[p] = HUGE_VALF;
+        }
+      } else if (both && big <= SCREEN_BIG) {
+        finish(t[0], em0, ev0);
+      } else {
+        gene(g + 256 * h, t[0]);
+      }
+#pragma unroll
+      for (int p = 0; p < PT; ++p) { em0[p] = em1[p]; ev0[p] = ev1[p]; }
+      run[0] = run[1];
+      t[0] = t[1];
+      big = big1;
     }
   }
-  if (score) {
+  if (SCORE) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int p = 0; p < PT; ++p) {
@@ -715,7 +799,7 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
   if (threadIdx.x < PT && i0 + threadIdx.x < n) {
     const int p = threadIdx.x;
     pass[i0 + p] = (uint8_t)hit[p];
-    if (score) {
+    if (SCORE) {
       // a prediction that is not finite passes whatever the threshold
       float a = 0.f, b = -HUGE_VALF;
       for (int w = 0; w < 4; ++w) { a += s_sum[w][p]; b = fmaxf(b, s_max[w][p]); }
@@ -724,6 +808,14 @@ __global__ __launch_bounds__(256) void screen_kernel(const float* __restrict__ y
     }
   }
 }
+template __global__ void screen_kernel<false>(const float*, int64_t, int, const float*,
+                                              const float*, float, const float*, const double*,
+                                              int64_t, const double*, float, double, uint8_t*,
+                                              float*);
+template __global__ void screen_kernel<true>(const float*, int64_t, int, const float*,
+                                             const float*, float, const float*, const double*,
+                                             int64_t, const double*, float, double, uint8_t*,
+                                             float*);
 
 struct abc_mlp {
   int device = 0;
