@@ -27,11 +27,11 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-enum { EPI_F32 = 0, EPI_SILU = 1, EPI_DSILU = 2 };
+enum { EPI_F32 = 0, EPI_SILU = 1, EPI_DSILU = 2, EPI_DW = 3 };
 
-// K per pipeline stage (two 32-deep MFMA steps) and the LDS row length
-// (+8 bf16 of padding against bank conflicts)
-constexpr int BK = 64, LDSK = BK + 8;
+// K per pipeline stage (32-deep MFMA steps): 64, and 128 for the weight
+// gradients, whose few workgroups per CU wait at every stage's barrier
+constexpr int stage_k(int epi) { return epi == EPI_DW ? 128 : 64; }
 
 // s = 1 / (1 + e^-z) of four values.  The reciprocals of x = 1 + e^-z >= 1 are
 // correctly rounded without the division sequence: the hardware's reciprocal
@@ -52,13 +52,26 @@ __device__ __forceinline__ void sigm4(const float* z, float* s) {
   }
 }
 
-// 256 threads, workgroup tile BM x BN (BM 128 or 64), wave tile BM/2 x BN/2
-// (2 x 2 waves).  blockIdx.z selects a K chunk [z*K, (z+1)*K) of rows with
-// leading dimension ld (split-K: EPI_F32 then writes its partial tile to
-// Cf + z*M*N).  K advances in stages of BK = 64 through two LDS buffers: while
-// the MFMAs read one stage, the next is loaded from global memory into
-// registers and stored to the other buffer, one barrier per stage.  Every
-// output sums its K in order, 32 at a time, whatever BM.
+struct GemmArgs {
+  const bf16 *A, *B;
+  int M, N, K, ld;
+  const float* bias;
+  float* Cf;
+  bf16 *Cb, *CbT;
+  const float* Zprev;
+  float* Zout;
+};
+
+// 256 threads, workgroup tile BM x BN (128 or 64 each), wave tile BM/2 x BN/2 (2
+// x 2 waves).  EPI_DW sums K chunk z, [z*K, (z+1)*K), of rows with leading
+// dimension ld (all of K): it writes its partial tile to Cf + z*M*N, and the
+// partial row sums of A, its product with a column of ones, to Zout + z*M: a
+// weight gradient and its bias's in one launch.  K advances in stages of BK
+// through two LDS buffers: while the MFMAs read one stage, the next is loaded
+// from global memory into registers and stored to the other buffer, one barrier
+// per stage (two or four stages in flight, or padded rows, measured the same:
+// the LDS is busy for 70 % of a workgroup's life).  Every output sums its K in
+// order, 32 at a time, whatever the tile.
 template <int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A,
                                                       const bf16* __restrict__ B, int M, int N,
@@ -68,48 +81,67 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
                                                       bf16* __restrict__ CbT,
                                                       const float* __restrict__ Zprev,
                                                       float* __restrict__ Zout) {
-  constexpr int WN = BN / 2, NCB = WN / 16, NBQ = BN / 32;
-  constexpr int WM = BM / 2, NRB = WM / 16, NAQ = BM / 32;
+  constexpr int WN = BN / 2, NCB = WN / 16;
+  constexpr int WM = BM / 2, NRB = WM / 16;
+  constexpr int BK = stage_k(EPI), LDSK = BK + 8;  // 8 of padding against bank conflicts
+  constexpr int BQ = BK / 8;                       // 16-byte pieces of a row's stage
+  constexpr int NAQ = BM * BQ / 256, NBQ = BN * BQ / 256;
   __shared__ bf16 As[2][BM][LDSK];
   __shared__ bf16 Bs[2][BN][LDSK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kbeg = blockIdx.z * K, kend = kbeg + K;
-  if (EPI == EPI_F32) Cf += (size_t)blockIdx.z * M * N;
+  // EPI_DW: K chunks fastest, so that one XCD's workgroups (every eighth) share
+  // their chunks of A and B; with the row tiles fastest each XCD read an eighth
+  // of A and all of B (8,192 x 512 x 512: 14.4 us, 13.7 so)
+  const int bx = EPI == EPI_DW ? blockIdx.y : blockIdx.x;
+  const int by = EPI == EPI_DW ? blockIdx.z : blockIdx.y, bz = EPI == EPI_DW ? blockIdx.x : 0;
+  const int m0 = bx * BM, n0 = by * BN;
+  const int kbeg = bz * K, kend = min(kbeg + K, ld);  // empty: past the last chunk
+  if (EPI == EPI_DW) {
+    Cf += (size_t)bz * M * N;
+    Zout += (size_t)bz * M;
+  }
+  const bool rows = EPI == EPI_DW && by == 0 && wn == 0;  // the wave sums A's rows
+  const bf16 one = (bf16)1.0f;
+  const bf16x8 ones = {one, one, one, one, one, one, one, one};
+  f32x4 rs[NRB];
+#pragma unroll
+  for (int a = 0; a < NRB; ++a) rs[a] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 acc[NRB][NCB];
 #pragma unroll
   for (int a = 0; a < NRB; ++a)
 #pragma unroll
     for (int b = 0; b < NCB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // this thread's slice of a stage: rows c >> 3, 8 columns at (c & 7) * 8
+  // this thread's slice of a stage: rows c / BQ, 8 columns at c % BQ * 8
   bf16x8 ra[NAQ], rb[NBQ];
   auto load = [&](int k0) {
 #pragma unroll
     for (int q = 0; q < NAQ; ++q) {
       const int c = tid + q * 256;
-      ra[q] = *reinterpret_cast<const bf16x8*>(A + (size_t)(m0 + (c >> 3)) * ld + k0 + (c & 7) * 8);
+      ra[q] = *reinterpret_cast<const bf16x8*>(A + (size_t)(m0 + c / BQ) * ld + k0 + c % BQ * 8);
     }
 #pragma unroll
     for (int q = 0; q < NBQ; ++q) {
       const int c = tid + q * 256;
-      rb[q] = *reinterpret_cast<const bf16x8*>(B + (size_t)(n0 + (c >> 3)) * ld + k0 + (c & 7) * 8);
+      rb[q] = *reinterpret_cast<const bf16x8*>(B + (size_t)(n0 + c / BQ) * ld + k0 + c % BQ * 8);
     }
   };
   auto stash = [&](int buf) {
 #pragma unroll
     for (int q = 0; q < NAQ; ++q) {
       const int c = tid + q * 256;
-      *reinterpret_cast<bf16x8*>(&As[buf][c >> 3][(c & 7) * 8]) = ra[q];
+      *reinterpret_cast<bf16x8*>(&As[buf][c / BQ][c % BQ * 8]) = ra[q];
     }
 #pragma unroll
     for (int q = 0; q < NBQ; ++q) {
       const int c = tid + q * 256;
-      *reinterpret_cast<bf16x8*>(&Bs[buf][c >> 3][(c & 7) * 8]) = rb[q];
+      *reinterpret_cast<bf16x8*>(&Bs[buf][c / BQ][c % BQ * 8]) = rb[q];
     }
   };
-  load(kbeg);
-  stash(0);
+  if (kbeg < kend) {
+    load(kbeg);
+    stash(0);
+  }
   __syncthreads();
   int buf = 0;
   for (int k0 = kbeg; k0 < kend; k0 += BK) {
@@ -132,11 +164,19 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
         for (int cb = 0; cb < NCB; ++cb)
           acc[r4][cb] =
               __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[r4], bfr[cb], acc[r4][cb], 0, 0, 0);
+      if (rows)
+#pragma unroll
+        for (int r4 = 0; r4 < NRB; ++r4)
+          rs[r4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[r4], ones, rs[r4], 0, 0, 0);
     }
     if (more) stash(buf ^ 1);  // the other buffer: its last readers passed the barrier below
     __syncthreads();
     buf ^= 1;
   }
+  if (rows && (lane & 15) == 0)
+#pragma unroll
+    for (int r4 = 0; r4 < NRB; ++r4)
+      *reinterpret_cast<f32x4*>(Zout + m0 + wm * WM + r4 * 16 + (lane >> 4) * 4) = rs[r4];
 #pragma unroll
   for (int r4 = 0; r4 < NRB; ++r4)
 #pragma unroll
@@ -147,7 +187,7 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
       const int n = n0 + wn * WN + cb * 16 + (lane & 15);
       bf16x4 tv;
       float z[4], s[4];
-      if (EPI != EPI_F32) {
+      if (EPI == EPI_SILU || EPI == EPI_DSILU) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           z[q] = EPI == EPI_SILU ? acc[r4][cb][q] + bias[n] : Zprev[(size_t)(mb + q) * N + n];
@@ -159,7 +199,9 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
         float v = acc[r4][cb][q];
         const size_t o = (size_t)m * N + n;
         if (EPI == EPI_F32) {
-          if (bias) v += bias[n];
+          v += bias[n];
+          Cf[o] = v;
+        } else if (EPI == EPI_DW) {
           Cf[o] = v;
         } else if (EPI == EPI_SILU) {
           Zout[o] = z[q];
@@ -172,36 +214,42 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
           tv[q] = d;
         }
       }
-      if (EPI != EPI_F32) *reinterpret_cast<bf16x4*>(CbT + (size_t)n * M + mb) = tv;
+      if (EPI == EPI_SILU || EPI == EPI_DSILU)
+        *reinterpret_cast<bf16x4*>(CbT + (size_t)n * M + mb) = tv;
     }
 }
 
-// C[i] = sum over the S split-K partials P[s][i], in the order s = 0, 1, ...
-__global__ void splitk_reduce_kernel(const float* __restrict__ P, int S, int64_t MN,
-                                     float* __restrict__ C) {
-  // four consecutive outputs per thread (MN is a multiple of 4)
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= MN) return;
-  float4 v = *reinterpret_cast<const float4*>(P + i);
-  for (int s = 1; s < S; ++s) {
-    const float4 w = *reinterpret_cast<const float4*>(P + (size_t)s * MN + i);
-    v.x += w.x;
-    v.y += w.y;
-    v.z += w.z;
-    v.w += w.w;
+// x (B x n_in FP32, row-major) -> X (B x in_pad bf16) and X^T (in_pad x B), one
+// workgroup per 64 x 64 tile, the transpose through LDS (element by element,
+// its scattered 2-byte stores took 7.0 us for 8,192 x 64, 4.2 so).  *loss, if
+// given, starts at 0.
+__global__ __launch_bounds__(256) void cast_input_kernel(const float* __restrict__ x, int Bn,
+                                                         int Bpad, int n_in, int in_pad,
+                                                         bf16* __restrict__ X,
+                                                         bf16* __restrict__ XT,
+                                                         float* __restrict__ loss) {
+  __shared__ bf16 tile[64][64 + 2];
+  const int b0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  if (loss && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *loss = 0.0f;
+  const int k = k0 + tx;
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int b = b0 + 4 * i + ty;
+    v[i] = x[(size_t)(b < Bn ? b : 0) * n_in + (k < n_in ? k : 0)];
   }
-  *reinterpret_cast<float4*>(C + i) = v;
-}
-
-// x (B x n_in FP32, row-major) -> X (B x in_pad bf16) and X^T (in_pad x B).
-__global__ void cast_input_kernel(const float* __restrict__ x, int Bn, int Bpad, int n_in,
-                                  int in_pad, bf16* __restrict__ X, bf16* __restrict__ XT) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (int64_t)Bpad * in_pad) return;
-  const int b = (int)(q / in_pad), k = (int)(q % in_pad);
-  const float v = (b < Bn && k < n_in) ? x[(size_t)b * n_in + k] : 0.0f;
-  X[q] = (bf16)v;
-  XT[(size_t)k * Bpad + b] = (bf16)v;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int b = b0 + 4 * i + ty;
+    const bf16 h = (bf16)(b < Bn && k < n_in ? v[i] : 0.0f);
+    X[(size_t)b * in_pad + k] = h;
+    tile[4 * i + ty][tx] = h;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    XT[(size_t)(k0 + 4 * i + ty) * Bpad + b0 + tx] = tile[tx][4 * i + ty];
 }
 
 // Gaussian negative log-likelihood per element, mean over B*ns.
@@ -225,38 +273,53 @@ __global__ __launch_bounds__(256) void nll_kernel(const float* __restrict__ O,
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 columns x 4 rows per pass
   const float scale = 1.0f / ((float)Bn * (float)ns);
   float l = 0.0f;
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int b = b0 + rr, k = k0 + tx;
-    float g = 0.0f;
-    if (b < Bn && k < 2 * ns) {
-      const int s = k < ns ? k : k - ns;
-      const float mu = O[(size_t)b * out_pad + s];
-      const float lv_raw = O[(size_t)b * out_pad + ns + s];
-      const bool clipped = lv_raw < -12.0f || lv_raw > 12.0f;
-      const float lv = fminf(fmaxf(lv_raw, -12.0f), 12.0f);
-      const float y = T[(size_t)b * ns + s];
-      const float r = y - mu;
-      const float inv = __expf(-lv);
-      if (s < n_cnt) {
-        if (k < ns) {
-          const float o = fminf(fmaxf(mu, -30.0f), 8.0f);
-          const float lam = __expf(o);
-          g = (lam - y) * scale;
-          l += ((lam - y * o) + (lam - y) * (mu - o)) * scale;
-        }
-      } else if (k < ns) {
-        g = -r * inv * scale;
-        l += 0.5f * (lv + r * r * inv) * scale;
-      } else {
-        g = clipped ? 0.0f : 0.5f * (1.0f - r * r * inv) * scale;
-      }
+  const int k = k0 + tx, s = k < ns ? k : k - ns;
+  const bool out = k < 2 * ns;
+  // eight rows' loads in flight at a time
+#pragma unroll
+  for (int h = 0; h < 16; h += 8) {
+    float mu8[8], lv8[8], y8[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int b = b0 + 4 * (h + i) + ty;
+      const size_t bb = b < Bn ? b : 0, ss = out ? s : 0;
+      mu8[i] = O[bb * out_pad + ss];
+      lv8[i] = O[bb * out_pad + ns + ss];
+      y8[i] = T[bb * ns + ss];
     }
-    const bf16 gb = (bf16)g;
-    dO[(size_t)b * out_pad + k] = gb;
-    tile[rr][tx] = gb;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int rr = 4 * (h + i) + ty, b = b0 + rr;
+      float g = 0.0f;
+      if (b < Bn && out) {
+        const float mu = mu8[i], lv_raw = lv8[i], y = y8[i];
+        const bool clipped = lv_raw < -12.0f || lv_raw > 12.0f;
+        const float lv = fminf(fmaxf(lv_raw, -12.0f), 12.0f);
+        const float r = y - mu;
+        const float inv = __expf(-lv);
+        if (s < n_cnt) {
+          if (k < ns) {
+            const float o = fminf(fmaxf(mu, -30.0f), 8.0f);
+            const float lam = __expf(o);
+            g = (lam - y) * scale;
+            l += ((lam - y * o) + (lam - y) * (mu - o)) * scale;
+          }
+        } else if (k < ns) {
+          g = -r * inv * scale;
+          l += 0.5f * (lv + r * r * inv) * scale;
+        } else {
+          g = clipped ? 0.0f : 0.5f * (1.0f - r * r * inv) * scale;
+        }
+      }
+      const bf16 gb = (bf16)g;
+      dO[(size_t)b * out_pad + k] = gb;
+      tile[rr][tx] = gb;
+    }
   }
   __syncthreads();
-  for (int kk = ty; kk < 64; kk += 4) dOT[(size_t)(k0 + kk) * Bpad + b0 + tx] = tile[tx][kk];
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    dOT[(size_t)(k0 + 4 * i + ty) * Bpad + b0 + tx] = tile[tx][4 * i + ty];
   red[threadIdx.x] = l;
   __syncthreads();
   for (int q = 128; q > 0; q >>= 1) {
@@ -264,25 +327,6 @@ __global__ __launch_bounds__(256) void nll_kernel(const float* __restrict__ O,
     __syncthreads();
   }
   if (threadIdx.x == 0) atomicAdd(loss, red[0]);
-}
-
-// bias gradient: row sums of dZ^T (rows x Bpad bf16), one workgroup per row:
-// 16-byte loads (8 values), then a wave reduction and one across the 4 waves
-__global__ __launch_bounds__(256) void rowsum_kernel(const bf16* __restrict__ dZT, int Bpad,
-                                                     float* __restrict__ db) {
-  const int r = blockIdx.x;
-  const bf16x8* row = reinterpret_cast<const bf16x8*>(dZT + (size_t)r * Bpad);
-  float s = 0.0f;
-  for (int v = threadIdx.x; v < Bpad / 8; v += blockDim.x) {
-    const bf16x8 x = row[v];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += (float)x[e];
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  __shared__ float red[4];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) db[r] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 struct LayerDesc {
@@ -311,13 +355,49 @@ __device__ __forceinline__ TilePos tile_pos(int blk, const LayerDesc* __restrict
   return TilePos{-1, blk * 256, 0};
 }
 
-// bias q (over all layers) as an index of the flat parameters, or -1
-__device__ __forceinline__ int64_t bias_at(int q, const LayerDesc* __restrict__ L, int nl) {
+// bias q (over all layers): its layer (-1: past the last) and its row
+struct BiasPos {
+  int layer, row;
+};
+__device__ __forceinline__ BiasPos bias_at(int q, const LayerDesc* __restrict__ L, int nl) {
   for (int l = 0; l < nl; ++l) {
-    if (q < L[l].out) return L[l].b_off + q;
+    if (q < L[l].out) return BiasPos{l, q};
     q -= L[l].out;
   }
-  return -1;
+  return BiasPos{-1, 0};
+}
+
+// The gradient as the EPI_DW launches left it: layer l's S[l] partial sums of its
+// weights (out x in each) from p[l] on, then those of its biases (out each).
+// Every reader adds them in the order 0, 1, ...
+constexpr int kMaxLayers = 17;
+struct GradParts {
+  const float* p[kMaxLayers];
+  int S[kMaxLayers];
+};
+__device__ __forceinline__ f32x4 grad_w4(const GradParts& P, int l, const LayerDesc& L, int64_t at) {
+  const float* q = P.p[l] + at;
+  const int64_t MN = (int64_t)L.out * L.in;
+  const int S = P.S[l];  // a power of two
+  f32x4 v = *reinterpret_cast<const f32x4*>(q);
+  if (S < 8) {
+    for (int s = 1; s < S; ++s) v += *reinterpret_cast<const f32x4*>(q + s * MN);
+    return v;
+  }
+  for (int s = 0; s < S; s += 8) {  // eight loads in flight
+    f32x4 x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = *reinterpret_cast<const f32x4*>(q + (s + e) * MN);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v = s + e > 0 ? v + x[e] : x[e];
+  }
+  return v;
+}
+__device__ __forceinline__ float grad_b(const GradParts& P, int l, const LayerDesc& L, int row) {
+  const float* q = P.p[l] + P.S[l] * (int64_t)L.out * L.in + row;
+  float v = q[0];
+  for (int s = 1; s < P.S[l]; ++s) v += q[(int64_t)s * L.out];
+  return v;
 }
 
 // the bf16 copies of a tile: v holds this thread's weights, v[j][e] that of
@@ -353,12 +433,17 @@ __device__ __forceinline__ void store_copies(const float (&v)[2][8], const TileP
 // Adam on the flat FP32 parameters; refreshes the bf16 copies W (out x in), W^T
 // (in x out) and W in fragment order of every weight.  Bound by memory: 8
 // weights a thread in 16- and 32-byte pieces (a weight a thread with scattered
-// copies: 12.1 us for 0.9 million weights, 9.2 now).
+// copies: 12.1 us for 0.9 million weights, 9.2 so).  It adds the gradient's
+// partial sums as it reads them, eight loads in flight: 17.5 us for 0.9 million
+// weights and 8,192 samples, where a launch per layer for the sums and one for
+// the biases took 45 us before it.  *loss goes to *loss_out if given.
 __global__ __launch_bounds__(256) void adam_kernel(
     float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-    const float* __restrict__ g, float lr, float b1, float b2, float eps, float wd, float c1,
+    GradParts P, float lr, float b1, float b2, float eps, float wd, float c1,
     float c2, const LayerDesc* __restrict__ L, int nl, const int64_t* __restrict__ bf_off,
-    bf16* __restrict__ Wb, bf16* __restrict__ WbT, bf16* __restrict__ Wf) {
+    bf16* __restrict__ Wb, bf16* __restrict__ WbT, bf16* __restrict__ Wf,
+    const float* __restrict__ loss, float* __restrict__ loss_out) {
+  if (loss_out && blockIdx.x == 0 && threadIdx.x == 0) *loss_out = *loss;
   auto step = [&](float gg, float& mp, float& vp, float ww) {
     const float mm = b1 * mp + (1.0f - b1) * gg;
     const float vv = b2 * vp + (1.0f - b2) * gg * gg;
@@ -368,8 +453,10 @@ __global__ __launch_bounds__(256) void adam_kernel(
   };
   const TilePos T = tile_pos((int)blockIdx.x, L, nl);
   if (T.layer < 0) {
-    const int64_t p = bias_at(T.o0 + (int)threadIdx.x, L, nl);
-    if (p >= 0) w[p] = step(g[p], m[p], v[p], w[p]);
+    const BiasPos b = bias_at(T.o0 + (int)threadIdx.x, L, nl);
+    if (b.layer < 0) return;
+    const int64_t p = L[b.layer].b_off + b.row;
+    w[p] = step(grad_b(P, b.layer, L[b.layer], b.row), m[p], v[p], w[p]);
     return;
   }
   const LayerDesc D = L[T.layer];
@@ -377,10 +464,10 @@ __global__ __launch_bounds__(256) void adam_kernel(
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int o = T.o0 + j * 32 + (threadIdx.x >> 3), i = T.i0 + (threadIdx.x & 7) * 8;
-    const int64_t p = D.w_off + (int64_t)o * D.in + i;
+    const int64_t at = (int64_t)o * D.in + i, p = D.w_off + at;
 #pragma unroll
     for (int h = 0; h < 8; h += 4) {
-      f32x4 gm = *reinterpret_cast<const f32x4*>(g + p + h);
+      const f32x4 gm = grad_w4(P, T.layer, D, at + h);
       f32x4 mm = *reinterpret_cast<const f32x4*>(m + p + h);
       f32x4 vv = *reinterpret_cast<const f32x4*>(v + p + h);
       f32x4 ww = *reinterpret_cast<const f32x4*>(w + p + h);
@@ -399,6 +486,25 @@ __global__ __launch_bounds__(256) void adam_kernel(
   store_copies(x, T, D, bf_off[T.layer], Wb, WbT, Wf);
 }
 
+// the gradient itself, for a caller that asks for it (launch as adam_kernel)
+__global__ __launch_bounds__(256) void grad_sum_kernel(GradParts P,
+                                                       const LayerDesc* __restrict__ L, int nl,
+                                                       float* __restrict__ g) {
+  const TilePos T = tile_pos((int)blockIdx.x, L, nl);
+  if (T.layer < 0) {
+    const BiasPos b = bias_at(T.o0 + (int)threadIdx.x, L, nl);
+    if (b.layer >= 0) g[L[b.layer].b_off + b.row] = grad_b(P, b.layer, L[b.layer], b.row);
+    return;
+  }
+  const LayerDesc D = L[T.layer];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = T.o0 + j * 16 + (threadIdx.x >> 4), i = T.i0 + (threadIdx.x & 15) * 4;
+    const int64_t at = (int64_t)o * D.in + i;
+    *reinterpret_cast<f32x4*>(g + D.w_off + at) = grad_w4(P, T.layer, D, at);
+  }
+}
+
 // the bf16 copies of every weight (launch: the weight tiles)
 __global__ __launch_bounds__(256) void refresh_bf16_kernel(
     const float* __restrict__ w, const LayerDesc* __restrict__ L, int nl,
@@ -415,11 +521,6 @@ __global__ __launch_bounds__(256) void refresh_bf16_kernel(
       x[j][e] = w[D.w_off + (int64_t)(T.o0 + j * 32 + (threadIdx.x >> 3)) * D.in + T.i0 +
                   (threadIdx.x & 7) * 8 + e];
   store_copies(x, T, D, bf_off[T.layer], Wb, WbT, Wf);
-}
-
-__global__ void zero_f32_kernel(float* __restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0f;
 }
 
 // copy the (mu, logvar) block of O (Bpad x out_pad) into y (B x 2 ns)
@@ -840,8 +941,8 @@ struct abc_mlp {
   float* O = nullptr;
   bf16 *dA = nullptr, *dAT = nullptr, *dB = nullptr, *dBT = nullptr;
   float* loss = nullptr;
-  float* splitk_ws = nullptr;  // split-K partial tiles of the weight gradients
-  size_t splitk_cap = 0;       // floats
+  float* parts = nullptr;      // partial sums of the gradient (GradParts)
+  std::vector<int64_t> part_off;  // per layer
   int64_t step = 0;
   std::string msg;
 };
@@ -859,15 +960,21 @@ int mfail(abc_mlp* p, int code, const std::string& s) {
     if (e_ != hipSuccess) return mfail(p, ABC_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// Workgroups of a gemm grid; splitting K fills the machine when M x N is small
-// (the weight gradients: M, N = layer widths, K = batch).
+// Sums that a weight gradient (M, N = layer widths, K = batch) is split into to
+// fill the machine: chunks of whole stages, the last shorter or, past the end,
+// empty (a sum of zeros).  With equal chunks only, a batch of 8,064 was split in
+// two and a step took 349 us, 209 so; 1,000 samples 139 and 109.
 int splitk_for(int M, int N, int K) {
   // counted in 64-row tiles, so the split does not depend on the tile rows
   // chosen below (results do not depend on them either)
   const int tiles = (M / 64) * (N / (N % 128 == 0 ? 128 : 64));
   int S = 1;
-  while (tiles * S < 256 && K % (2 * S * BK) == 0 && K / (2 * S) >= 4 * BK) S *= 2;
+  while (tiles * S < 256 && K / (2 * S) >= 256) S *= 2;
   return S;
+}
+int splitk_chunk(int K, int S) {
+  const int bk = stage_k(EPI_DW);
+  return (K / bk + S - 1) / S * bk;  // K, the padded batch, is a multiple of bk
 }
 
 // Workgroup tile rows: 64 when 128-row tiles would leave fewer than two
@@ -883,50 +990,48 @@ int tile_cols(int M, int N, int S, int bm) {
   return (M / bm) * (N / 128) * S < 1024 ? 64 : 128;
 }
 
-template <int EPI>
-void gemm(abc_mlp* p, const bf16* A, const bf16* B, int M, int N, int K, const float* bias,
-          float* Cf, bf16* Cb, bf16* CbT, const float* Zprev, float* Zout) {
-  int S = 1;
-  float* out = Cf;
-  if (EPI == EPI_F32 && !bias && p->splitk_ws) {
-    S = splitk_for(M, N, K);
-    if ((size_t)S * M * N > p->splitk_cap) S = 1;
-    if (S > 1) out = p->splitk_ws;
-  }
+struct Tile {
+  int bm, bn;
+};
+Tile tile_for(const abc_mlp* p, int M, int N, int S) {
   const int bm = p->tile_rows ? p->tile_rows : tile_rows(M, N, S);
   const int bn = N % 128 != 0 ? 64 : (p->tile_cols ? p->tile_cols : tile_cols(M, N, S, bm));
-  if (bn == 128 && bm == 128) {
-    hipLaunchKernelGGL((gemm_nt_kernel<128, 128, EPI>), dim3(M / 128, N / 128, S), dim3(256), 0,
-                       p->stream, A, B, M, N, K / S, K, bias, out, Cb, CbT, Zprev, Zout);
-  } else if (bn == 128) {
-    hipLaunchKernelGGL((gemm_nt_kernel<64, 128, EPI>), dim3(M / 64, N / 128, S), dim3(256), 0,
-                       p->stream, A, B, M, N, K / S, K, bias, out, Cb, CbT, Zprev, Zout);
-  } else if (bm == 128) {
-    hipLaunchKernelGGL((gemm_nt_kernel<128, 64, EPI>), dim3(M / 128, N / 64, S), dim3(256), 0,
-                       p->stream, A, B, M, N, K / S, K, bias, out, Cb, CbT, Zprev, Zout);
-  } else {
-    hipLaunchKernelGGL((gemm_nt_kernel<64, 64, EPI>), dim3(M / 64, N / 64, S), dim3(256), 0,
-                       p->stream, A, B, M, N, K / S, K, bias, out, Cb, CbT, Zprev, Zout);
-  }
-  if (S > 1)
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(g1((int64_t)M * N / 4, 256)), dim3(256), 0,
-                       p->stream, p->splitk_ws, S, (int64_t)M * N, Cf);
+  return Tile{bm, bn};
 }
 
-int forward(abc_mlp* p, int64_t Bn, const float* x_dev) {
+// the product of g (whose K is that of one of its S sums)
+template <int EPI>
+void gemm(abc_mlp* p, const GemmArgs& g, int S = 1) {
+  const Tile t = tile_for(p, g.M, g.N, S);
+  const dim3 grid = EPI == EPI_DW ? dim3(S, g.M / t.bm, g.N / t.bn) : dim3(g.M / t.bm, g.N / t.bn);
+  if (t.bn == 128 && t.bm == 128)
+    hipLaunchKernelGGL((gemm_nt_kernel<128, 128, EPI>), grid, dim3(256), 0, p->stream, g.A, g.B, g.M,
+                       g.N, g.K, g.ld, g.bias, g.Cf, g.Cb, g.CbT, g.Zprev, g.Zout);
+  else if (t.bn == 128)
+    hipLaunchKernelGGL((gemm_nt_kernel<64, 128, EPI>), grid, dim3(256), 0, p->stream, g.A, g.B, g.M,
+                       g.N, g.K, g.ld, g.bias, g.Cf, g.Cb, g.CbT, g.Zprev, g.Zout);
+  else if (t.bm == 128)
+    hipLaunchKernelGGL((gemm_nt_kernel<128, 64, EPI>), grid, dim3(256), 0, p->stream, g.A, g.B, g.M,
+                       g.N, g.K, g.ld, g.bias, g.Cf, g.Cb, g.CbT, g.Zprev, g.Zout);
+  else
+    hipLaunchKernelGGL((gemm_nt_kernel<64, 64, EPI>), grid, dim3(256), 0, p->stream, g.A, g.B, g.M,
+                       g.N, g.K, g.ld, g.bias, g.Cf, g.Cb, g.CbT, g.Zprev, g.Zout);
+}
+
+int forward(abc_mlp* p, int64_t Bn, const float* x_dev, float* loss) {
   const int Bpad = (int)((Bn + 127) / 128 * 128);
-  hipLaunchKernelGGL(cast_input_kernel, dim3(g1((int64_t)Bpad * p->in_pad, 256)), dim3(256), 0,
-                     p->stream, x_dev, (int)Bn, Bpad, p->n_in, p->in_pad, p->X, p->XT);
+  hipLaunchKernelGGL(cast_input_kernel, dim3(Bpad / 64, p->in_pad / 64), dim3(256), 0, p->stream,
+                     x_dev, (int)Bn, Bpad, p->n_in, p->in_pad, p->X, p->XT, loss);
   const bf16* in = p->X;
   for (int l = 0; l < p->depth; ++l) {
     const LayerDesc& L = p->layers[l];
-    gemm<EPI_SILU>(p, in, p->Wb + p->bf_off[l], Bpad, L.out, L.in, p->w + L.b_off, nullptr,
-                   p->H[l], p->HT[l], nullptr, p->Z[l]);
+    gemm<EPI_SILU>(p, GemmArgs{in, p->Wb + p->bf_off[l], Bpad, L.out, L.in, L.in, p->w + L.b_off,
+                               nullptr, p->H[l], p->HT[l], nullptr, p->Z[l]});
     in = p->H[l];
   }
   const LayerDesc& L = p->layers[p->depth];
-  gemm<EPI_F32>(p, in, p->Wb + p->bf_off[p->depth], Bpad, L.out, L.in, p->w + L.b_off, p->O,
-                nullptr, nullptr, nullptr, nullptr);
+  gemm<EPI_F32>(p, GemmArgs{in, p->Wb + p->bf_off[p->depth], Bpad, L.out, L.in, L.in,
+                            p->w + L.b_off, p->O, nullptr, nullptr, nullptr, nullptr});
   MCHK(p, hipGetLastError());
   return ABC_OK;
 }
@@ -970,12 +1075,11 @@ bool infer(abc_mlp* p, int64_t n, const float* x, float* y) {
   }
 }
 
-// fwd + loss + bwd into p->g; loss (mean NLL) accumulated in p->loss
-int grad(abc_mlp* p, int64_t Bn, const float* x_dev, const float* t_dev) {
-  int rc = forward(p, Bn, x_dev);
+// fwd + loss + bwd into p->parts, described by P; loss (mean NLL) in p->loss
+int grad(abc_mlp* p, int64_t Bn, const float* x_dev, const float* t_dev, GradParts& P) {
+  int rc = forward(p, Bn, x_dev, p->loss);
   if (rc) return rc;
   const int Bpad = (int)((Bn + 127) / 128 * 128);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, p->stream, p->loss, (int64_t)1);
   hipLaunchKernelGGL(nll_kernel, dim3(Bpad / 64, p->out_pad / 64), dim3(256), 0, p->stream,
                      p->O, t_dev, (int)Bn, Bpad, p->ns, p->n_cnt, p->out_pad, p->dA, p->dAT,
                      p->loss);
@@ -984,15 +1088,21 @@ int grad(abc_mlp* p, int64_t Bn, const float* x_dev, const float* t_dev) {
   for (int l = p->depth; l >= 0; --l) {
     const LayerDesc& L = p->layers[l];
     const bf16* Hin_T = l == 0 ? p->XT : p->HT[l - 1];
-    // dW_l = dZ_l^T H_{l-1}: (out x Bpad) . (in x Bpad)^T
-    gemm<EPI_F32>(p, curT, Hin_T, L.out, L.in, Bpad, nullptr, p->g + L.w_off, nullptr, nullptr,
-                  nullptr, nullptr);
-    hipLaunchKernelGGL(rowsum_kernel, dim3(L.out), dim3(256), 0, p->stream, curT, Bpad,
-                       p->g + L.b_off);
+    // dW_l = dZ_l^T H_{l-1}: (out x Bpad) . (in x Bpad)^T, and db_l
+    const int64_t MN = (int64_t)L.out * L.in;
+    int S = splitk_for(L.out, L.in, Bpad);
+    // one sum is the gradient itself, which lies in the same order
+    float* part = S > 1 ? p->parts + p->part_off[l] : p->g + L.w_off;
+    P.S[l] = S;
+    P.p[l] = part;
+    const GemmArgs w{curT, Hin_T, L.out, L.in, splitk_chunk(Bpad, S), Bpad,
+                     nullptr, part, nullptr, nullptr,
+                     nullptr, part + S * MN};
+    gemm<EPI_DW>(p, w, S);
     if (l > 0) {
       // dZ_{l-1} = (dZ_l W_l) * silu'(Z_{l-1}); W_l^T copy is (in x out)
-      gemm<EPI_DSILU>(p, cur, p->WbT + p->bf_off[l], Bpad, L.in, L.out, nullptr, nullptr, nxt,
-                      nxtT, p->Z[l - 1], nullptr);
+      gemm<EPI_DSILU>(p, GemmArgs{cur, p->WbT + p->bf_off[l], Bpad, L.in, L.out, L.out, nullptr,
+                                  nullptr, nxt, nxtT, p->Z[l - 1], nullptr});
       std::swap(cur, nxt);
       std::swap(curT, nxtT);
     }
@@ -1067,9 +1177,15 @@ int32_t abc_mlp_create(abc_mlp** out, int32_t device, int32_t n_in, int32_t widt
   A(&p->dA, 2 * Bp * dmax); A(&p->dAT, 2 * Bp * dmax);
   A(&p->dB, 2 * Bp * dmax); A(&p->dBT, 2 * Bp * dmax);
   A(&p->loss, 64);
-  // split-K partials: at most 256 tiles of 128 x 128 floats in flight
-  p->splitk_cap = (size_t)256 * 128 * 128;
-  A(&p->splitk_ws, 4 * p->splitk_cap);
+  // partial sums of the gradients: as many as any batch up to max_batch splits into
+  int64_t n_part = 0;
+  for (const LayerDesc& L : p->layers) {
+    int S = 1;
+    for (int64_t K = 128; K <= Bp; K += 128) S = std::max(S, splitk_for(L.out, L.in, (int)K));
+    p->part_off.push_back(n_part);
+    if (S > 1) n_part += (int64_t)S * (L.out * (int64_t)L.in + L.out);
+  }
+  A(&p->parts, 4 * std::max<int64_t>(n_part, 4));
   if (!ok) { abc_mlp_destroy(p); return ABC_E_OOM; }
   std::vector<float> zeros(off, 0.0f);
   if (hipMemcpy(p->w, w0.data(), 4 * off, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1095,7 +1211,7 @@ int32_t abc_mlp_destroy(abc_mlp* p) {
   if (!p) return ABC_OK;
   if (p->stream) hipStreamSynchronize(p->stream);
   void* bufs[] = {p->w, p->m, p->v, p->g, p->Wb, p->WbT, p->Wf, p->d_layers, p->d_bf_off, p->X, p->XT,
-                  p->O, p->dA, p->dAT, p->dB, p->dBT, p->loss, p->splitk_ws};
+                  p->O, p->dA, p->dAT, p->dB, p->dBT, p->loss, p->parts};
   for (void* b : bufs)
     if (b) hipFree(b);
   for (auto* z : p->Z) if (z) hipFree(z);
@@ -1167,7 +1283,7 @@ int32_t abc_mlp_forward_dev(abc_mlp* p, int64_t n, const float* x_dev, float* y_
   }
   for (int64_t o = 0; o < n; o += p->max_batch) {
     const int64_t b = std::min<int64_t>(p->max_batch, n - o);
-    int rc = forward(p, b, x_dev + o * p->n_in);
+    int rc = forward(p, b, x_dev + o * p->n_in, nullptr);
     if (rc) return rc;
     hipLaunchKernelGGL(gather_out_kernel, dim3(g1(b * p->n_out, 256)), dim3(256), 0, p->stream,
                        p->O, (int)b, p->ns, p->out_pad, y_dev + o * p->n_out);
@@ -1179,8 +1295,11 @@ int32_t abc_mlp_forward_dev(abc_mlp* p, int64_t n, const float* x_dev, float* y_
 int32_t abc_mlp_grad_dev(abc_mlp* p, int64_t n, const float* x_dev, const float* t_dev,
                          float* grad_host, float* loss_host) {
   if (!p || n < 1 || n > p->max_batch || !x_dev || !t_dev) return ABC_E_ARG;
-  int rc = grad(p, n, x_dev, t_dev);
+  GradParts P;
+  int rc = grad(p, n, x_dev, t_dev, P);
   if (rc) return rc;
+  hipLaunchKernelGGL(grad_sum_kernel, dim3(p->w_tiles + g1(p->n_bias, 256)), dim3(256), 0,
+                     p->stream, P, p->d_layers, (int)p->layers.size(), p->g);
   MCHK(p, hipStreamSynchronize(p->stream));
   if (grad_host) MCHK(p, hipMemcpy(grad_host, p->g, 4 * p->n_par, hipMemcpyDeviceToHost));
   if (loss_host) MCHK(p, hipMemcpy(loss_host, p->loss, 4, hipMemcpyDeviceToHost));
@@ -1191,16 +1310,16 @@ int32_t abc_mlp_train_step_dev(abc_mlp* p, int64_t n, const float* x_dev, const 
                                float lr, float beta1, float beta2, float eps, float weight_decay,
                                float* loss_dev_or_null) {
   if (!p || n < 1 || n > p->max_batch || !x_dev || !t_dev) return ABC_E_ARG;
-  int rc = grad(p, n, x_dev, t_dev);
+  GradParts P;
+  int rc = grad(p, n, x_dev, t_dev, P);
   if (rc) return rc;
   p->step++;
   const float c1 = 1.0f - std::pow(beta1, (float)p->step);
   const float c2 = 1.0f - std::pow(beta2, (float)p->step);
   hipLaunchKernelGGL(adam_kernel, dim3(p->w_tiles + g1(p->n_bias, 256)), dim3(256), 0, p->stream,
-                     p->w, p->m, p->v, p->g, lr, beta1, beta2, eps, weight_decay, c1, c2,
-                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf);
-  if (loss_dev_or_null)
-    MCHK(p, hipMemcpyAsync(loss_dev_or_null, p->loss, 4, hipMemcpyDeviceToDevice, p->stream));
+                     p->w, p->m, p->v, P, lr, beta1, beta2, eps, weight_decay, c1, c2,
+                     p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf,
+                     p->loss, loss_dev_or_null);
   MCHK(p, hipGetLastError());
   return ABC_OK;
 }
