@@ -168,6 +168,38 @@ ABC_DEV double fma2(double a, double b, double c) { return fma(a, b, c); }
 // in registers and each step is one instruction
 ABC_DEV double ex_core(double x) { return ex_core_with<fma3>(x); }
 
+// ex_core of two arguments, step by step side by side and without a branch:
+// alone, each step waits for the one before it
+ABC_DEV void ex_core2(double x, double y, double& ex, double& ey) {
+  const double kx = floor(x * 0x1.71547652b82fep+0 + 0.5);
+  const double ky = floor(y * 0x1.71547652b82fep+0 + 0.5);
+  const double r = (x - kx * 0x1.62e42fee00000p-1) - kx * 0x1.a39ef35793c76p-33;
+  const double s = (y - ky * 0x1.62e42fee00000p-1) - ky * 0x1.a39ef35793c76p-33;
+  double p = 0x1.6124613a86d09p-33, q = p;
+#define ABC_EX2(c)     \
+  p = fma3(p, r, c); \
+  q = fma3(q, s, c);
+  ABC_EX2(0x1.1eed8eff8d898p-29)
+  ABC_EX2(0x1.ae64567f544e4p-26)
+  ABC_EX2(0x1.27e4fb7789f5cp-22)
+  ABC_EX2(0x1.71de3a556c734p-19)
+  ABC_EX2(0x1.a01a01a01a01ap-16)
+  ABC_EX2(0x1.a01a01a01a01ap-13)
+  ABC_EX2(0x1.6c16c16c16c17p-10)
+  ABC_EX2(0x1.1111111111111p-7)
+  ABC_EX2(0x1.5555555555555p-5)
+  ABC_EX2(0x1.5555555555555p-3)
+#undef ABC_EX2
+  p = fma(p, r, 0.5);
+  q = fma(q, s, 0.5);
+  p = fma(p, r, 1.0);
+  q = fma(q, s, 1.0);
+  p = fma(p, r, 1.0);
+  q = fma(q, s, 1.0);
+  ex = x < -745.2 ? 0.0 : ldexp(p, (int)kx);
+  ey = y < -745.2 ? 0.0 : ldexp(q, (int)ky);
+}
+
 ABC_DEV double ex(double x) {
   if (x != x) return x;
   if (x > 709.78) return __longlong_as_double(0x7ff0000000000000ll);

@@ -394,7 +394,8 @@ __device__ __forceinline__ void burn_accum(double& lu, double& lt, bool g, doubl
                                            double ku, double iku, double kt, double ikt, double D) {
   if (!(D > 0.0)) return;
   // arguments <= 0 (D > 0, rates > 0): no NaN or overflow test
-  const double eu = ex_core(-(ku * D)), et = ex_core(-(kt * D));
+  double eu, et;
+  ex_core2(-(ku * D), -(kt * D), eu, et);
   lu = lu * eu;
   lt = lt * et;
   if (g) {
@@ -529,7 +530,12 @@ __device__ __forceinline__ CellSetup cell_setup(const DesignDev* __restrict__ D,
 // first): the gene path from the start of the burn-in to the labelling window
 // start ws, carrying the Poisson means of the cell's observed unspliced (lu)
 // and all (lt) molecules; the cell's state at ws goes to rec[p * C + c].
-__global__ __launch_bounds__(SSA_WG) void burn_kernel(const DesignDev* __restrict__ D,
+// A small launch ends with its longest cell's chain of steps, so the step's two
+// exponentials run side by side: 16 particles of 550 cells 7.9 -> 7.1 ms (the
+// next waiting time drawn one step ahead as well: 6.8, but 42 ms for 38 in a
+// launch of 5 x 1,024 particles of 2,500 cells, which VALU issue bounds; fewer
+// lanes per wave: 8 to 15 ms).  Five waves per SIMD: 37.9 ms there, four 38.9.
+__global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(5))) void burn_kernel(const DesignDev* __restrict__ D,
                                                       const PRates* __restrict__ R,
                                                       const int32_t* __restrict__ order, int64_t n,
                                                       uint32_t first, uint32_t k0, uint32_t k1,
