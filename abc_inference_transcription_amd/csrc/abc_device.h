@@ -200,6 +200,13 @@ ABC_DEV void ex_core2(double x, double y, double& ex, double& ey) {
   ey = y < -745.2 ? 0.0 : ldexp(q, (int)ky);
 }
 
+// x > m ? x : m in one instruction, m not NaN (a NaN x leaves m)
+ABC_DEV double max_num(double x, double m) {
+  double d;
+  asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(x), "v"(m));
+  return d;
+}
+
 ABC_DEV double ex(double x) {
   if (x != x) return x;
   if (x > 709.78) return __longlong_as_double(0x7ff0000000000000ll);

@@ -162,6 +162,14 @@ ABC_DEV void eval(const Piece& pc, const Particle& P, const Cycle& cycle, double
   rhs(p, pc.lam, y, dy);
 }
 
+// the step's change for the scaled error err.  One evaluation for accepted and
+// rejected steps: lanes of a wave do both kinds.
+ABC_DEV double step_factor(double err, const LogEntry* ltab) {
+  const double f = 0.9 * ex_core(-0.2 * ln(err, ltab));
+  if (err <= 1.0) return err == 0.0 || f > 5.0 ? 5.0 : f;
+  return f < 0.2 ? 0.2 : f;
+}
+
 // Adaptive Dormand-Prince 5(4) over one smooth piece [a, b]; returns the
 // attempted steps.
 ABC_DEV int64_t dopri_piece(const Piece& pc, const Particle& P, const MomCfgDev& cfg, double a,
@@ -205,7 +213,7 @@ ABC_DEV int64_t dopri_piece(const Piece& pc, const Particle& P, const MomCfgDev&
           h * (kE1 * k1[i] + kE3 * k3[i] + kE4 * k4[i] + kE5 * k5[i] + kE6 * k6[i] + kE7 * k7[i]);
       const double sc = atol + rtol * fmax(fabs(y[i]), fabs(yn[i]));
       const double r = fabs(ei) / sc;
-      if (r > err) err = r;
+      err = max_num(r, err);
     }
     steps++;
     if (err <= 1.0) {
@@ -215,14 +223,8 @@ ABC_DEV int64_t dopri_piece(const Piece& pc, const Particle& P, const MomCfgDev&
         y[i] = yn[i];
         k1[i] = k7[i];
       }
-      double fac = err == 0.0 ? 5.0 : 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac > 5.0) fac = 5.0;
-      h *= fac;
-    } else {
-      double fac = 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac < 0.2) fac = 0.2;
-      h *= fac;
     }
+    h *= step_factor(err, ltab);
     if (h < 1e-14 * (fabs(t) + 1.0)) h = 1e-14 * (fabs(t) + 1.0);
   }
   return steps;
@@ -302,8 +304,8 @@ ABC_DEV void gb_setup(GBlock& q, const double* p, double al1, double lam, const 
 
 // the gene block at a + s into y[0], y[3], y[4], y[5]
 ABC_DEV void gb_eval(const GBlock& q, double s, double* y) {
-  const double e1 = ex_core(-(q.K * s));
-  const double eg = ex_core(-(q.gam * s));
+  double e1, eg;
+  ex_core2(-(q.K * s), -(q.gam * s), e1, eg);
   const double e2 = e1 * e1;
   const double en = e1 * eg;
   double E10, E20, E1K, E2K, E12, E22;
@@ -397,7 +399,7 @@ ABC_DEV int64_t egb_piece(const Piece& pc, const Particle& P, const MomCfgDev& c
           h * (kE1 * k1[i] + kE3 * k3[i] + kE4 * k4[i] + kE5 * k5[i] + kE6 * k6[i] + kE7 * k7[i]);
       const double sc = atol + rtol * fmax(fabs(y[i]), fabs(yn[i]));
       const double r = fabs(ei) / sc;
-      if (r > err) err = r;
+      err = max_num(r, err);
     }
     steps++;
     if (err <= 1.0) {
@@ -407,14 +409,8 @@ ABC_DEV int64_t egb_piece(const Piece& pc, const Particle& P, const MomCfgDev& c
         y[i] = yn[i];
         k1[i] = k7[i];
       }
-      double fac = err == 0.0 ? 5.0 : 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac > 5.0) fac = 5.0;
-      h *= fac;
-    } else {
-      double fac = 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac < 0.2) fac = 0.2;
-      h *= fac;
     }
+    h *= step_factor(err, ltab);
     if (h < 1e-14 * (fabs(t) + 1.0)) h = 1e-14 * (fabs(t) + 1.0);
   }
   return steps;
@@ -493,11 +489,29 @@ ABC_DEV void periodic_boundary(const double* e, double* v) {
 // lane r < 5 does it for stage r + 2.  Lane 0 then carries E u and Var u, lane 1
 // E l and Var l, lane 2 Cov ul; every lane takes the same step decisions.  Each
 // value is formed by the operations of egb_piece in the same order, so the
-// results and the steps are the same bits.  About 600 instructions and 4,600
-// cycles a step against 2,000 and 13,700 by one lane; 503 particles of model 3
-// (27,665 trajectories, the machine mostly idle): 96 -> 36 ms, 4,096 of model 4:
-// 72 -> 43 ms.
+// results and the steps are the same bits.  About 600 instructions a step
+// against 2,000 by one lane; 503 particles of model 3 (27,665 trajectories, the
+// machine mostly idle): 96 -> 36 ms, 4,096 of model 4: 72 -> 43 ms; 33 and 41 ms
+// with each step's chain shortened: its exponentials in pairs (gb_eval), one
+// step factor for accepted and rejected steps, maxima in one instruction and,
+// over the team, without the LDS unit.
 constexpr int kTeam = 8, kTeams = 64 / kTeam;
+
+// the largest of the team's eight values (none NaN), in every lane: neighbours,
+// then pairs, by lane permutations within a quad, then the other quad's by the
+// mirror of eight lanes: no step waits for the LDS unit, as __shfl_xor's do
+template <int CTRL>
+ABC_DEV double dpp64(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp((int)__double2loint(x), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)__double2hiint(x), CTRL, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+ABC_DEV double team_max(double x) {
+  static_assert(kTeam == 8, "row_half_mirror");
+  x = max_num(dpp64<0xB1>(x), x);   // quad_perm 1, 0, 3, 2
+  x = max_num(dpp64<0x4E>(x), x);   // quad_perm 2, 3, 0, 1
+  return max_num(dpp64<0x141>(x), x);  // row_half_mirror
+}
 
 // what a stage time contributes to the five right-hand sides
 struct Forcing {
@@ -614,13 +628,7 @@ ABC_DEV int64_t egb_piece_team(const Piece& pc, const Particle& P, const MomCfgD
                              kE7 * kv[7]);
       const double rm = fabs(em) / (atol + rtol * fmax(fabs(m), fabs(nm)));
       const double rv = fabs(ev) / (atol + rtol * fmax(fabs(v), fabs(nv)));
-      if (rm > err) err = rm;
-      if (rv > err) err = rv;
-#pragma unroll
-      for (int o = 1; o < kTeam; o <<= 1) {
-        const double x = __shfl_xor(err, o);
-        if (x > err) err = x;
-      }
+      err = team_max(max_num(rv, max_num(rm, err)));
     }
     steps++;
     if (err <= 1.0) {
@@ -633,14 +641,8 @@ ABC_DEV int64_t egb_piece_team(const Piece& pc, const Particle& P, const MomCfgD
       S.g[3] = ys[3];
       S.g[4] = ys[4];
       S.g[5] = ys[5];
-      double fac = err == 0.0 ? 5.0 : 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac > 5.0) fac = 5.0;
-      h *= fac;
-    } else {
-      double fac = 0.9 * ex_core(-0.2 * ln(err, ltab));
-      if (fac < 0.2) fac = 0.2;
-      h *= fac;
     }
+    h *= step_factor(err, ltab);
     if (h < 1e-14 * (fabs(t) + 1.0)) h = 1e-14 * (fabs(t) + 1.0);
   }
   S.m = m;
