@@ -570,7 +570,7 @@ def reference_shape_leg(stream, a):
            "genes_with_acceptance": int((counts > 0).sum()), "fp64_rescorings": nres,
            "ms_per_step": round(wall / a.ref_steps * 1e3, 3),
            "timing": "host clock around the session (simulation, screening, FP64 rescoring, "
-                     "per-batch merge, sorted lists on the host)"}
+                     "sorting and packing of the lists)"}
     print(f"[bench] reference shape: {res['value']:.1f} particles/s, "
           f"{res['accepted_pairs']} accepted pairs", file=sys.stderr, flush=True)
     return res
