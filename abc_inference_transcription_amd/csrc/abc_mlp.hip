@@ -69,9 +69,11 @@ struct GemmArgs {
 // weight gradient and its bias's in one launch.  K advances in stages of BK
 // through two LDS buffers: while the MFMAs read one stage, the next is loaded
 // from global memory into registers and stored to the other buffer, one barrier
-// per stage (two or four stages in flight, or padded rows, measured the same:
-// the LDS is busy for 70 % of a workgroup's life).  Every output sums its K in
-// order, 32 at a time, whatever the tile.
+// per stage.  8,192 x 512 x 512 with the SiLU epilogue: 13.6 us, 8 of them its
+// 34 MB of stores (K = 64 takes as long), then 0.8 us per stage; two or four
+// stages in flight, padded rows, or B from the L2 in fragment order measured
+// within 0.3 us or slower.  Every output sums its K in order, 32 at a time,
+// whatever the tile.
 template <int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A,
                                                       const bf16* __restrict__ B, int M, int N,
