@@ -223,17 +223,14 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
 
 // x (B x n_in FP32, row-major) -> X (B x in_pad bf16) and X^T (in_pad x B), one
 // workgroup per 64 x 64 tile, the transpose through LDS (element by element,
-// its scattered 2-byte stores took 7.0 us for 8,192 x 64, 4.2 so).  *loss, if
-// given, starts at 0.
+// its scattered 2-byte stores took 7.0 us for 8,192 x 64, 4.2 so).
 __global__ __launch_bounds__(256) void cast_input_kernel(const float* __restrict__ x, int Bn,
                                                          int Bpad, int n_in, int in_pad,
                                                          bf16* __restrict__ X,
-                                                         bf16* __restrict__ XT,
-                                                         float* __restrict__ loss) {
+                                                         bf16* __restrict__ XT) {
   __shared__ bf16 tile[64][64 + 2];
   const int b0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  if (loss && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *loss = 0.0f;
   const int k = k0 + tx;
   float v[16];
 #pragma unroll
@@ -254,6 +251,26 @@ __global__ __launch_bounds__(256) void cast_input_kernel(const float* __restrict
     XT[(size_t)(k0 + 4 * i + ty) * Bpad + b0 + tx] = tile[tx][4 * i + ty];
 }
 
+// the sum of 256 threads' values, in thread 0
+__device__ __forceinline__ float block_sum(float x, float* red) {
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// The loss from nll_kernel's n tiles, by one workgroup: *loss, and *out if given.
+__device__ __forceinline__ void loss_total(const float* __restrict__ parts, int n,
+                                           float* __restrict__ loss, float* __restrict__ out) {
+  __shared__ float red[4];
+  float x = 0.0f;
+  for (int i = threadIdx.x; i < n; i += 256) x += parts[i];
+  x = block_sum(x, red);
+  if (threadIdx.x != 0) return;
+  *loss = x;
+  if (out) *out = x;
+}
+
 // Gaussian negative log-likelihood per element, mean over B*ns.
 // O row: [mu (ns) | logvar (ns) | pad]; dO and dO^T in bf16.  The first n_cnt
 // statistics are counts: their mu slot is a log-rate o with the Poisson
@@ -263,14 +280,16 @@ __global__ __launch_bounds__(256) void cast_input_kernel(const float* __restrict
 // logvar slot is unused.
 // One workgroup per 64 x 64 tile of (sample b, output k): the gradient is
 // written row-major to dO with k fastest, and through an LDS transpose to dO^T
-// with b fastest, so both stores are coalesced; one loss atomic per tile.
+// with b fastest, so both stores are coalesced.  The tile's share of the loss
+// goes to loss[tile], summed by loss_total (with one float atomic per tile, 512 at
+// one address, 8,192 samples of 180 outputs took 12.1 us, 7.0 so).
 __global__ __launch_bounds__(256) void nll_kernel(const float* __restrict__ O,
                                                   const float* __restrict__ T, int Bn, int Bpad,
                                                   int ns, int n_cnt, int out_pad,
                                                   bf16* __restrict__ dO, bf16* __restrict__ dOT,
                                                   float* __restrict__ loss) {
   __shared__ bf16 tile[64][64 + 2];
-  __shared__ float red[256];
+  __shared__ float red[4];
   const int b0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 columns x 4 rows per pass
   const float scale = 1.0f / ((float)Bn * (float)ns);
@@ -322,13 +341,8 @@ __global__ __launch_bounds__(256) void nll_kernel(const float* __restrict__ O,
 #pragma unroll
   for (int i = 0; i < 16; ++i)
     dOT[(size_t)(k0 + 4 * i + ty) * Bpad + b0 + tx] = tile[tx][4 * i + ty];
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int q = 128; q > 0; q >>= 1) {
-    if ((int)threadIdx.x < q) red[threadIdx.x] += red[threadIdx.x + q];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicAdd(loss, red[0]);
+  l = block_sum(l, red);
+  if (threadIdx.x == 0) loss[blockIdx.y * gridDim.x + blockIdx.x] = l;
 }
 
 struct LayerDesc {
@@ -438,14 +452,15 @@ __device__ __forceinline__ void store_copies(const float (&v)[2][8], const TileP
 // copies: 12.1 us for 0.9 million weights, 9.2 so).  It adds the gradient's
 // partial sums as it reads them, eight loads in flight: 17.5 us for 0.9 million
 // weights and 8,192 samples, where a launch per layer for the sums and one for
-// the biases took 45 us before it.  *loss goes to *loss_out if given.
+// the biases took 45 us before it.  The last workgroup sums the loss.
 __global__ __launch_bounds__(256) void adam_kernel(
     float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
     GradParts P, float lr, float b1, float b2, float eps, float wd, float c1,
     float c2, const LayerDesc* __restrict__ L, int nl, const int64_t* __restrict__ bf_off,
     bf16* __restrict__ Wb, bf16* __restrict__ WbT, bf16* __restrict__ Wf,
-    const float* __restrict__ loss, float* __restrict__ loss_out) {
-  if (loss_out && blockIdx.x == 0 && threadIdx.x == 0) *loss_out = *loss;
+    const float* __restrict__ loss_parts, int n_loss, float* __restrict__ loss,
+    float* __restrict__ loss_out) {
+  if (blockIdx.x == gridDim.x - 1) loss_total(loss_parts, n_loss, loss, loss_out);
   auto step = [&](float gg, float& mp, float& vp, float ww) {
     const float mm = b1 * mp + (1.0f - b1) * gg;
     const float vv = b2 * vp + (1.0f - b2) * gg * gg;
@@ -491,7 +506,10 @@ __global__ __launch_bounds__(256) void adam_kernel(
 // the gradient itself, for a caller that asks for it (launch as adam_kernel)
 __global__ __launch_bounds__(256) void grad_sum_kernel(GradParts P,
                                                        const LayerDesc* __restrict__ L, int nl,
-                                                       float* __restrict__ g) {
+                                                       float* __restrict__ g,
+                                                       const float* __restrict__ loss_parts,
+                                                       int n_loss, float* __restrict__ loss) {
+  if (blockIdx.x == gridDim.x - 1) loss_total(loss_parts, n_loss, loss, nullptr);
   const TilePos T = tile_pos((int)blockIdx.x, L, nl);
   if (T.layer < 0) {
     const BiasPos b = bias_at(T.o0 + (int)threadIdx.x, L, nl);
@@ -942,7 +960,7 @@ struct abc_mlp {
   std::vector<bf16*> H, HT;
   float* O = nullptr;
   bf16 *dA = nullptr, *dAT = nullptr, *dB = nullptr, *dBT = nullptr;
-  float* loss = nullptr;
+  float *loss = nullptr, *loss_parts = nullptr;  // loss_parts: one per tile of nll_kernel
   float* parts = nullptr;      // partial sums of the gradient (GradParts)
   std::vector<int64_t> part_off;  // per layer
   int64_t step = 0;
@@ -1020,10 +1038,10 @@ void gemm(abc_mlp* p, const GemmArgs& g, int S = 1) {
                        g.N, g.K, g.ld, g.bias, g.Cf, g.Cb, g.CbT, g.Zprev, g.Zout);
 }
 
-int forward(abc_mlp* p, int64_t Bn, const float* x_dev, float* loss) {
+int forward(abc_mlp* p, int64_t Bn, const float* x_dev) {
   const int Bpad = (int)((Bn + 127) / 128 * 128);
   hipLaunchKernelGGL(cast_input_kernel, dim3(Bpad / 64, p->in_pad / 64), dim3(256), 0, p->stream,
-                     x_dev, (int)Bn, Bpad, p->n_in, p->in_pad, p->X, p->XT, loss);
+                     x_dev, (int)Bn, Bpad, p->n_in, p->in_pad, p->X, p->XT);
   const bf16* in = p->X;
   for (int l = 0; l < p->depth; ++l) {
     const LayerDesc& L = p->layers[l];
@@ -1077,14 +1095,20 @@ bool infer(abc_mlp* p, int64_t n, const float* x, float* y) {
   }
 }
 
-// fwd + loss + bwd into p->parts, described by P; loss (mean NLL) in p->loss
+// nll_kernel's workgroups for a batch of Bn
+int loss_tiles(const abc_mlp* p, int64_t Bn) {
+  return (int)((Bn + 127) / 128 * 128 / 64) * (p->out_pad / 64);
+}
+
+// fwd + loss + bwd into p->parts, described by P; shares of the loss (mean NLL)
+// in p->loss_parts
 int grad(abc_mlp* p, int64_t Bn, const float* x_dev, const float* t_dev, GradParts& P) {
-  int rc = forward(p, Bn, x_dev, p->loss);
+  int rc = forward(p, Bn, x_dev);
   if (rc) return rc;
   const int Bpad = (int)((Bn + 127) / 128 * 128);
   hipLaunchKernelGGL(nll_kernel, dim3(Bpad / 64, p->out_pad / 64), dim3(256), 0, p->stream,
                      p->O, t_dev, (int)Bn, Bpad, p->ns, p->n_cnt, p->out_pad, p->dA, p->dAT,
-                     p->loss);
+                     p->loss_parts);
   // dA / dAT hold dZ of the current layer (output layer first)
   bf16 *cur = p->dA, *curT = p->dAT, *nxt = p->dB, *nxtT = p->dBT;
   for (int l = p->depth; l >= 0; --l) {
@@ -1178,7 +1202,7 @@ int32_t abc_mlp_create(abc_mlp** out, int32_t device, int32_t n_in, int32_t widt
   A(&p->O, 4 * Bp * p->out_pad);
   A(&p->dA, 2 * Bp * dmax); A(&p->dAT, 2 * Bp * dmax);
   A(&p->dB, 2 * Bp * dmax); A(&p->dBT, 2 * Bp * dmax);
-  A(&p->loss, 64);
+  A(&p->loss, 64); A(&p->loss_parts, 4 * (Bp / 64) * (p->out_pad / 64));
   // partial sums of the gradients: as many as any batch up to max_batch splits into
   int64_t n_part = 0;
   for (const LayerDesc& L : p->layers) {
@@ -1213,7 +1237,7 @@ int32_t abc_mlp_destroy(abc_mlp* p) {
   if (!p) return ABC_OK;
   if (p->stream) hipStreamSynchronize(p->stream);
   void* bufs[] = {p->w, p->m, p->v, p->g, p->Wb, p->WbT, p->Wf, p->d_layers, p->d_bf_off, p->X, p->XT,
-                  p->O, p->dA, p->dAT, p->dB, p->dBT, p->loss, p->parts};
+                  p->O, p->dA, p->dAT, p->dB, p->dBT, p->loss, p->loss_parts, p->parts};
   for (void* b : bufs)
     if (b) hipFree(b);
   for (auto* z : p->Z) if (z) hipFree(z);
@@ -1285,7 +1309,7 @@ int32_t abc_mlp_forward_dev(abc_mlp* p, int64_t n, const float* x_dev, float* y_
   }
   for (int64_t o = 0; o < n; o += p->max_batch) {
     const int64_t b = std::min<int64_t>(p->max_batch, n - o);
-    int rc = forward(p, b, x_dev + o * p->n_in, nullptr);
+    int rc = forward(p, b, x_dev + o * p->n_in);
     if (rc) return rc;
     hipLaunchKernelGGL(gather_out_kernel, dim3(g1(b * p->n_out, 256)), dim3(256), 0, p->stream,
                        p->O, (int)b, p->ns, p->out_pad, y_dev + o * p->n_out);
@@ -1301,7 +1325,8 @@ int32_t abc_mlp_grad_dev(abc_mlp* p, int64_t n, const float* x_dev, const float*
   int rc = grad(p, n, x_dev, t_dev, P);
   if (rc) return rc;
   hipLaunchKernelGGL(grad_sum_kernel, dim3(p->w_tiles + g1(p->n_bias, 256)), dim3(256), 0,
-                     p->stream, P, p->d_layers, (int)p->layers.size(), p->g);
+                     p->stream, P, p->d_layers, (int)p->layers.size(), p->g, p->loss_parts,
+                     loss_tiles(p, n), p->loss);
   MCHK(p, hipStreamSynchronize(p->stream));
   if (grad_host) MCHK(p, hipMemcpy(grad_host, p->g, 4 * p->n_par, hipMemcpyDeviceToHost));
   if (loss_host) MCHK(p, hipMemcpy(loss_host, p->loss, 4, hipMemcpyDeviceToHost));
@@ -1321,7 +1346,7 @@ int32_t abc_mlp_train_step_dev(abc_mlp* p, int64_t n, const float* x_dev, const 
   hipLaunchKernelGGL(adam_kernel, dim3(p->w_tiles + g1(p->n_bias, 256)), dim3(256), 0, p->stream,
                      p->w, p->m, p->v, P, lr, beta1, beta2, eps, weight_decay, c1, c2,
                      p->d_layers, (int)p->layers.size(), p->d_bf_off, p->Wb, p->WbT, p->Wf,
-                     p->loss, loss_dev_or_null);
+                     p->loss_parts, loss_tiles(p, n), p->loss, loss_dev_or_null);
   MCHK(p, hipGetLastError());
   return ABC_OK;
 }
