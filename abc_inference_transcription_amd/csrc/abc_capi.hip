@@ -466,11 +466,16 @@ int make_spec(abc_ctx* c, int K, const int32_t* parts, int n_parts, double clamp
   return ABC_OK;
 }
 
-// Error matrix of n particles x G genes.  64-particle tiles from one workgroup
-// per CU up, 16-particle tiles while those fill most CUs, one lane per pair
-// below that, where a tile's chain over the statistics sets the time (53
-// statistics, us: 1,000 x 1,000 pairs 40 / 41 / 64, 700 x 620 37 / 29 / 38,
-// 300 x 300 35 / 24 / 24, 100 x 500 35 / 24 / 20).
+// Error matrix of n particles x G genes: one lane per pair, or tiles of 64 genes
+// x 64 or 16 particles a workgroup, whose lanes past the last gene are idle and
+// whose chain over the statistics is the longer.  Times in units of one wave of
+// the pair kernel (3.5 ns at 53 statistics; all three scale with their number):
+// waves + 2,900, at least 5,100; 17.5 per workgroup of 64 particles + 5,700, at
+// least 9,700; 6.8 per workgroup of 16 + 4,600, at least 6,570.  The smallest of
+// the three is taken.  Measured with 53 statistics, us, pair / 64 / 16, n x G:
+// 1,000,000 x 1 101 / 1,030 / -, 300,000 x 8 166 / 289 / 430, x 16 311 / 288 / 433,
+// x 64 1,125 / 308 / 444; 16,000 x 24 30 / 35 / 36, x 32 39 / 36 / 37; 4,000 x 48
+// 23 / 34 / 24, x 64 26 / 35 / 24; 1,000 x 200 25 / 35 / 24, x 1,000 61 / 38 / 40.
 void launch_errors(abc_ctx* c, int64_t n, const double* stats, int64_t G, const double* data,
                    const double* se, const ErrSpec& E, double* err) {
   const int64_t gt = (G + 63) / 64;
@@ -480,8 +485,12 @@ void launch_errors(abc_ctx* c, int64_t n, const double* stats, int64_t G, const 
                        (PoolEntry*)nullptr, (int64_t)0, (int64_t)0, (const int64_t*)nullptr,
                        (const uint32_t*)nullptr);
   };
-  if (n >= 16 && gt <= 65535 && (n + 63) / 64 * gt >= c->num_cu) return tile(err_tile_kernel<16, false>, 16);
-  if (n >= 4 && gt <= 65535 && (n + 15) / 16 * gt >= 200) return tile(err_tile_kernel<4, false>, 4);
+  const double pair = std::max(5100.0, (double)((n + 63) / 64) * (double)G + 2900.0);
+  const double t16 = std::max(9700.0, 17.5 * (double)((n + 63) / 64) * (double)gt + 5700.0);
+  const double t4 = std::max(6570.0, 6.8 * (double)((n + 15) / 16) * (double)gt + 4600.0);
+  if (gt <= 65535 && n >= 16 && t16 < std::min(pair, t4))
+    return tile(err_tile_kernel<16, false>, 16);
+  if (gt <= 65535 && n >= 4 && t4 < pair) return tile(err_tile_kernel<4, false>, 4);
   // grid.y is limited to 65535: split genes into slices
   for (int64_t g0 = 0; g0 < G; g0 += 65535) {
     const int64_t gn = std::min<int64_t>(65535, G - g0);
