@@ -104,15 +104,16 @@ ABC_DEV double div_by(double x, double y, double zh, double zl) {
 }
 // v is zero or 2^-120 <= |v| < 2^200: differences of two such values are zero
 // or at least 2^-172, their squares over a denominator in [2^-300, 2^300] and
-// the remainders above stay normal numbers
+// the remainders above stay normal numbers.  NaN is in range too: it makes the
+// quotient, and so the error, NaN either way.
 ABC_DEV bool err_range(double v) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);
   const uint32_t e = (uint32_t)(b >> 52) & 0x7FFu;
-  return (e - (1023u - 120u)) < 320u || (b << 1) == 0ull;
+  return (e - (1023u - 120u)) < 320u || (b << 1) - 1ull >= 0xFFE0000000000000ull;  // 0 or NaN
 }
 ABC_DEV bool den_range(double y) {
   const uint32_t e = (uint32_t)((uint64_t)__double_as_longlong(y) >> 52);  // y > 0: no sign bit
-  return (e - (1023u - 300u)) < 600u;
+  return (e - (1023u - 300u)) < 600u || y != y;
 }
 
 // One gene's data value and denominator for one statistic.
