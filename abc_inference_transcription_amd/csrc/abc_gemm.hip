@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void gene_prep_kernel(const double* __restrict
       s_c[k][p] = WD * d;
       const Divisor v = divisor_of(den);
       genes[g * K + k] = ErrGene{d, v.y, v.zh, v.zl};
-      if (!err_range(d) || !den_range(den)) flag |= 2u;
+      if (!gene_range(d, den)) flag |= 2u;
       if (!(fabs(W) <= SCREEN_LIMIT) || !(fabs(WD) <= SCREEN_LIMIT)) flag |= 1u;
       Wf[g + G * k] = (float)W;
       b1 = -2.0 * WD;

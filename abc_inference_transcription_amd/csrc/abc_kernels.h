@@ -115,6 +115,11 @@ ABC_DEV bool den_range(double y) {
   const uint32_t e = (uint32_t)((uint64_t)__double_as_longlong(y) >> 52);  // y > 0: no sign bit
   return (e - (1023u - 300u)) < 600u || y != y;
 }
+// data value and denominator of a gene; an infinite value's denominator is
+// infinite (or NaN) and every quotient NaN, by div_by as by a division
+ABC_DEV bool gene_range(double d, double y) {
+  return (err_range(d) && den_range(y)) || __builtin_isinf(d);
+}
 
 // One gene's data value and denominator for one statistic.
 struct __align__(32) ErrGene {

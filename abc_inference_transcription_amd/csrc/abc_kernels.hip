@@ -1190,25 +1190,44 @@ __global__ __launch_bounds__(256) void stats_kernel(const DesignDev* __restrict_
 }
 
 // ------------------------------------------------------------------ errors
-// One FP64 error in the order of compute_errors.jl:30-64.
+// FP64 errors of gene g and N particles in the order of compute_errors.jl:30-64.
+template <int N>
+__device__ __forceinline__ void err_pairs(const double* __restrict__ data,
+                                          const double* __restrict__ se, int64_t G, int64_t g,
+                                          const double* __restrict__ stats, int64_t n,
+                                          const int64_t (&i)[N], const ErrSpec& E,
+                                          double (&err)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) err[j] = 0.0;
+  int k = 0;
+  for (int pp = 0; pp < E.n_parts; ++pp) {
+    double e[N] = {};
+    const int end = k + E.parts[pp];
+    for (; k < end; ++k) {
+      const double d = data[g + G * k];
+      const double den = err_den(d, se[g + G * k]);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const double diff = d - stats[i[j] + n * k];
+        e[j] += (diff * diff) / den;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) err[j] += e[j] / (double)E.K;
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    if (err[j] > E.clamp) err[j] = E.clamp;
+}
+
 __device__ __forceinline__ double err_pair(const double* __restrict__ data,
                                            const double* __restrict__ se, int64_t G, int64_t g,
                                            const double* __restrict__ stats, int64_t n,
                                            int64_t i, const ErrSpec& E) {
-  double err = 0.0;
-  int k = 0;
-  for (int pp = 0; pp < E.n_parts; ++pp) {
-    double e = 0.0;
-    const int end = k + E.parts[pp];
-    for (; k < end; ++k) {
-      const double d = data[g + G * k];
-      const double diff = d - stats[i + n * k];
-      e += (diff * diff) / err_den(d, se[g + G * k]);
-    }
-    err += e / (double)E.K;
-  }
-  if (err > E.clamp) err = E.clamp;
-  return err;
+  const int64_t at[1] = {i};
+  double err[1];
+  err_pairs<1>(data, se, G, g, stats, n, at, E, err);
+  return err[0];
 }
 
 // err holds the columns of genes g0 .. g0 + gridDim.y - 1; one lane per pair,
@@ -1233,8 +1252,11 @@ __global__ __launch_bounds__(256) void err_fp64_kernel(const double* __restrict_
 // known denominator, sum) against 22 with a division sequence and the
 // denominator formed per pair.  The operations and their order are err_pair's
 // and the quotients correctly rounded, so the bits are the same.  Pairs whose
-// operands leave err_range / den_range (infinite and NaN statistics among
-// them) are formed again by err_pair.  Waves at the end of the particles
+// operands leave err_range / gene_range (infinite statistics among them) are
+// formed by err_pairs: a tile's few such genes one pair a lane, such particles
+// four at a time (9,973 x 3,419 pairs, one such value in every particle or in 5 %
+// of the genes: 1.3 and 0.7 ms; one particle at a time for every lane that had
+// one of either, 3.1 and 2.7).  Waves at the end of the particles
 // overlap the ones before (the same values are written twice).  POOL: errors
 // and global particle indices behind the pool_n[g] entries of the genes'
 // acceptance pools instead, for a batch that meets no threshold yet.
@@ -1266,6 +1288,8 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
     if (!err_range(stats[i0 + p + ld * k])) bad |= 1u << p;
   }
   for (int o = 32; o > 0; o >>= 1) bad |= (uint32_t)__shfl_xor((int)bad, o);
+  bad = __builtin_amdgcn_readfirstlane(bad);
+  const bool none = bad == (1u << PT) - 1u;  // no particle in range: only the genes are looked at
   const int64_t gc = g < G ? g : G - 1;  // lanes past the last gene repeat it and store nothing
   const Divisor dk = divisor_of((double)K);
   double err[PT], e[PT], s[PT];
@@ -1284,7 +1308,7 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
       const int k = k0 + kk < K ? k0 + kk : K - 1;
       const double d = data[gc + G * k];
       const Divisor w = divisor_of(err_den(d, se[gc + G * k]));
-      gbad |= !err_range(d) || !den_range(w.y);
+      gbad |= !gene_range(d, w.y);
       s_d[kk][lane] = d;
       s_y[kk][lane] = w.y;
       s_zh[kk][lane] = w.zh;
@@ -1293,7 +1317,7 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
     const unsigned long long gb = __ballot(gbad);
     if (lane == 0 && gb) atomicOr(&s_gbad, gb);
     __syncthreads();
-    const int kc = K - k0 < ERR_KC ? K - k0 : ERR_KC;
+    const int kc = none ? 0 : (K - k0 < ERR_KC ? K - k0 : ERR_KC);
     double d = s_d[0][lane], y = s_y[0][lane], zh = s_zh[0][lane], zl = s_zl[0][lane];
     // waited for here, so that the wait at the top of the loop is not for them
     asm volatile("" : "+v"(d), "+v"(y), "+v"(zh), "+v"(zl));
@@ -1346,24 +1370,45 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
   }
 #pragma unroll
   for (int p = 0; p < PT; ++p) err[p] += div_by(e[p], dk.y, dk.zh, dk.zl);
-  if (g >= G) return;
-  PoolEntry* pg = POOL ? pool + g * capg + pool_n[g] : nullptr;
-  double* eg = POOL ? nullptr : err_out + n * g;
-#pragma unroll
-  for (int p = 0; p < PT; ++p) {
-    const double v = err[p] > E.clamp ? E.clamp : err[p];
+  auto store = [&](int64_t gene, int p, double v) {
     if (POOL)
-      pg[i0 + p] = PoolEntry{v, pidx ? pidx[i0 + p] : first_index + i0 + p};
+      pool[gene * capg + pool_n[gene] + i0 + p] =
+          PoolEntry{v, pidx ? pidx[i0 + p] : first_index + i0 + p};
     else
-      eg[i0 + p] = v;
+      err_out[n * gene + i0 + p] = v;
+  };
+  const int64_t left = G - (int64_t)blockIdx.y * 64;  // genes of this tile
+  const unsigned long long gbad = s_gbad & (left < 64 ? (1ull << left) - 1ull : ~0ull);
+  const bool mine = g < G && !((gbad >> lane) & 1ull);
+  if (mine) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+      if (!((bad >> p) & 1u)) store(g, p, err[p] > E.clamp ? E.clamp : err[p]);
   }
-  uint32_t again = (s_gbad >> lane) & 1ull ? (1u << PT) - 1u : bad;
-  while (again) {
-    const int p = __ffs(again) - 1;
-    again &= again - 1;
-    const double v = err_pair(data, se, G, g, stats, ld, i0 + p, E);
-    if (POOL) pg[i0 + p].err = v;
-    else eg[i0 + p] = v;
+  if (gbad) {
+    // lane r: the tile's r-th gene outside the range
+    const int nb = __popcll(gbad);
+    const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(gbad >> 32),
+                                                __builtin_amdgcn_mbcnt_lo((unsigned)gbad, 0u));
+    const int at = (gbad >> lane) & 1ull ? below : nb + lane - below;
+    const int ordered = __builtin_amdgcn_ds_permute(4 * at, lane);
+    for (int q0 = 0; q0 < nb * PT; q0 += 64) {
+      const int q = q0 + lane, p = q % PT;
+      const int64_t gene = (int64_t)blockIdx.y * 64 + __shfl(ordered, (q / PT) & 63);
+      if (q < nb * PT) store(gene, p, err_pair(data, se, G, gene, stats, ld, i0 + p, E));
+    }
+  }
+  while (mine && bad) {
+    int64_t at[4];
+    double v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // the last one again where fewer are left
+      at[j] = i0 + __ffs(bad) - 1;
+      if (bad & (bad - 1u) || j == 3) bad &= bad - 1u;
+    }
+    err_pairs<4>(data, se, G, g, stats, ld, at, E, v);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) store(g, (int)(at[j] - i0), v[j]);
   }
 }
 
