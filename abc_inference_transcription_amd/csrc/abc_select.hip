@@ -38,9 +38,9 @@ ABC_DEV double jl_quantile_sorted(const double* v, int n, double p) {
 }  // namespace
 
 // Workgroup (x, y): gene g0 + x, resamples y * rpb .. y * rpb + rpb - 1, one
-// wave per resample; each resample's share of every group goes to
-// shares[(x M + m) n_boot + b].  A gene with at most one accepting group is
-// written here by y = 0.
+// wave per resample (four or two on the labels of one or two resamples); each
+// resample's share of every group goes to shares[(x M + m) n_boot + b].  A gene
+// with at most one accepting group is written here by y = 0.
 // Bound by VALU issue: a label is half a Philox block (30 slots) and one 64-bit
 // comparison per group boundary.  A label idx = floor(u S / 2^64) reaches the
 // cumulative count A (idx >= A) exactly when u >= ceil(A 2^64 / S), so the
@@ -96,7 +96,11 @@ __global__ __launch_bounds__(ABC_SEL_WG) void model_prob_kernel(
   const int b_lo = (int)blockIdx.y * rpb;
   const int b_hi = b_lo + rpb < n_boot ? b_lo + rpb : n_boot;
   const uint32_t full = S32 >> 1;  // whole blocks of two draws
-  for (int b = b_lo + wave; b < b_hi; b += ABC_SEL_WG / 64) {
+  // waves per resample: more than one only where there are fewer resamples than waves
+  const int share = b_hi - b_lo > 2 ? 1 : (b_hi - b_lo == 2 ? 2 : 4);
+  const int piece = wave & (share - 1);
+  __shared__ uint32_t s_r[ABC_SEL_WG / 64][M];
+  for (int b = b_lo + wave / share; b < b_hi; b += ABC_SEL_WG / 64 / share) {
     uint32_t r[M];  // draws that reach A_k, uniform over the wave
 #pragma unroll
     for (int k = 0; k < M; ++k) r[k] = 0u;
@@ -108,16 +112,30 @@ __global__ __launch_bounds__(ABC_SEL_WG) void model_prob_kernel(
         r[k] += (uint32_t)__popcll(__ballot(in && ua > over[k])) +
                 (uint32_t)__popcll(__ballot(in && ub_ > over[k]));
     };
-    uint32_t q0 = 0;  // uniform: the counts stay in scalar registers
-    for (; q0 + 64u <= full; q0 += 64u) count(q0 + (uint32_t)lane, true);
-    if (q0 < full) count(q0 + (uint32_t)lane, q0 + (uint32_t)lane < full);
-    if (S32 & 1u) {  // the last draw of an odd number
+    // q0 is uniform: the counts stay in scalar registers
+    auto draws = [&](uint32_t q0, uint32_t step) {
+      for (; q0 + 64u <= full; q0 += step) count(q0 + (uint32_t)lane, true);
+      if (q0 < full) count(q0 + (uint32_t)lane, q0 + (uint32_t)lane < full);
+    };
+    if (share == 1) draws(0u, 64u);  // a loop of its own: with a variable step, 2 % more
+    else draws(64u * (uint32_t)piece, 64u * (uint32_t)share);
+    if (piece == 0 && (S32 & 1u)) {  // the last draw of an odd number
       const u4 w = philox(full, (uint32_t)b, (uint32_t)g, 0u, k0, k1);
       const uint64_t ua = (uint64_t)w.y << 32 | w.x;
 #pragma unroll
       for (int k = 0; k < M - 1; ++k) r[k] += ua > over[k] ? 1u : 0u;
     }
-    if (lane == 0) {
+    if (share > 1) {  // the whole workgroup: every wave is at its only piece
+      if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < M; ++k) s_r[wave][k] = r[k];
+      __syncthreads();
+      if (piece == 0)
+        for (int w = 1; w < share; ++w)
+#pragma unroll
+          for (int k = 0; k < M; ++k) r[k] += s_r[wave + w][k];
+    }
+    if (piece == 0 && lane == 0) {
       uint32_t reach = S32;
 #pragma unroll
       for (int m = 0; m < M; ++m) {
