@@ -1907,21 +1907,33 @@ int data_meta(abc_ctx* c, int64_t G, int64_t n, int32_t nc, const int32_t* age, 
 }
 
 // Refuses counts of 2^20 or more, in any cell.  Up to 65,536 counts each are
-// looked at on the host, before any device work, which also tells whether any
-// gene can need the 64-bit walk; more of them on the device, before the
-// resampling: a host scan of 18.5 million of each took 4 ms of the call.
+// looked at on the host, before any device work; more of them on the device,
+// before the resampling: a host scan of 18.5 million of each took 4 ms of the
+// call.  The host's look also tells which walks of data_stats_sorted_kernel
+// have genes (*walks: 1 the 32-bit one, 2 the 64-bit one), from the cells that
+// data_pack_kernel takes the largest u + l of: an empty launch is 10 us.
 constexpr size_t kDataHostScan = 65536;
 
-int data_check_host(abc_ctx* c, size_t nu, const uint32_t* u, const uint32_t* l, int64_t mm,
-                    bool* all_small) {
+int data_check_host(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t* l,
+                    const int32_t* cond, const int32_t* pulse, int64_t np, const int32_t* chase,
+                    int64_t nch, int* walks) {
+  std::vector<int32_t> used((size_t)n);  // a mask: the cell is in a group
+  for (int64_t i = 0; i < n; ++i) used[(size_t)i] = cond[i] >= 0 ? -1 : 0;
+  for (int64_t i = 0; i < np; ++i) used[(size_t)pulse[i]] = -1;
+  for (int64_t i = 0; i < nch; ++i) used[(size_t)chase[i]] = -1;
+  const uint64_t mm = (uint64_t)std::max(n, std::max(np, nch));
   uint32_t any = 0;
-  int32_t most = 0;  // no sum passes 2^21 unless it is refused
-  for (size_t i = 0; i < nu; ++i) {
-    any |= u[i] | l[i];
-    most = std::max(most, (int32_t)(u[i] + l[i]));
+  *walks = 0;
+  for (int64_t g = 0; g < G; ++g) {
+    int32_t most = 0;  // no sum passes 2^21 unless it is refused
+    for (int64_t i = 0; i < n; ++i) {
+      const uint32_t x = u[g * n + i], y = l[g * n + i];
+      any |= x | y;
+      most = std::max(most, (int32_t)(x + y) & used[(size_t)i]);
+    }
+    *walks |= (uint64_t)most * (uint64_t)most * mm < (1ull << 32) ? 1 : 2;
   }
   if (any >= (1u << 20)) return fail(c, ABC_E_ARG, "counts must be below 2^20");
-  *all_small = (uint64_t)most * (uint64_t)most * (uint64_t)mm < (1ull << 32);
   return ABC_OK;
 }
 
@@ -1943,10 +1955,10 @@ int data_check_dev(abc_ctx* c, size_t nu) {
 }
 
 // the kernel over every gene, in launches whose resample scratch stays near 1 GiB;
-// all_small: no gene is known to need the 64-bit walk
+// walks: 1 where genes may take the 32-bit walk, 2 where they may take the other
 int data_run(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t* l, int32_t nc,
              int32_t J, int64_t np, int64_t nch, int32_t n_boot, uint64_t seed, double* out,
-             bool all_small) {
+             int walks) {
   int rc;
   const int64_t K1 = 4 * nc + 3 * J;
   // families of at most ABC_DATA_SORTED_MAX cells: each gene's cells packed in
@@ -1991,7 +2003,8 @@ int data_run(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t
       const int64_t items = cnt * nsb;
       const size_t lds = data_sorted_lds(mmax);
       // every gene is one instantiation's: by its counts, which only the device knows
-      for (int small = 1; small >= (all_small ? 1 : 0); --small) {
+      for (int small = 1; small >= 0; --small) {
+        if (!(walks & (small ? 1 : 2))) continue;
         hipLaunchKernelGGL(small ? data_stats_sorted_kernel<true> : data_stats_sorted_kernel<false>,
                            dim3((unsigned)((items + 7) / 8 * 8)), dim3(ABC_DATA_WG), lds, c->stream,
                            cnt, nsb, g0, P<unsigned long long>(c->dxs), slots, xmax, n, np, nch, nc,
@@ -2034,7 +2047,7 @@ int32_t abc_data_stats_dev(abc_ctx* c, int64_t n_genes, int64_t n_cells, const u
   if ((n_cells > 0 && (!u_dev || !l_dev)) || !out_dev)
     return fail(c, ABC_E_ARG, "u, l and out are required");
   return data_run(c, n_genes, n_cells, u_dev, l_dev, n_clusters, n_conds, n_pulse, n_chase, n_boot,
-                  seed, out_dev, false);
+                  seed, out_dev, 3);
 }
 
 int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint32_t* u,
@@ -2051,9 +2064,9 @@ int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint3
   if ((n_cells > 0 && (!u || !l)) || !out) return fail(c, ABC_E_ARG, "u, l and out are required");
   const size_t nu = (size_t)n_genes * (size_t)n_cells;
   const size_t K = (size_t)(8 * n_clusters + 6 * n_conds);
-  bool all_small = false;
-  if (nu <= kDataHostScan &&
-      (rc = data_check_host(c, nu, u, l, std::max(n_cells, std::max(n_pulse, n_chase)), &all_small)))
+  int walks = 3;
+  if (nu <= kDataHostScan && (rc = data_check_host(c, n_genes, n_cells, u, l, cond, pulse, n_pulse,
+                                                   chase, n_chase, &walks)))
     return rc;
   if ((rc = ensure(c, c->du, sizeof(uint32_t) * (nu > 0 ? nu : 1)))) return rc;
   if ((rc = ensure(c, c->dl, sizeof(uint32_t) * (nu > 0 ? nu : 1)))) return rc;
@@ -2064,7 +2077,7 @@ int32_t abc_data_stats(abc_ctx* c, int64_t n_genes, int64_t n_cells, const uint3
   }
   if (nu > kDataHostScan && (rc = data_check_dev(c, nu))) return rc;
   rc = data_run(c, n_genes, n_cells, P<uint32_t>(c->du), P<uint32_t>(c->dl), n_clusters, n_conds,
-                n_pulse, n_chase, n_boot, seed, P<double>(c->dout), all_small);
+                n_pulse, n_chase, n_boot, seed, P<double>(c->dout), walks);
   if (rc) return rc;
   HIPCHK(c, hipMemcpyAsync(out, c->dout.p, sizeof(double) * (size_t)n_genes * K,
                            hipMemcpyDeviceToHost, c->stream));

@@ -63,11 +63,20 @@ def test_refused_in_any_place(eng, n, G, value, place):
     eng.data_stats(u, l, *rest, n_boot=3)
 
 
-# the largest u + l squared times the cells on both sides of 2^32
-@pytest.mark.parametrize("n,G,top", [(300, 40, 3784), (300, 40, 3785), (300, 300, 3785),
+# the largest u + l squared times the cells on both sides of 2^32: in one gene,
+# in every gene, in a cell that is in no group, and in one that only the pulse
+# list holds
+@pytest.mark.parametrize("n,G,top", [(300, 40, 3783), (300, 40, 3784), (300, 300, 3784),
                                      (64, 9, 1 << 19)])
-def test_walks_of_small_calls(oracle, eng, n, G, top):
+@pytest.mark.parametrize("where", ["one gene", "every gene", "no group", "pulse only"])
+def test_walks_of_small_calls(oracle, eng, n, G, top, where):
     u, l, rest = _cells(n, G, 1 + top // 3, seed=top)
-    u[3, 1], l[3, 1] = top // 2, top - top // 2
+    rest[1][3] = 0 if "gene" in where else -1
+    pulse, chase = (a[a != 3] for a in rest[4:6])
+    if where == "pulse only":
+        pulse = np.append(pulse, 3)
+    rest = (*rest[:4], pulse, chase, rest[6])
+    genes = slice(None) if where == "every gene" else slice(1, 2)
+    u[3, genes], l[3, genes] = top // 2, top - top // 2
     got = eng.data_stats(u, l, *rest, n_boot=5, seed=7)
     assert _same_bits(got, oracle.data_stats(u, l, *rest, n_boot=5, seed=7))
