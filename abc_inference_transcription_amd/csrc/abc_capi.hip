@@ -68,7 +68,8 @@ struct AcceptState {
   double eps = 0.0, margin_rel = 0.0;
   int64_t k = 0;
   int64_t n_candidates = 0, n_screened = 0;
-  unsigned long long cand_cap = 0;
+  unsigned long long cand_cap = 0;  // candidates a batch has room for
+  unsigned long long cand_max = 0;  // the session's largest batch of them
   // top-k (mode 1): per-gene pools of capg = k + n_sub entries in device
   // memory; batches are screened n_sub rows at a time
   bool pooled = false;
@@ -1040,14 +1041,18 @@ int screen_batch_pooled(abc_ctx* c, int64_t n, const double* stats_dev, int64_t 
   return ABC_OK;
 }
 
-// Accepted pairs kept in device memory at most (1.6 GB); more move to the host.
+// Accepted pairs the device list holds at most: 2 GB with the buffer's slack, and
+// 2.7 more for the lists of abc_accept_end.  Beyond it, pairs move to the host.
 constexpr int64_t kAccOnDevice = (int64_t)1 << 26;
+// Lists larger than this are given back when the session ends.
+constexpr size_t kAccKeepBytes = (size_t)256 << 20;
 
-// room for `more` accepted pairs behind the n_acc in the list, which are kept
-int acc_reserve(abc_ctx* c, int64_t more) {
+// the device list gets room for `pairs` accepted pairs; the n_acc in it are kept
+int acc_reserve(abc_ctx* c, int64_t pairs) {
   AcceptState& A = c->acc;
-  const size_t need = sizeof(Candidate) * (size_t)(A.n_acc + more);
+  const size_t need = sizeof(Candidate) * (size_t)pairs;
   if (c->acclist.bytes >= need) return ABC_OK;
+  if (A.n_acc == 0) return ensure(c, c->acclist, need, false);
   DevBuf old = c->acclist;
   c->acclist = DevBuf{};
   const int rc = ensure(c, c->acclist, need, false);
@@ -1055,23 +1060,20 @@ int acc_reserve(abc_ctx* c, int64_t more) {
     c->acclist = old;
     return rc;
   }
-  if (old.p) {
-    if (A.n_acc > 0)
-      HIPCHK(c, hipMemcpyAsync(c->acclist.p, old.p, sizeof(Candidate) * (size_t)A.n_acc,
-                               hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    hipFree(old.p);
-  }
+  HIPCHK(c, hipMemcpyAsync(c->acclist.p, old.p, sizeof(Candidate) * (size_t)A.n_acc,
+                           hipMemcpyDeviceToDevice, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  hipFree(old.p);
   return ABC_OK;
 }
 
 // the accepted pairs of the device list into the host's per-gene lists
 int acc_to_host(abc_ctx* c) {
   AcceptState& A = c->acc;
-  if (A.n_acc == 0) return ABC_OK;
   std::vector<Candidate> h((size_t)A.n_acc);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->acclist.p, sizeof(Candidate) * h.size(),
-                           hipMemcpyDeviceToHost, c->stream));
+  if (A.n_acc > 0)
+    HIPCHK(c, hipMemcpyAsync(h.data(), c->acclist.p, sizeof(Candidate) * h.size(),
+                             hipMemcpyDeviceToHost, c->stream));
   hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1((A.G + 1) / 2, 256)), dim3(256), 0, c->stream,
                      P<unsigned long long>(c->accgn), (A.G + 1) / 2);
   hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
@@ -1081,6 +1083,15 @@ int acc_to_host(abc_ctx* c) {
   for (const Candidate& x : h) A.kept[x.gene].push_back({x.err, x.particle});
   A.n_acc = 0;
   return ABC_OK;
+}
+
+// the session's lists have been returned
+void acc_release(abc_ctx* c) {
+  for (DevBuf* b : {&c->acclist, &c->accent, &c->accidx, &c->accerr})
+    if (b->bytes > kAccKeepBytes) {
+      hipFree(b->p);
+      *b = DevBuf{};
+    }
 }
 
 int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_index,
@@ -1107,8 +1118,7 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
   unsigned long long cap = std::max<unsigned long long>(A.cand_cap, 1ull << 16);
   for (;;) {
     if ((rc = ensure(c, c->cand, sizeof(Candidate) * cap))) return rc;
-    if (A.n_acc > 0 && A.n_acc + (int64_t)cap > kAccOnDevice && (rc = acc_to_host(c))) return rc;
-    if ((rc = acc_reserve(c, (int64_t)cap))) return rc;
+    if ((rc = acc_reserve(c, std::min(A.n_acc + (int64_t)cap, kAccOnDevice)))) return rc;
     hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, c->stream,
                        P<unsigned long long>(c->ccount), (int64_t)1);
     hipLaunchKernelGGL(gemm_screen_kernel, dim3((unsigned)(npad / 64), (unsigned)(A.Gpad / 64)),
@@ -1119,11 +1129,16 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
                        P<unsigned long long>(c->ccount), cap, (float*)nullptr, (float*)nullptr,
                        (PoolEntry*)nullptr, (int64_t)0, (uint32_t*)nullptr);
     HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(rescore_kernel, dim3(grid1((int64_t)cap, 256)), dim3(256), 0, c->stream,
-                       stats_dev, n, P<double>(c->edata), P<double>(c->ese), A.G, A.E,
-                       P<Candidate>(c->cand), P<unsigned long long>(c->ccount), cap, A.eps,
-                       first_index, pidx_dev, P<Candidate>(c->acclist),
-                       P<unsigned long long>(c->accn), P<uint32_t>(c->accgn));
+    // candidates [q0, q0 + nq) rescored, the accepted ones into the device list
+    const int64_t room = std::min<int64_t>((int64_t)(c->acclist.bytes / sizeof(Candidate)), kAccOnDevice);
+    auto rescore = [&](int64_t q0, int64_t nq) {
+      hipLaunchKernelGGL(rescore_kernel, dim3(grid1(nq, 256)), dim3(256), 0, c->stream, stats_dev, n,
+                         P<double>(c->edata), P<double>(c->ese), A.G, A.E, P<Candidate>(c->cand),
+                         P<unsigned long long>(c->ccount), cap, q0, A.eps, first_index, pidx_dev,
+                         P<Candidate>(c->acclist), (unsigned long long)room,
+                         P<unsigned long long>(c->accn), P<uint32_t>(c->accgn));
+    };
+    rescore(0, (int64_t)cap);
     HIPCHK(c, hipGetLastError());
     unsigned long long cnt = 0, nacc = 0;
     HIPCHK(c, hipMemcpyAsync(&cnt, c->ccount.p, 8, hipMemcpyDeviceToHost, c->stream));
@@ -1135,7 +1150,22 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
       continue;
     }
     A.n_candidates += (int64_t)cnt;
-    A.n_acc = (int64_t)nacc;
+    A.cand_max = std::max(A.cand_max, cnt);
+    if ((int64_t)nacc > room) {
+      // the list ended within this batch: its pairs from before move to the
+      // host, and the batch's candidates are rescored again, a list's worth a time
+      if ((rc = acc_to_host(c))) return rc;
+      for (int64_t q0 = 0; q0 < (int64_t)cnt; q0 += room) {
+        if (q0 > 0 && (rc = acc_to_host(c))) return rc;
+        rescore(q0, std::min<int64_t>(room, (int64_t)cnt - q0));
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipMemcpyAsync(&nacc, c->accn.p, 8, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        A.n_acc = (int64_t)nacc;
+      }
+    } else {
+      A.n_acc = (int64_t)nacc;
+    }
     break;
   }
   A.n_screened += n;
@@ -1158,6 +1188,12 @@ int32_t abc_accept_begin(abc_ctx* c, int32_t K, int64_t G, const double* data, c
   int rc = make_spec(c, K, parts, n_parts, clamp, &A.E);
   if (rc) return rc;
   if (K > 128) return fail(c, ABC_E_ARG, "screening supports K <= 128");
+  // a session starts with the room that earlier ones needed, beyond 4 million
+  // candidates with the last one's: the lists of a batch are sized by it
+  if (A.mode == 0 && A.n_screened > 0)
+    A.cand_cap = std::max<unsigned long long>(std::min(A.cand_cap, 1ull << 22),
+                                              A.cand_max + A.cand_max / 8);
+  A.cand_max = 0;
   A.G = G;
   A.Kp = (int)pad_to(K, 32);
   A.Gpad = pad_to(std::max<int64_t>(G, 1), 64);
@@ -1466,6 +1502,7 @@ int32_t abc_accept_end(abc_ctx* c, int64_t* counts, int64_t* idx, double* err_ou
   if (total > cap) return fail(c, ABC_E_CAPACITY, "accepted entries exceed cap");
   A.active = false;
   A.kept.clear();
+  acc_release(c);
   return ABC_OK;
 }
 
@@ -1479,6 +1516,7 @@ int32_t abc_accept(abc_ctx* c, int64_t n, int32_t K, const double* stats, int64_
   if (rc) return rc;
   if ((rc = abc_accept_add(c, n, stats, first_index))) { c->acc.active = false; return rc; }
   rc = abc_accept_end(c, counts, idx, err_out, cap, nullptr);
+  if (rc) acc_release(c);
   c->acc.active = false;
   return rc;
 }

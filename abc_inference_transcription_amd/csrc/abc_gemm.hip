@@ -308,10 +308,11 @@ __global__ __launch_bounds__(256) void gemm_screen_kernel(
   }
 }
 
-// FP64 rescoring of the batch's *count candidates in the reference operation
-// order (compute_errors.jl:30-64); those with err <= eps_acc join the session's
-// accepted pairs acc[0 .. *n_acc), counted per gene.  With more candidates than
-// cap the batch is screened again, so nothing is accepted.  Candidate.particle
+// FP64 rescoring of the batch's *count candidates from q0 on, one per thread, in
+// the reference operation order (compute_errors.jl:30-64); those with err <=
+// eps_acc join the session's accepted pairs acc[0 .. *n_acc), counted per gene.
+// With more candidates than cap the batch is screened again, so nothing is
+// accepted; pairs past room are counted and not stored.  Candidate.particle
 // holds the batch-local row on entry, the global particle index (pidx[row], or
 // first_index + row) in acc.
 __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__ stats, int64_t n,
@@ -320,13 +321,14 @@ __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__
                                                       ErrSpec E,
                                                       const Candidate* __restrict__ cand,
                                                       const unsigned long long* __restrict__ count,
-                                                      unsigned long long cap, double eps_acc,
-                                                      int64_t first_index,
+                                                      unsigned long long cap, int64_t q0,
+                                                      double eps_acc, int64_t first_index,
                                                       const int64_t* __restrict__ pidx,
                                                       Candidate* __restrict__ acc,
+                                                      unsigned long long room,
                                                       unsigned long long* __restrict__ n_acc,
                                                       uint32_t* __restrict__ gene_n) {
-  const unsigned long long q = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned long long q = q0 + (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
   const unsigned long long m = *count;
   if (m > cap || q >= m) return;
   Candidate c = cand[q];
@@ -351,7 +353,8 @@ __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__
   if (err <= eps_acc) {  // never for NaN
     c.err = err;
     c.particle = pidx ? pidx[i] : first_index + i;
-    acc[atomicAdd(n_acc, 1ull)] = c;
+    const unsigned long long at = atomicAdd(n_acc, 1ull);
+    if (at < room) acc[at] = c;
     atomicAdd(gene_n + g, 1u);
   }
 }
