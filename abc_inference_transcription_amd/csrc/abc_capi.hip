@@ -22,13 +22,10 @@
 // Device memory of abc_simulate_noalloc_dev: one array per GPU, alive until
 // the process ends.  Host code reaches it only through the address
 // hipGetSymbolAddress returns for the current device (scratch_address).
-// The limit on the particles of a call is a formula of its own
-// (noalloc_bytes); the workspace carved for an accepted call never exceeds it
-// by more than the fixed bucket tables, which the margin holds.
-#define ABC_NOALLOC_SCRATCH_BYTES ((size_t)256 << 20)
-#define ABC_NOALLOC_MARGIN_BYTES ((size_t)64 << 10)
-static __device__ __align__(256) unsigned char
-    scratch[ABC_NOALLOC_SCRATCH_BYTES + ABC_NOALLOC_MARGIN_BYTES];
+// A call is accepted when its workspace (ws_carve) fits: 77 bytes per cell,
+// 592 per particle and 21 KiB of tables, for which the array has 64 KiB.
+#define ABC_NOALLOC_SCRATCH_BYTES (((size_t)256 << 20) + ((size_t)64 << 10))
+static __device__ __align__(256) unsigned char scratch[ABC_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 
@@ -255,20 +252,6 @@ size_t ws_carve(char* base, int64_t n, int C, SimWs* w) {
   v.tally = reinterpret_cast<unsigned long long*>(take(16));
   v.steps = reinterpret_cast<unsigned long long*>(take(sizeof(uint64_t) * nn));
   if (base && w) *w = v;
-  return at;
-}
-
-// Bytes that bound a call of abc_simulate_noalloc_dev: about 77 per cell and
-// 620 per particle, rounded up array by array.
-size_t noalloc_bytes(int64_t n, int C) {
-  const size_t nn = (size_t)n, cells = nn * (size_t)C;
-  const size_t blk = (size_t)((n + 1023) / 1024);
-  const size_t part[] = {sizeof(PRates) * nn, 4 * nn, 8 * ABC_NBUCKET, 4 * nn, 8 * blk,
-                         8 * (nn + 1), sizeof(CellStart) * cells, 4 * nn * (size_t)(C + 1),
-                         8 * nn, 8 * (size_t)cell_words(n, C), 8 * (size_t)cell_words(n, C),
-                         cells, 8 * nn, 64, 16, 8 * nn};
-  size_t at = 0;
-  for (size_t b : part) at += (std::max<size_t>(b, 16) + 255) / 256 * 256;
   return at;
 }
 
@@ -864,19 +847,17 @@ int32_t abc_simulate_noalloc_dev(abc_ctx* c, int32_t model, uint64_t seed, int64
   if ((rc = check_range(c, model, first, n))) return rc;
   if (n == 0) return ABC_OK;
   const int C = c->hd.C;
-  if (noalloc_bytes(n, C) > ABC_NOALLOC_SCRATCH_BYTES) {
+  if (ws_carve(nullptr, n, C, nullptr) > ABC_NOALLOC_SCRATCH_BYTES) {
     int64_t lo = 0, hi = (int64_t)1 << 31;  // the largest n whose workspace fits
     while (hi - lo > 1) {
       const int64_t mid = lo + (hi - lo) / 2;
-      (noalloc_bytes(mid, C) <= ABC_NOALLOC_SCRATCH_BYTES ? lo : hi) = mid;
+      (ws_carve(nullptr, mid, C, nullptr) <= ABC_NOALLOC_SCRATCH_BYTES ? lo : hi) = mid;
     }
     return fail(c, ABC_E_ARG,
                 "abc_simulate_noalloc_dev takes at most " + std::to_string(lo) +
                     " particles of " + std::to_string(C) + " cells per call (" +
                     std::to_string(ABC_NOALLOC_SCRATCH_BYTES >> 20) + " MiB of scratch)");
   }
-  if (ws_carve(nullptr, n, C, nullptr) > ABC_NOALLOC_SCRATCH_BYTES + ABC_NOALLOC_MARGIN_BYTES)
-    return fail(c, ABC_E_ARG, "the scratch array is too small");
   SimWs w;
   ws_carve(static_cast<char*>(c->scratch), n, C, &w);
   w.timed = false;  // its burn-in draws are not in the context's tally

@@ -199,7 +199,7 @@ int32_t abc_simulate_multi_idx_dev(abc_ctx* ctx, int32_t n_models, const int32_t
  * results, bit for bit, as abc_simulate_dev; its workspace (rates, queue
  * order, burn-in records, sub-lane offsets, cell counts, counters) is carved
  * from one 256 MiB array per GPU held by the library until the process ends,
- * so a call needs about 77 * cells + 400 bytes per particle: at most about
+ * so a call needs about 77 * cells + 592 bytes per particle: at most about
  * 1,390 particles of 2,500 cells (ABC_E_ARG beyond the limit, with the limit
  * in abc_last_error).  Every call on a GPU uses the same array, and each call
  * clears what it needs cleared: calls that overlap on one GPU (two streams,
