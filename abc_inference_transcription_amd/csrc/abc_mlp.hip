@@ -503,10 +503,12 @@ __global__ __launch_bounds__(256) void adam_kernel(
   store_copies(x, T, D, bf_off[T.layer], Wb, WbT, Wf);
 }
 
-// the gradient itself, for a caller that asks for it (launch as adam_kernel)
+// the gradient itself, for a caller that asks for it (launch as adam_kernel).  A
+// layer with one sum has it in g already (P.p points there): each value is read
+// by the thread that writes it
 __global__ __launch_bounds__(256) void grad_sum_kernel(GradParts P,
                                                        const LayerDesc* __restrict__ L, int nl,
-                                                       float* __restrict__ g,
+                                                       float* g,
                                                        const float* __restrict__ loss_parts,
                                                        int n_loss, float* __restrict__ loss) {
   if (blockIdx.x == gridDim.x - 1) loss_total(loss_parts, n_loss, loss, nullptr);
