@@ -1584,14 +1584,24 @@ int moment_cfg(abc_ctx* c, int model, const abc_moment_cfg* u, MomCfgDev* m) {
 // Particles, the costliest first, that the integrating kernels give to teams of
 // eight lanes (a multiple of 8).  Teams shorten an integration's chain 2.6 times
 // for about 2.4 times the issue slots, so they pay while the longest chains set
-// the time: for nearly all particles of a small call, for ever fewer of the
-// costliest as the call fills the machine.  Team waves 0 / 512 / 2,048 / 16,384,
-// ms per call of models 1 to 5 (reference prior): n = 4,096 model 1 62 / 36 / 30 /
-// 26, model 4 72 / 56 / 51 / 43; n = 8,192 model 3 139 / 87 / 66 / 69, model 5
-// 91 / 92 / 95 / 114; n = 32,768 model 3 155 / 144 / 153 / 192, model 5 248 / 252 /
-// 259 / 314.
-int64_t moment_heavy(int64_t n, int64_t items) {
-  const int64_t waves = n <= 4096 ? 16384 : (n <= 12288 ? 1024 : 512);
+// the time: for every particle while the waves of a launch without teams are at
+// most `full` times the machine's wave slots (two per SIMD), then for as many of
+// the costliest as fill 3/4 of the slots, ever fewer beyond twice that many
+// waves.  full is 1 for the cycle maps and 2 for the trajectories,
+// whose items are partly short.  Both sides of the lines, ms per call of models 1
+// to 5 (reference prior, 55 items, 2,048 slots), all teams / 3/4 of the slots:
+// trajectories, n = 4,096 23 21 47 39 63 / 26 22 52 43 62, 4,600 24 24 47 45 69 /
+// 27 23 53 52 67, 5,500 28 24 49 51 83 / 30 24 56 51 69, 8,192 38 34 68 72 122 /
+// 33 25 61 57 86; cycle maps, n = 12,288 43 27 78 65 115 / 44 30 85 69 115, 20,000
+// 51 43 106 99 178 / 50 42 105 95 165.  3/4 / 1/4 of the slots: trajectories, n =
+// 8,192 33 25 61 57 86 / 36 23 72 50 82, 24,000 63 52 116 119 214 / 60 51 112 117
+// 211.  No one line suits every model: the spread of the particles' costs decides,
+// which only the device knows.
+int64_t moment_heavy(const abc_ctx* c, int64_t n, int64_t items, int full) {
+  const int64_t slots = (int64_t)c->num_cu * 8;
+  const int64_t plain = (n + 63) / 64 * items;
+  if (plain <= full * slots) return (n + 7) / 8 * 8;
+  const int64_t waves = std::min(slots * 3 / 4, 3 * full * slots * slots / (2 * plain));
   return std::min<int64_t>((n + 7) / 8, waves / items) * 8;
 }
 
@@ -1623,7 +1633,7 @@ int moment_run(abc_ctx* c, int model, int64_t n, const double* theta_dev, int64_
   hipLaunchKernelGGL(moment_order_kernel, dim3(1), dim3(ABC_MOM_ORDER_WG), 0, c->stream, n, key,
                      ord_map);
   hipLaunchKernelGGL(zero_u64_kernel, dim3(grid1(n, 256)), dim3(256), 0, c->stream, cost, n);
-  const int64_t hc = m.method == 1 ? moment_heavy(n, 10) : 0;
+  const int64_t hc = m.method == 1 ? moment_heavy(c, n, 10, 1) : 0;
   const unsigned wc = moment_waves(n, hc, 10);
   auto cyclemap = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(wc), dim3(64), 0, c->stream, m, model, n, theta_dev, ld, ord_map,
@@ -1640,7 +1650,7 @@ int moment_run(abc_ctx* c, int model, int64_t n, const double* theta_dev, int64_
   HIPCHK(c, hipGetLastError());
   // one wave per (group of ordered particles, condition x age item)
   const int64_t items = (int64_t)m.n_conds * m.n_ages;
-  const int64_t ht = m.method == 1 ? moment_heavy(n, items) : 0;
+  const int64_t ht = m.method == 1 ? moment_heavy(c, n, items, 2) : 0;
   const unsigned wt = moment_waves(n, ht, items);
   auto traj = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(wt), dim3(64), 0, c->stream, m, model, n, theta_dev, ld,
