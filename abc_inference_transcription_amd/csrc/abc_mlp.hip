@@ -29,9 +29,13 @@ namespace {
 
 enum { EPI_F32 = 0, EPI_SILU = 1, EPI_DSILU = 2, EPI_DW = 3 };
 
-// K per pipeline stage (32-deep MFMA steps): 64, and 128 for the weight
-// gradients, whose few workgroups per CU wait at every stage's barrier
-constexpr int stage_k(int epi) { return epi == EPI_DW ? 128 : 64; }
+// K per pipeline stage (32-deep MFMA steps): 64, and 128 for the weight gradients
+// in 64 x 64 tiles, whose few workgroups per CU wait at every stage's barrier.
+// Larger tiles are for products that fill the machine, where the LDS of a deeper
+// stage leaves room for one workgroup per CU instead of two (a step of width
+// 4,096 and 8,192 samples 1,700 us with 128, 1,600 with 64).
+constexpr int stage_k(int epi, int bm, int bn) { return epi == EPI_DW && bm * bn == 64 * 64 ? 128 : 64; }
+constexpr int kDwChunk = 128;  // a chunk of a split gradient is whole stages
 
 // s = 1 / (1 + e^-z) of four values.  The reciprocals of x = 1 + e^-z >= 1 are
 // correctly rounded without the division sequence: the hardware's reciprocal
@@ -85,7 +89,7 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const bf16* __restrict__ A
                                                       float* __restrict__ Zout) {
   constexpr int WN = BN / 2, NCB = WN / 16;
   constexpr int WM = BM / 2, NRB = WM / 16;
-  constexpr int BK = stage_k(EPI), LDSK = BK + 8;  // 8 of padding against bank conflicts
+  constexpr int BK = stage_k(EPI, BM, BN), LDSK = BK + 8;  // 8 of padding against bank conflicts
   constexpr int BQ = BK / 8;                       // 16-byte pieces of a row's stage
   constexpr int NAQ = BM * BQ / 256, NBQ = BN * BQ / 256;
   __shared__ bf16 As[2][BM][LDSK];
@@ -995,8 +999,7 @@ int splitk_for(int M, int N, int K) {
   return S;
 }
 int splitk_chunk(int K, int S) {
-  const int bk = stage_k(EPI_DW);
-  return (K / bk + S - 1) / S * bk;  // K, the padded batch, is a multiple of bk
+  return (K / kDwChunk + S - 1) / S * kDwChunk;  // K, the padded batch, is a multiple of it
 }
 
 // Workgroup tile rows: 64 when 128-row tiles would leave fewer than two
