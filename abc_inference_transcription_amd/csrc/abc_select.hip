@@ -41,13 +41,14 @@ ABC_DEV double jl_quantile_sorted(const double* v, int n, double p) {
 // wave per resample (four or two on the labels of one or two resamples); each
 // resample's share of every group goes to shares[(x M + m) n_boot + b].  A gene
 // with at most one accepting group is written here by y = 0.
-// Bound by VALU issue: a label is half a Philox block (30 slots) and one 64-bit
-// comparison per group boundary.  A label idx = floor(u S / 2^64) reaches the
+// Bound by VALU issue: a label is half a Philox block and one 64-bit comparison
+// per group boundary, 41 instructions per two labels of two groups.  A label idx = floor(u S / 2^64) reaches the
 // cumulative count A (idx >= A) exactly when u >= ceil(A 2^64 / S), so the
 // boundaries are scaled once per workgroup and the index, a 64 x 32
 // multiply-high per label, is never formed; the comparisons are counted by
 // scalar popcounts of their lane masks, the M - 1 counts in scalar registers.  2,000 genes,
-// 2 groups, 33,000 labels a gene on average, 100 resamples: the call 8.8 -> 3.7 ms.
+// 2 groups, 29,500 resampled labels a gene on average, 100 resamples: the call 8.8 ->
+// 3.7 ms, of the 3.1 that the instructions take at one a cycle and lane.
 template <int M>
 __global__ __launch_bounds__(ABC_SEL_WG) void model_prob_kernel(
     int64_t G, int64_t g0, const int64_t* __restrict__ counts, uint32_t k0, uint32_t k1,
