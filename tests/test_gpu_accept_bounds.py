@@ -81,7 +81,7 @@ def test_tight_session_after_a_loose_one(engine_factory):
 
     def tight(eng):
         best, out = np.inf, None
-        for _ in range(3):
+        for _ in range(8):
             _begin(eng, data, se, eps)
             t = time.perf_counter()
             for a in range(0, 2000, 250):

@@ -32,7 +32,7 @@ def test_one_more_particle(eng, model):
             eng.recover(model, x, cfg)
             best[n] = min(best[n], 1e3 * (time.perf_counter() - t))
     print(f"\n[moment lines] model {model}: {best}", flush=True)
-    assert best[4097] < 1.08 * best[4096]
+    assert best[4097] < 1.12 * best[4096]
 
 
 # (condition, age) items, and particles on both sides of the rule's lines on 256
