@@ -1288,8 +1288,6 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
     if (!err_range(stats[i0 + p + ld * k])) bad |= 1u << p;
   }
   for (int o = 32; o > 0; o >>= 1) bad |= (uint32_t)__shfl_xor((int)bad, o);
-  bad = __builtin_amdgcn_readfirstlane(bad);
-  const bool none = bad == (1u << PT) - 1u;  // no particle in range: only the genes are looked at
   const int64_t gc = g < G ? g : G - 1;  // lanes past the last gene repeat it and store nothing
   const Divisor dk = divisor_of((double)K);
   double err[PT], e[PT], s[PT];
@@ -1317,6 +1315,10 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
     const unsigned long long gb = __ballot(gbad);
     if (lane == 0 && gb) atomicOr(&s_gbad, gb);
     __syncthreads();
+    // no particle in range: only the genes are looked at.  bad stays in a vector
+    // register, since the loop's statistics fill the scalar ones
+    asm volatile("" : "+v"(bad));
+    const bool none = __builtin_amdgcn_readfirstlane(bad) == (1u << PT) - 1u;
     const int kc = none ? 0 : (K - k0 < ERR_KC ? K - k0 : ERR_KC);
     double d = s_d[0][lane], y = s_y[0][lane], zh = s_zh[0][lane], zl = s_zl[0][lane];
     // waited for here, so that the wait at the top of the loop is not for them
@@ -1370,20 +1372,30 @@ __global__ __launch_bounds__(256) void err_tile_kernel(const double* __restrict_
   }
 #pragma unroll
   for (int p = 0; p < PT; ++p) err[p] += div_by(e[p], dk.y, dk.zh, dk.zl);
-  auto store = [&](int64_t gene, int p, double v) {
-    if (POOL)
-      pool[gene * capg + pool_n[gene] + i0 + p] =
-          PoolEntry{v, pidx ? pidx[i0 + p] : first_index + i0 + p};
-    else
-      err_out[n * gene + i0 + p] = v;
-  };
+  bad = __builtin_amdgcn_readfirstlane(bad);
   const int64_t left = G - (int64_t)blockIdx.y * 64;  // genes of this tile
   const unsigned long long gbad = s_gbad & (left < 64 ? (1ull << left) - 1ull : ~0ull);
   const bool mine = g < G && !((gbad >> lane) & 1ull);
+  auto put = [&](PoolEntry* pg, double* eg, int p, double v) {
+    if (POOL)
+      pg[i0 + p] = PoolEntry{v, pidx ? pidx[i0 + p] : first_index + i0 + p};
+    else
+      eg[i0 + p] = v;
+  };
+  auto store = [&](int64_t gene, int p, double v) {
+    put(POOL ? pool + gene * capg + pool_n[gene] : nullptr, POOL ? nullptr : err_out + n * gene, p, v);
+  };
   if (mine) {
+    PoolEntry* pg = POOL ? pool + g * capg + pool_n[g] : nullptr;
+    double* eg = POOL ? nullptr : err_out + n * g;
+    if (bad == 0u) {
 #pragma unroll
-    for (int p = 0; p < PT; ++p)
-      if (!((bad >> p) & 1u)) store(g, p, err[p] > E.clamp ? E.clamp : err[p]);
+      for (int p = 0; p < PT; ++p) put(pg, eg, p, err[p] > E.clamp ? E.clamp : err[p]);
+    } else {
+#pragma unroll
+      for (int p = 0; p < PT; ++p)
+        if (!((bad >> p) & 1u)) put(pg, eg, p, err[p] > E.clamp ? E.clamp : err[p]);
+    }
   }
   if (gbad) {
     // lane r: the tile's r-th gene outside the range
