@@ -1110,13 +1110,13 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
                        P<unsigned long long>(c->ccount), cap, (float*)nullptr, (float*)nullptr,
                        (PoolEntry*)nullptr, (int64_t)0, (uint32_t*)nullptr);
     HIPCHK(c, hipGetLastError());
-    // candidates [q0, q0 + nq) rescored, the accepted ones into the device list
+    // candidates [q0, q1) rescored, the accepted ones into the device list
     const int64_t room = std::min<int64_t>((int64_t)(c->acclist.bytes / sizeof(Candidate)), kAccOnDevice);
-    auto rescore = [&](int64_t q0, int64_t nq) {
-      hipLaunchKernelGGL(rescore_kernel, dim3(grid1(nq, 256)), dim3(256), 0, c->stream, stats_dev, n,
+    auto rescore = [&](int64_t q0, int64_t q1) {
+      hipLaunchKernelGGL(rescore_kernel, dim3(grid1(q1 - q0, 256)), dim3(256), 0, c->stream, stats_dev, n,
                          P<double>(c->edata), P<double>(c->ese), A.G, A.E, P<Candidate>(c->cand),
-                         P<unsigned long long>(c->ccount), cap, q0, A.eps, first_index, pidx_dev,
-                         P<Candidate>(c->acclist), (unsigned long long)room,
+                         P<unsigned long long>(c->ccount), cap, q0, q1, A.eps, first_index,
+                         pidx_dev, P<Candidate>(c->acclist), (unsigned long long)room,
                          P<unsigned long long>(c->accn), P<uint32_t>(c->accgn));
     };
     rescore(0, (int64_t)cap);
@@ -1138,7 +1138,7 @@ int screen_batch(abc_ctx* c, int64_t n, const double* stats_dev, int64_t first_i
       if ((rc = acc_to_host(c))) return rc;
       for (int64_t q0 = 0; q0 < (int64_t)cnt; q0 += room) {
         if (q0 > 0 && (rc = acc_to_host(c))) return rc;
-        rescore(q0, std::min<int64_t>(room, (int64_t)cnt - q0));
+        rescore(q0, std::min<int64_t>(q0 + room, (int64_t)cnt));
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipMemcpyAsync(&nacc, c->accn.p, 8, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -308,8 +308,8 @@ __global__ __launch_bounds__(256) void gemm_screen_kernel(
   }
 }
 
-// FP64 rescoring of the batch's *count candidates from q0 on, one per thread, in
-// the reference operation order (compute_errors.jl:30-64); those with err <=
+// FP64 rescoring of the batch's *count candidates, those of [q0, q1), in the
+// reference operation order (compute_errors.jl:30-64); those with err <=
 // eps_acc join the session's accepted pairs acc[0 .. *n_acc), counted per gene.
 // With more candidates than cap the batch is screened again, so nothing is
 // accepted; pairs past room are counted and not stored.  Candidate.particle
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__
                                                       ErrSpec E,
                                                       const Candidate* __restrict__ cand,
                                                       const unsigned long long* __restrict__ count,
-                                                      unsigned long long cap, int64_t q0,
+                                                      unsigned long long cap, int64_t q0, int64_t q1,
                                                       double eps_acc, int64_t first_index,
                                                       const int64_t* __restrict__ pidx,
                                                       Candidate* __restrict__ acc,
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256) void rescore_kernel(const double* __restrict__
                                                       uint32_t* __restrict__ gene_n) {
   const unsigned long long q = q0 + (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
   const unsigned long long m = *count;
-  if (m > cap || q >= m) return;
+  if (m > cap || q >= m || q >= (unsigned long long)q1) return;
   Candidate c = cand[q];
   const int64_t i = c.particle, g = c.gene;
   const double s2 = 0.1 * 0.1;

@@ -317,6 +317,6 @@ __global__ void thr_min_kernel(double* thr, const double* lower, int64_t G);
 __global__ void rescore_kernel(const double* stats, int64_t n, const double* data,
                                const double* se, int64_t G, ErrSpec E, const Candidate* cand,
                                const unsigned long long* count, unsigned long long cap,
-                               int64_t q0, double eps_acc, int64_t first_index,
+                               int64_t q0, int64_t q1, double eps_acc, int64_t first_index,
                                const int64_t* pidx, Candidate* acc, unsigned long long room,
                                unsigned long long* n_acc, uint32_t* gene_n);
