@@ -66,9 +66,11 @@ struct __align__(16) CellStart {
 };
 
 // Tables of the cell order (cell_scan_kernel), by rank from the heaviest
-// bucket: first item (and all items at the end), first cell, scatter cursor.
+// bucket: first item (and all items at the end), first cell, scatter cursor;
+// and the expected draws of all items, by their classes.
 struct CellTables {
   unsigned long long ioff[ABC_CELL_BUCKETS + 1];
+  double draws;
   unsigned cbase[ABC_CELL_BUCKETS], cursor[ABC_CELL_BUCKETS];
 };
 

@@ -319,6 +319,13 @@ __global__ __launch_bounds__(ABC_CELL_BUCKETS) void cell_scan_kernel(
   T->cursor[t] = sc[t] - x;
   T->ioff[t] = si[t] - it;
   if (t == ABC_CELL_BUCKETS - 1) T->ioff[ABC_CELL_BUCKETS] = si[t];
+  __shared__ double sd[ABC_CELL_BUCKETS];
+  sd[t] = (double)it * ex(0x1.62e42fee00000p-1 * (2.0 + 0.25 * (id >> 4)));  // 4 draws in class 0
+  for (int d = ABC_CELL_BUCKETS / 2; d > 0; d >>= 1) {
+    __syncthreads();
+    if (t < d) sd[t] += sd[t + d];
+  }
+  if (t == 0) T->draws = sd[0];
 }
 
 // Each workgroup places a tile of cells: ranks within the tile from LDS
@@ -725,6 +732,8 @@ __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) voi
   for (int q = threadIdx.x; q <= ABC_CELL_BUCKETS; q += blockDim.x) ioff[q] = tabs->ioff[q];
   __syncthreads();
   const unsigned long long total = ioff[ABC_CELL_BUCKETS];
+  // expected draws of two lanes' shares of the call, which no claim exceeds
+  const float share = 2.0f * (float)tabs->draws / (float)(gridDim.x * SSA_WG);
 
   uint32_t cw = 0;  // counter word of the current item: cell | model << 24
   // per-lane item state
@@ -759,7 +768,12 @@ __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) voi
   // ones singly, since a second one waiting behind the first would end late.
   // 5 x 1,024 particles: 329 ms with one item a claim throughout, 312 ms with
   // claims of `claim` items below class 36, 296 ms so; the line at class 32 or
-  // 40 measured 297 and 299 ms.
+  // 40 measured 297 and 299 ms.  Nor more than twice a lane's share of the call's
+  // draws, or a call of light items alone ends with the lanes that claimed many:
+  // 20,000 particles of 55 cells with 43 / 128 draws a cell 6.2 / 9.4 ms without
+  // that, 4.7 / 7.1 with it (with `claim` 8 12 / 19 and 4.7 / 7.3).  Half a share,
+  // one, two, no limit: 3,000 particles of 2,000 cells 12.7, 11.0, 9.9, 10.5 ms,
+  // 20,000 of 55 cells with 969 draws 15.0, 14.3, 16.8, 16.5.
   unsigned long long qnext = 0;
   uint32_t qleft = 0;
   // the bucket that the lane's last item lies in: its rank, first item, the
@@ -773,7 +787,12 @@ __global__ __launch_bounds__(SSA_WG) __attribute__((amdgpu_waves_per_eu(4))) voi
     if (!have) {
       if (qleft == 0u) {
         const int cls = (ABC_CELL_BUCKETS - 1 - qrank) >> 4;
-        qleft = cls < ABC_LIGHT_CLASS ? claim << ((ABC_LIGHT_CLASS + 8 - cls) >> 3) : 1u;
+        qleft = 1u;
+        if (cls < ABC_LIGHT_CLASS) {
+          const uint32_t want = claim << ((ABC_LIGHT_CLASS + 8 - cls) >> 3);
+          const float cap = share * __builtin_amdgcn_exp2f(-2.0f - 0.25f * (float)cls);
+          qleft = cap < (float)want ? (cap > 1.0f ? (uint32_t)cap : 1u) : want;
+        }
         qnext = atomicAdd(queue, (unsigned long long)qleft);
       }
       const unsigned long long q = qnext++;

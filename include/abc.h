@@ -428,8 +428,9 @@ int32_t abc_set_ssa_blocks(abc_ctx* ctx, int32_t blocks);
 int32_t abc_get_ssa_blocks(const abc_ctx* ctx);
 /* Unit of the work items (cell sub-lanes) a lane of the SSA kernel claims per
  * atomic on its work queue: 1, 2, 4 or 8 (default 2).  Items are queued
- * heaviest first; light ones are claimed in small multiples of the unit, heavy
- * ones singly.  Items are independent, so this changes the schedule only.
+ * heaviest first; light ones are claimed in small multiples of the unit, within
+ * twice a lane's share of the call, heavy ones singly.  Items are independent,
+ * so this changes the schedule only.
  * Set by the autotuner. */
 int32_t abc_set_ssa_claim(abc_ctx* ctx, int32_t claim);
 int32_t abc_get_ssa_claim(const abc_ctx* ctx);
