@@ -654,9 +654,10 @@ __global__ __launch_bounds__(512) void infer_kernel(const float* __restrict__ x,
     }
     __syncthreads();
   }
-  // the output layer, 32 features per wave at a time (its padding ends on one)
+  // the output layer, 32 features per wave at a time (its padding ends on one),
+  // every gridDim.y-th 256 of them
   const LayerDesc L = layers[depth];
-  for (int f0 = wave * 32; f0 < n_out; f0 += 256) {
+  for (int f0 = (int)blockIdx.y * 256 + wave * 32; f0 < n_out; f0 += 256 * (int)gridDim.y) {
     f32x4 acc[2][RT];
     product(Wf + bf_off[depth], L.in, f0, acc);
 #pragma unroll
@@ -1065,7 +1066,10 @@ int forward(abc_mlp* p, int64_t Bn, const float* x_dev) {
 // and LDS (width up to 512); false: not launched.  Rows per workgroup: 16 while
 // those give at most one workgroup per CU, 32 up to two, 64 above, two of which
 // share a CU and overlap one's MFMAs with the other's activations (with 128, one
-// a CU, they do not).  16 / 32 / 64 / 128 rows, us: n = 77 39 / 43 / 60 / 86, 8,192
+// a CU, they do not).  Outputs beyond 256 are shared by as many workgroups per
+// row tile as leave at most one per CU, each with the hidden layers of its own:
+// 100 rows, 512 units, one layer, 2,048 outputs 44 us by one, 23 so (32 layer by
+// layer).  16 / 32 / 64 / 128 rows, us: n = 77 39 / 43 / 60 / 86, 8,192
 // 60 / 51 / 65 / 96, 16,384 97 / 70 / 69 / 101, 40,000 212 / 143 / 131 / 186.
 template <int RT, int FT>
 bool infer_launch(abc_mlp* p, int64_t n, const float* x, float* y) {
@@ -1075,9 +1079,11 @@ bool infer_launch(abc_mlp* p, int64_t n, const float* x, float* y) {
     (void)hipGetLastError();
     return false;
   }
-  hipLaunchKernelGGL((infer_kernel<RT, FT>), dim3((unsigned)((n + 16 * RT - 1) / (16 * RT))),
-                     dim3(512), lds, p->stream, x, n, p->n_in, p->d_layers, p->depth, p->d_bf_off,
-                     p->Wf, p->w, p->n_out,
+  const int64_t tiles = (n + 16 * RT - 1) / (16 * RT);
+  const int64_t parts = std::max<int64_t>(1, std::min<int64_t>((p->n_out + 255) / 256, 256 / tiles));
+  hipLaunchKernelGGL((infer_kernel<RT, FT>), dim3((unsigned)tiles, (unsigned)parts), dim3(512),
+                     lds, p->stream, x, n, p->n_in, p->d_layers, p->depth, p->d_bf_off, p->Wf, p->w,
+                     p->n_out,
                      (int)(p->n_out % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0), y);
   return true;
 }
