@@ -1935,13 +1935,14 @@ int data_meta(abc_ctx* c, int64_t G, int64_t n, int32_t nc, const int32_t* age, 
   return ABC_OK;
 }
 
-// Refuses counts of 2^20 or more, in any cell.  Up to 65,536 counts each are
+// Refuses counts of 2^20 or more, in any cell.  Up to 131,072 counts each are
 // looked at on the host, before any device work; more of them on the device,
 // before the resampling: a host scan of 18.5 million of each took 4 ms of the
-// call.  The host's look also tells which walks of data_stats_sorted_kernel
+// call (20 resamples, host / device, us: 66,000 counts 266 / 282, 129,000 324 /
+// 333, 244,000 391 / 380, 976,000 860 / 715).  The host's look also tells which walks of data_stats_sorted_kernel
 // have genes (*walks: 1 the 32-bit one, 2 the 64-bit one), from the cells that
 // data_pack_kernel takes the largest u + l of: an empty launch is 10 us.
-constexpr size_t kDataHostScan = 65536;
+constexpr size_t kDataHostScan = 131072;
 
 int data_check_host(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t* l,
                     const int32_t* cond, const int32_t* pulse, int64_t np, const int32_t* chase,

@@ -48,8 +48,8 @@ def test_refused_before_the_resampling(eng):
     assert refused < 0.6 * done
 
 
-# either side of 65,536 counts (scanned on the host, checked on the device)
-@pytest.mark.parametrize("n,G", [(1, 1), (256, 256), (257, 256)])
+# either side of 131,072 counts (scanned on the host, checked on the device)
+@pytest.mark.parametrize("n,G", [(1, 1), (256, 512), (257, 512)])
 @pytest.mark.parametrize("value", [1 << 20, 1 << 31, (1 << 32) - 1])
 @pytest.mark.parametrize("place", [0, -1])
 def test_refused_in_any_place(eng, n, G, value, place):
