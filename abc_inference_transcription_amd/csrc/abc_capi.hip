@@ -1939,9 +1939,10 @@ int data_meta(abc_ctx* c, int64_t G, int64_t n, int32_t nc, const int32_t* age, 
 // looked at on the host, before any device work; more of them on the device,
 // before the resampling: a host scan of 18.5 million of each took 4 ms of the
 // call (20 resamples, host / device, us: 66,000 counts 266 / 282, 129,000 324 /
-// 333, 244,000 391 / 380, 976,000 860 / 715).  The host's look also tells which walks of data_stats_sorted_kernel
-// have genes (*walks: 1 the 32-bit one, 2 the 64-bit one), from the cells that
-// data_pack_kernel takes the largest u + l of: an empty launch is 10 us.
+// 333, 244,000 391 / 380, 976,000 860 / 715).  The host's look also tells which
+// walks of data_stats_sorted_kernel have genes (*walks: 1 the 32-bit one, 2 the
+// 64-bit one), from the cells that data_pack_kernel takes the largest u + l of: an
+// empty launch is 10 us.
 constexpr size_t kDataHostScan = 131072;
 
 int data_check_host(abc_ctx* c, int64_t G, int64_t n, const uint32_t* u, const uint32_t* l,
